@@ -16,7 +16,7 @@ LIBDIR = os.path.join(HERE, "lib")
 LIB = os.path.join(LIBDIR, "libpqs.so")
 ARCH = "gfx950"
 
-SOURCES = ["plan.cpp", "jit.cpp", "engine.hip"]
+SOURCES = ["plan.cpp", "jit.cpp", "engine.hip", "measure.hip"]
 
 
 def hipcc():

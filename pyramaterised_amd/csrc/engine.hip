@@ -31,6 +31,7 @@
 #include <string>
 #include <vector>
 
+#include "measure.hpp"
 #include "plan.hpp"
 
 namespace pqs {
@@ -1108,99 +1109,6 @@ __global__ __launch_bounds__(RB) void k_sum_rows(const double2 *__restrict__ par
   if (threadIdx.x == 0) out[row] = double2{v[0], v[1]};
 }
 
-// Meyer-Wallach: per chunk of 2^c amplitudes, per qubit (rho00, rho11, rho01).
-template <typename R>
-__global__ __launch_bounds__(RB) void k_mw_partial(const typename CT<R>::V *__restrict__ states, int n, int c,
-                                                   int64_t n_chunks, double *__restrict__ part) {
-  using V = typename CT<R>::V;
-  __shared__ double sh[4 * RB];
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  V *tile = reinterpret_cast<V *>(smem_raw);
-  const int64_t b = blockIdx.x / n_chunks;
-  const int64_t chunk = blockIdx.x - b * n_chunks;
-  const int64_t dim = int64_t(1) << n;
-  const V *st = states + b * dim;
-  const int64_t cbase = chunk << c;
-  const int CS = 1 << c;
-  for (int j = threadIdx.x; j < CS; j += RB) tile[j] = st[cbase + j];
-  __syncthreads();
-  double *out = part + (b * n_chunks + chunk) * int64_t(n) * 4;
-  // in-chunk qubits: bit position pos < c  <=>  qubit q = n-1-pos
-  for (int pos = 0; pos < c; ++pos) {
-    double v[4] = {0, 0, 0, 0};
-    for (int u = threadIdx.x; u < (CS >> 1); u += RB) {
-      const int j0 = ins0(u, pos), j1 = j0 | (1 << pos);
-      const V a0 = tile[j0], a1 = tile[j1];
-      v[0] += double(a0.x) * a0.x + double(a0.y) * a0.y;
-      v[1] += double(a1.x) * a1.x + double(a1.y) * a1.y;
-      const double2 r = cmulc(a0, a1);
-      v[2] += r.x;
-      v[3] += r.y;
-    }
-    block_sum<4>(v, sh);
-    if (threadIdx.x == 0) {
-      const int q = n - 1 - pos;
-      out[4 * q + 0] = v[0];
-      out[4 * q + 1] = v[1];
-      out[4 * q + 2] = v[2];
-      out[4 * q + 3] = v[3];
-    }
-  }
-  if (c < n) {
-    double tot[1] = {0};
-    for (int j = threadIdx.x; j < CS; j += RB) tot[0] += double(tile[j].x) * tile[j].x + double(tile[j].y) * tile[j].y;
-    block_sum<1>(tot, sh);
-    for (int pos = c; pos < n; ++pos) {
-      const int bit = int((cbase >> pos) & 1);
-      double v[2] = {0, 0};
-      if (!bit) {
-        const V *pt = st + (cbase | (int64_t(1) << pos));
-        for (int j = threadIdx.x; j < CS; j += RB) {
-          const double2 r = cmulc(tile[j], pt[j]);
-          v[0] += r.x;
-          v[1] += r.y;
-        }
-        block_sum<2>(v, sh);
-      }
-      if (threadIdx.x == 0) {
-        const int q = n - 1 - pos;
-        out[4 * q + 0] = bit ? 0.0 : tot[0];
-        out[4 * q + 1] = bit ? tot[0] : 0.0;
-        out[4 * q + 2] = v[0];
-        out[4 * q + 3] = v[1];
-      }
-    }
-  }
-}
-
-__global__ __launch_bounds__(RB) void k_mw_final(const double *__restrict__ part, int n, int64_t n_chunks,
-                                                 double *__restrict__ rho, double *__restrict__ qout) {
-  __shared__ double sh[4 * RB];
-  const int64_t b = blockIdx.x;
-  double purity = 0;
-  for (int q = 0; q < n; ++q) {
-    double v[4] = {0, 0, 0, 0};
-    for (int64_t ch = threadIdx.x; ch < n_chunks; ch += RB) {
-      const double *p = part + ((b * n_chunks + ch) * n + q) * 4;
-      v[0] += p[0];
-      v[1] += p[1];
-      v[2] += p[2];
-      v[3] += p[3];
-    }
-    block_sum<4>(v, sh);
-    if (threadIdx.x == 0) {
-      if (rho) {
-        rho[(b * n + q) * 4 + 0] = v[0];
-        rho[(b * n + q) * 4 + 1] = v[1];
-        rho[(b * n + q) * 4 + 2] = v[2];
-        rho[(b * n + q) * 4 + 3] = v[3];
-      }
-      purity += v[0] * v[0] + v[1] * v[1] + 2 * (v[2] * v[2] + v[3] * v[3]);
-    }
-  }
-  if (threadIdx.x == 0 && qout) qout[b] = 2 * (1 - purity / n);
-}
-
 // Complex Gram  out[i][j] = sum_d conj(a_i[d]) b_j[d]: 16x16 output tile per
 // block, K split over blockIdx.z, partials reduced in order afterwards.
 constexpr int GT = 16, GK = 16;
@@ -1838,55 +1746,6 @@ __global__ __launch_bounds__(256) void k_fill_batch_table(InstDev *__restrict__ 
 __global__ void k_zero_u64(unsigned long long *p, int64_t n) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i < n) p[i] = 0;
-}
-
-// Stabiliser Renyi entropy sum (reference measure.py:318-349): for every
-// X-part j, f(m) = conj(c_m) c_{m^j}; a Walsh-Hadamard transform over m gives
-// F(i) = sum_m (-1)^{i.m} f(m) = <psi|X^j Z^i|psi> up to a phase; the block
-// returns sum_i |2^{-n/2} F(i)|^{2 alpha}.  One block per (instance, j).
-template <typename R>
-__global__ __launch_bounds__(RB) void k_magic_partial(const typename CT<R>::V *__restrict__ states, int n,
-                                                      double alpha, double *__restrict__ part) {
-  __shared__ double sh[RB];
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  double2 *f = reinterpret_cast<double2 *>(smem_raw);
-  const int64_t D = int64_t(1) << n;
-  const int64_t b = blockIdx.x / D;
-  const int64_t j = blockIdx.x - b * D;
-  const auto *c = states + b * D;
-  for (int64_t m = threadIdx.x; m < D; m += RB) {
-    const auto x = c[m], y = c[m ^ j];
-    f[m] = double2{double(x.x) * y.x + double(x.y) * y.y, double(x.x) * y.y - double(x.y) * y.x};
-  }
-  for (int bit = 0; bit < n; ++bit) {
-    __syncthreads();
-    for (int64_t u = threadIdx.x; u < D / 2; u += RB) {
-      const int64_t i0 = ((u >> bit) << (bit + 1)) | (u & ((int64_t(1) << bit) - 1));
-      const int64_t i1 = i0 | (int64_t(1) << bit);
-      const double2 a = f[i0], d = f[i1];
-      f[i0] = double2{a.x + d.x, a.y + d.y};
-      f[i1] = double2{a.x - d.x, a.y - d.y};
-    }
-  }
-  __syncthreads();
-  const double scale = 1.0 / double(D);  // (2^{-n/2})^2 on |F|^2
-  double v[1] = {0};
-  for (int64_t i = threadIdx.x; i < D; i += RB) {
-    const double a2 = (f[i].x * f[i].x + f[i].y * f[i].y) * scale;
-    v[0] += alpha == 2.0 ? a2 * a2 : (alpha == 0.5 ? sqrt(a2) : pow(a2, alpha));
-  }
-  block_sum<1>(v, sh);
-  if (threadIdx.x == 0) part[blockIdx.x] = v[0];
-}
-
-__global__ __launch_bounds__(RB) void k_sum_rows_real(const double *__restrict__ part, int64_t n_chunks,
-                                                      double *__restrict__ out) {
-  __shared__ double sh[RB];
-  const int64_t row = blockIdx.x;
-  double v[1] = {0};
-  for (int64_t c = threadIdx.x; c < n_chunks; c += RB) v[0] += part[row * n_chunks + c];
-  block_sum<1>(v, sh);
-  if (threadIdx.x == 0) out[row] = v[0];
 }
 
 inline unsigned grid_for(int64_t n, int b) { return unsigned((n + b - 1) / b); }
@@ -3050,24 +2909,9 @@ int pqs_mw(pqs_ctx *ctx, int32_t dtype, const void *states, int32_t n, int64_t b
   if (batch == 0) return PQS_OK;
   DeviceGuard g(ctx->device);
   hipStream_t st = (hipStream_t)stream;
-  const int c = std::min(n, 11);
-  const int64_t nch = int64_t(1) << (n - c);
-  int rc = ws_reserve(ctx, size_t(batch * nch * n * 4) * sizeof(double), st);
+  const int rc = ws_reserve(ctx, pqs::mw_ws(n, batch), st);
   if (rc) return rc;
-  double *part = (double *)ctx->ws;
-  const int64_t grid = batch * nch;
-  if (grid > 0x7fffffff) return fail(PQS_ERR_UNSUPPORTED, "batch too large");
-  const size_t lds = (size_t(1) << c) * amp_bytes(dtype);
-  if (dtype == PQS_C128)
-    hipLaunchKernelGGL(k_mw_partial<double>, dim3(unsigned(grid)), dim3(RB), lds, st, (const double2 *)states, n, c,
-                       nch, part);
-  else
-    hipLaunchKernelGGL(k_mw_partial<float>, dim3(unsigned(grid)), dim3(RB), lds, st, (const float2 *)states, n, c,
-                       nch, part);
-  HIPCHECK(hipGetLastError());
-  hipLaunchKernelGGL(k_mw_final, dim3(unsigned(batch)), dim3(RB), 0, st, part, n, nch, rho, q);
-  HIPCHECK(hipGetLastError());
-  return PQS_OK;
+  return pqs::mw_launch(dtype, states, n, batch, rho, q, ctx->ws, st);
 }
 
 }  // extern "C"
@@ -3565,34 +3409,9 @@ int pqs_magic(pqs_ctx *ctx, int32_t dtype, const void *states, int32_t n, int64_
   if (batch == 0) return PQS_OK;
   DeviceGuard g(ctx->device);
   hipStream_t st = (hipStream_t)stream;
-  const int64_t D = int64_t(1) << n;
-  int rc = ws_reserve(ctx, size_t(batch * D) * sizeof(double), st);
+  const int rc = ws_reserve(ctx, pqs::magic_ws(n, batch), st);
   if (rc) return rc;
-  const size_t lds = size_t(D) * sizeof(double2);
-  if (int(lds) > ctx->max_lds) return fail(PQS_ERR_UNSUPPORTED, "state does not fit in LDS");
-  static bool attr[2] = {false, false};
-  if (lds > 65536) {
-    if (!attr[0]) {
-      HIPCHECK(hipFuncSetAttribute((const void *)k_magic_partial<double>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, ctx->max_lds));
-      HIPCHECK(hipFuncSetAttribute((const void *)k_magic_partial<float>,
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, ctx->max_lds));
-      attr[0] = true;
-    }
-  }
-  const int64_t grid = batch * D;
-  if (grid > 0x7fffffff) return fail(PQS_ERR_UNSUPPORTED, "batch too large");
-  double *part = (double *)ctx->ws;
-  if (dtype == PQS_C128)
-    hipLaunchKernelGGL(k_magic_partial<double>, dim3(unsigned(grid)), dim3(RB), lds, st, (const double2 *)states, n,
-                       alpha, part);
-  else
-    hipLaunchKernelGGL(k_magic_partial<float>, dim3(unsigned(grid)), dim3(RB), lds, st, (const float2 *)states, n,
-                       alpha, part);
-  HIPCHECK(hipGetLastError());
-  hipLaunchKernelGGL(k_sum_rows_real, dim3(unsigned(batch)), dim3(RB), 0, st, part, D, out);
-  HIPCHECK(hipGetLastError());
-  return PQS_OK;
+  return pqs::magic_launch(dtype, states, n, batch, alpha, out, ctx->ws, st);
 }
 
 int pqs_plan_jit_source(const pqs_plan *p, char *buf, int64_t cap, int64_t *len, int32_t *n_jit_sweeps) {
