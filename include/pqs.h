@@ -89,7 +89,7 @@ typedef struct pqs_op {
 typedef struct pqs_plan_opts {
   int32_t tile_bits;    /* qubits resident per tile (<= 13 for c128)          */
   int32_t low_bits;     /* lowest bit positions forced into every tile        */
-  int32_t block;        /* threads per workgroup (256, 512 or 1024)           */
+  int32_t block;        /* 0, 256, 512 or 1024; the executors size their own   */
   int32_t dtype;        /* pqs_dtype                                          */
   int32_t flags;        /* PQS_PLAN_* tuning switches (0: defaults)           */
 } pqs_plan_opts;

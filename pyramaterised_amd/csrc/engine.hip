@@ -29,6 +29,7 @@
 #include <cstdio>
 #include <cstring>
 #include <string>
+#include <type_traits>
 #include <vector>
 
 #include "measure.hpp"
@@ -358,8 +359,8 @@ __device__ __forceinline__ void apply_lds_op(typename CT<R>::V *tile, const int 
   }
 }
 
-// One tile of one instance through one sweep, op by op in LDS (tiles below
-// 10 qubits).  `sw` is the sweep (a kernel argument, or a record in device
+// One tile of one instance through one sweep, op by op in LDS (complex64 tiles
+// below 10 qubits).  `sw` is the sweep (a kernel argument, or a record in device
 // memory for launches that mix plans).
 template <typename R, int BLOCK>
 __device__ __forceinline__ void sweep_lds_body(const DevSweep &sw, const DevOp *__restrict__ ops,
@@ -421,7 +422,7 @@ __device__ __forceinline__ void sweep_lds_body(const DevSweep &sw, const DevOp *
     const int tg = op->tangent;
     if (tg >= 0 && tg != in.tangent) continue;
     __syncthreads();
-    apply_lds_op<R, (1 << (sizeof(R) == 8 ? 13 : 14)) / BLOCK, false>(tile, S, op, base, params, terms, tid, BLOCK);
+    apply_lds_op<R, 512 / BLOCK, false>(tile, S, op, base, params, terms, tid, BLOCK);
   }
   __syncthreads();
 
@@ -620,6 +621,81 @@ __device__ __forceinline__ void reg_z(V (&a)[NA]) {
 #pragma unroll
   for (int v = 0; v < NA; ++v)
     if (v & (1 << B)) a[v] = cneg(a[v]);
+}
+
+// 1 - i t P (form A) or u - i P (form B) on register bits B0, B1, with P =
+// X(x)X, or Y(x)Y = X(x)X on 01, 10 and -X(x)X on 00, 11
+template <int B0, int B1, bool FB, bool YY, typename V, typename R>
+__device__ __forceinline__ void reg_rpp(V (&a)[NA], R t) {
+  if constexpr (B0 != B1) {
+#pragma unroll
+    for (int v = 0; v < NA; ++v) {
+      const int w = v ^ (1 << B0) ^ (1 << B1);
+      if (w < v) continue;
+      const bool neg = YY && !(((v >> B0) ^ (v >> B1)) & 1);
+      const V x = a[v], y = a[w];
+      if constexpr (!FB) {
+        const R u = neg ? -t : t;
+        a[v] = V{fma(u, y.y, x.x), fma(-u, y.x, x.y)};
+        a[w] = V{fma(u, x.y, y.x), fma(-u, x.x, y.y)};
+      } else {
+        const V p = neg ? V{-y.x, -y.y} : y, q = neg ? V{-x.x, -x.y} : x;
+        a[v] = V{fma(t, x.x, p.y), fma(t, x.y, -p.x)};
+        a[w] = V{fma(t, y.x, q.y), fma(t, y.y, -q.x)};
+      }
+    }
+  }
+}
+
+// fSim and its derivatives: [[d, -i o], [-i o, d]] on 01, 10 and p on 11
+template <int B0, int B1, typename V, typename R>
+__device__ __forceinline__ void reg_fsim(V (&a)[NA], R d, R o, V p) {
+  if constexpr (B0 != B1) {
+#pragma unroll
+    for (int v = 0; v < NA; ++v) {
+      if ((v >> B0) & 1) {
+        if ((v >> B1) & 1) a[v] = cmul(a[v], p);
+        continue;
+      }
+      if (!((v >> B1) & 1)) continue;
+      const int w = v ^ (1 << B0) ^ (1 << B1);
+      const V x = a[v], y = a[w];
+      a[v] = V{fma(d, x.x, o * y.y), fma(d, x.y, -o * y.x)};
+      a[w] = V{fma(d, y.x, o * x.y), fma(d, y.y, -o * x.x)};
+    }
+  }
+}
+
+// dense 4x4, BH the more significant register bit of its basis
+template <int BH, int BL, typename V>
+__device__ __forceinline__ void reg_mat2(V (&a)[NA], const V (&m)[16]) {
+  if constexpr (BH != BL) {
+#pragma unroll
+    for (int v = 0; v < NA; ++v) {
+      if (((v >> BH) | (v >> BL)) & 1) continue;
+      V x[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) x[c] = a[v | ((c >> 1) << BH) | ((c & 1) << BL)];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        V y = cmul(m[4 * r], x[0]);
+#pragma unroll
+        for (int c = 1; c < 4; ++c) y = cadd(y, cmul(m[4 * r + c], x[c]));
+        a[v | ((r >> 1) << BH) | ((r & 1) << BL)] = y;
+      }
+    }
+  }
+}
+
+// (d, o, p) of an fSim (sel 0) or its derivative matrices as the reference
+// writes them (sel 1 d_theta, 2 d_phi, 3 fixed fSim's d_theta; gates.py:609-648,
+// 719-737) from (sin, cos) of theta and phi
+__device__ __forceinline__ void fsim_coef(int sel, double st, double ct, double sp, double cp, double &d, double &o,
+                                          double2 &p) {
+  const bool dth = sel == 1 || sel == 3;
+  d = dth ? -st : ct;
+  o = dth ? ct : st;
+  p = sel == 3 ? double2{1, 0} : sel == 2 ? double2{-sp, -cp} : double2{cp, -sp};
 }
 
 // Compact op record staged in LDS (32 bytes).
@@ -899,6 +975,41 @@ __device__ __forceinline__ void sweep_reg_body(const DevSweep &sw, const DevOp *
           }
           break;
         }
+        case PQS_OP_RXX:
+          if constexpr (LDSOPS) {
+            fscale *= op.f;
+            if (fb) {
+              SW4(r0, SW4C(r1, reg_rpp<B_, C_, true, false>(a, t)));
+            } else {
+              SW4(r0, SW4C(r1, reg_rpp<B_, C_, false, false>(a, t)));
+            }
+          }
+          break;
+        case PQS_OP_RYY:
+          if constexpr (LDSOPS) {
+            fscale *= op.f;
+            if (fb) {
+              SW4(r0, SW4C(r1, reg_rpp<B_, C_, true, true>(a, t)));
+            } else {
+              SW4(r0, SW4C(r1, reg_rpp<B_, C_, false, true>(a, t)));
+            }
+          }
+          break;
+        case PQS_OP_FSIM:
+        case PQS_OP_GEN_FSIM:
+        case PQS_OP_MAT2: {
+          if constexpr (LDSOPS) {
+            const DevOp *d = ops + o;
+            if (kind == PQS_OP_GEN_FSIM && d->tangent != in.tangent) break;  // uniform per block
+            M4 M;
+            mat2_of(d, params, M);
+            V m[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) m[i] = cvt<R>(M.m[i]);
+            SW4(r0, SW4C(r1, reg_mat2<B_, C_>(a, m)));
+          }
+          break;
+        }
         case PQS_OP_CX:
           if (r0 != 0xff) {
             SW4(r1, SW4C(r0, reg_cx<B_, C_>(a)));
@@ -977,6 +1088,530 @@ __global__ __launch_bounds__(MAXT) void k_sweep_reg(const DevSweep sw, const Dev
   sweep_reg_body<R, MAXT, LDSOPS>(sw, ops, terms, phases, in, tile_id, init_tab, n, s, n_sweeps);
 }
 
+// ---------------------------------------------------------- wave executor
+// complex128 tiles below 10 qubits: 64 >> (k - r) of them per wave, NA = 2^r
+// amplitudes per lane (plan.hpp), no barriers.  A rotation layer is straight
+// code over the bits: register bits pair amplitudes of the lane, lane bits
+// fetch them from the partner lane by DPP (bits 4 and 5 trade places with a
+// register bit, v_permlane16/32_swap).  A run of CNOTs is one write and read of the tile in LDS, and so is
+// the partner fetch of any other op.  Op records come 64 at a time, one per
+// lane, and are read out into scalar registers, so no op waits for memory and
+// dispatch is scalar.  Angles belong to the instance: at a refill each lane
+// computes (tan, cos) of kWaveAngles of its tile's angles (their parameters
+// were loaded a refill ahead) into 4 KB of LDS.  Rotations are in scaled
+// form, the scale clamped and checked as in the specialised kernels (jit.cpp).
+//
+// Bound by instruction latency for a few hundred states, then by vector
+// issue (about 590 vector instructions per HEA layer of 8 qubits).  Measured,
+// 8 qubits, 10 layers of (R_y, R_z, CNOT chain): one state 153 -> 29 us, 2000
+// states 763 -> 43 us, 16,000 states 234 us; 4 qubits, 3 layers, one state
+// 26 -> 11 us.  Before: a pass over LDS, a barrier and a sincos in every
+// thread for each op (still the route of complex64 tiles of this size).
+// Tried and slower: one dispatch case per op and register bit on 16
+// amplitudes per lane (143 us for the 2000 states: the joins of some 90 cases
+// move the whole register file), and one generic op at a time with partners
+// fetched lane by lane (172 us).
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// the value of lane ^ M
+template <int M>
+__device__ __forceinline__ int xor_lane(int v) {
+  if constexpr (M == 1) {
+    return __builtin_amdgcn_update_dpp(0, v, 0xb1, 0xf, 0xf, true);  // quad_perm 1 0 3 2
+  } else if constexpr (M == 2) {
+    return __builtin_amdgcn_update_dpp(0, v, 0x4e, 0xf, 0xf, true);  // quad_perm 2 3 0 1
+  } else if constexpr (M == 4) {
+    const int h = __builtin_amdgcn_update_dpp(0, v, 0x141, 0xf, 0xf, true);  // row_half_mirror: ^ 7
+    return __builtin_amdgcn_update_dpp(0, h, 0x1b, 0xf, 0xf, true);          // quad_perm 3 2 1 0: ^ 3
+  } else {
+    static_assert(M == 8);
+    return __builtin_amdgcn_update_dpp(0, v, 0x128, 0xf, 0xf, true);  // row_ror 8
+  }
+}
+
+// Trade lane bit LB (5 or 4) with register bit RB - 1 in every pair.
+template <int LB, int RB>
+__device__ __forceinline__ void lane_reg_swap(double2 (&a)[1 << RB]) {
+  constexpr int H = 1 << (RB - 1);
+#pragma unroll
+  for (int v = 0; v < H; ++v) {
+    unsigned x[4], y[4];
+    __builtin_memcpy(x, &a[v], 16);
+    __builtin_memcpy(y, &a[v | H], 16);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if constexpr (LB == 5) {
+        const auto r = __builtin_amdgcn_permlane32_swap(x[i], y[i], false, false);
+        x[i] = r[0];
+        y[i] = r[1];
+      } else {
+        const auto r = __builtin_amdgcn_permlane16_swap(x[i], y[i], false, false);
+        x[i] = r[0];
+        y[i] = r[1];
+      }
+    }
+    __builtin_memcpy(&a[v], x, 16);
+    __builtin_memcpy(&a[v | H], y, 16);
+  }
+}
+
+template <int M>
+__device__ __forceinline__ double2 xor_lane(double2 x) {
+  int w[4];
+  __builtin_memcpy(w, &x, 16);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) w[i] = xor_lane<M>(w[i]);
+  __builtin_memcpy(&x, w, 16);
+  return x;
+}
+
+// x with its sign flipped where bit 0 of s is set
+__device__ __forceinline__ double sign_flip(double x, uint32_t s) {
+  return __hiloint2double(int(uint32_t(__double2hiint(x)) ^ (s << 31)), __double2loint(x));
+}
+
+// R_y (REAL) or R_x with t = tan(a/2) on lane bit B
+template <int B, bool REAL, int N>
+__device__ __forceinline__ void wave_lane_rot(double2 (&a)[N], double t, int lane) {
+  const double u = REAL ? (((lane >> B) & 1) ? t : -t) : t;
+#pragma unroll
+  for (int v = 0; v < N; ++v) {
+    const double2 p = xor_lane<(1 << B)>(a[v]);
+    if constexpr (REAL) a[v] = double2{fma(u, p.x, a[v].x), fma(u, p.y, a[v].y)};
+    else a[v] = double2{fma(u, p.y, a[v].x), fma(-u, p.x, a[v].y)};
+  }
+}
+
+// the same on register bit B
+template <int B, bool REAL, int N>
+__device__ __forceinline__ void wave_reg_rot(double2 (&a)[N], double t) {
+#pragma unroll
+  for (int v = 0; v < N; ++v) {
+    if ((v >> B) & 1) continue;
+    const double2 x = a[v], y = a[v | (1 << B)];
+    if constexpr (REAL) {
+      a[v] = double2{fma(-t, y.x, x.x), fma(-t, y.y, x.y)};
+      a[v | (1 << B)] = double2{fma(t, x.x, y.x), fma(t, x.y, y.y)};
+    } else {
+      a[v] = double2{fma(t, y.y, x.x), fma(-t, y.x, x.y)};
+      a[v | (1 << B)] = double2{fma(t, x.y, y.x), fma(-t, x.x, y.y)};
+    }
+  }
+}
+
+// One wave: `in` and `tile_id` are those of the lane's tile, live false for
+// lanes without one.  lds: 64 kWaveAngles entries of the angle table, then
+// the wave's 64 NA amplitudes.
+template <int RB>
+__device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp *__restrict__ stream,
+                                          const pqs::WaveAngle *__restrict__ angles, const int n_angles,
+                                          const DevOp *__restrict__ dops, const DevTerm *__restrict__ terms,
+                                          const InstDev &in, const bool live, const int64_t tile_id,
+                                          const double2 *__restrict__ init_tab, int n, int s, int n_sweeps,
+                                          double2 *lds) {
+  constexpr int N = 1 << RB;
+  constexpr double cmin = 1e-20, rescale = 1e-100;
+  constexpr int NANG = pqs::kWaveAngles;
+  const int lane = threadIdx.x;
+  const int k = sw.k, lt = k - RB, T = 1 << lt;
+  const int l = lane & (T - 1);
+  double2 *mine_tab = lds + (lane - l) * NANG;
+  double2 *tile = lds + 64 * NANG + (lane - l) * N;  // this tile's 2^k amplitudes
+
+  uint64_t base = 0;
+  for (int r = 0; r < sw.cnruns; ++r)
+    base |= (uint64_t(tile_id >> sw.crun_shift[r]) & ((uint64_t(1) << sw.crun_len[r]) - 1)) << sw.crun_pos[r];
+  const double2 *src;
+  double2 *dst;
+  int init = 0;
+  if (in.pingpong) {
+    dst = ((n_sweeps - 1 - s) & 1) == 0 ? (double2 *)in.state : (double2 *)in.alt;
+    if (s == in.start_sweep) {
+      src = (const double2 *)in.src;
+      init = in.src ? 0 : in.init;
+    } else {
+      src = ((n_sweeps - s) & 1) == 0 ? (const double2 *)in.state : (const double2 *)in.alt;
+    }
+  } else {
+    dst = (double2 *)in.state;
+    if (s == in.start_sweep) {
+      src = in.src ? (const double2 *)in.src : dst;
+      init = in.src ? 0 : in.init;
+    } else {
+      src = dst;
+    }
+  }
+  const double *params = in.params;
+
+  // parameters of the next refill, loaded ahead
+  double praw[NANG], pscale[NANG], poff[NANG];
+  auto ahead = [&](int a0) {
+#pragma unroll
+    for (int m = 0; m < NANG; ++m) {
+      const int i = a0 + l + m * T;
+      praw[m] = pscale[m] = poff[m] = 0.0;
+      if (live && i < n_angles) {
+        const pqs::WaveAngle &w = angles[i];
+        pscale[m] = w.scale;
+        poff[m] = w.offset;
+        if (w.slot >= 0) praw[m] = params[w.slot];
+      }
+    }
+  };
+  ahead(0);
+  const uint4 *recs = reinterpret_cast<const uint4 *>(stream);
+  uint4 held[2] = {recs[2 * lane], recs[2 * lane + 1]}, next[2] = {recs[2 * lane + 128], recs[2 * lane + 129]};
+
+  // the amplitude's offset in the state (index j of the tile)
+  auto offset = [&](int v) -> uint64_t {
+    const int j = l | (v << lt);
+    if (sw.n_tiles == 1) return uint64_t(j);
+    uint64_t g = base;
+    for (int r = 0; r < sw.nruns; ++r)
+      g |= uint64_t((j >> sw.run_shift[r]) & ((1 << sw.run_len[r]) - 1)) << sw.run_pos[r];
+    return g;
+  };
+  double2 a[N];
+#pragma unroll
+  for (int v = 0; v < N; ++v) {
+    a[v] = double2{0, 0};
+    if (live) {
+      const uint64_t g = offset(v);
+      if (init == 0) {
+        a[v] = src[g];
+      } else if (init == 1) {
+        a[v].x = g == 0 ? 1.0 : 0.0;
+      } else {
+        a[v].x = 1.0;
+        for (int q = 0; q < n; ++q) a[v] = cmul(a[v], init_tab[2 * q + int((g >> (n - 1 - q)) & 1)]);
+      }
+    }
+  }
+
+  double fs = 1.0;
+  auto field = [](uint32_t v, int i) { return uint32_t(__builtin_amdgcn_readlane(int(v), i)); };
+  // the lane's part of the parity of j & z and base & zg
+  auto lane_parity = [&](uint32_t zl, uint64_t zg) -> uint32_t {
+    uint32_t q = uint32_t(__popc(uint32_t(l) & zl));
+    if (zg) q += uint32_t(__popcll(base & zg));
+    return q & 1;
+  };
+  auto reg_parity = [](int v, uint32_t zr) -> uint32_t { return uint32_t(__builtin_popcount(uint32_t(v) & zr)) & 1; };
+  // LDS in order within the wave: a write of the tile follows every read of
+  // the previous one
+  auto put = [&]() {
+#pragma unroll
+    for (int v = 0; v < N; ++v) tile[l | (v << lt)] = a[v];
+    wave_fence();
+  };
+  auto partner = [&](double2(&p)[N], uint32_t x) {
+#pragma unroll
+    for (int v = 0; v < N; ++v) p[v] = tile[uint32_t(l | (v << lt)) ^ x];
+  };
+#pragma unroll 1
+  for (int o = 0;; ++o) {
+    const int i = o & 63;
+    if (i == 0 && o) {  // streams are padded to whole blocks of 64 and one more
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        held[h] = next[h];
+        next[h] = recs[2 * (o + 64 + lane) + h];
+      }
+    }
+    const uint32_t w0 = field(held[0].x, i);
+    const int code = int(w0 & 0xffff), ang = int(w0 >> 16);
+    if (code == pqs::kWEnd) break;
+    if (code == pqs::kWLayerRy || code == pqs::kWLayerRx) {
+      const double2 *ca = mine_tab + ang;
+      double2 cur[6];  // the table holds kWaveAngles per lane: entries past k are not used
+#pragma unroll
+      for (int b = 0; b < 6; ++b) cur[b] = ca[b];
+      auto layer = [&](auto real) {
+        constexpr bool RE = decltype(real)::value;
+        if (lt > 0) wave_lane_rot<0, RE>(a, cur[0].x, lane), fs *= cur[0].y;
+        if (lt > 1) wave_lane_rot<1, RE>(a, cur[1].x, lane), fs *= cur[1].y;
+        if (lt > 2) wave_lane_rot<2, RE>(a, cur[2].x, lane), fs *= cur[2].y;
+        if (lt > 3) wave_lane_rot<3, RE>(a, cur[3].x, lane), fs *= cur[3].y;
+        // lane bits 4 and 5 trade places with the top register bit
+        if (lt > 4) {
+          fs *= cur[4].y;
+          lane_reg_swap<4, RB>(a);
+          wave_reg_rot<RB - 1, RE>(a, cur[4].x);
+          lane_reg_swap<4, RB>(a);
+        }
+        if (lt > 5) {
+          fs *= cur[5].y;
+          lane_reg_swap<5, RB>(a);
+          wave_reg_rot<RB - 1, RE>(a, cur[5].x);
+          lane_reg_swap<5, RB>(a);
+        }
+        double2 c = ca[lt];
+        fs *= c.y;
+        wave_reg_rot<0, RE>(a, c.x);
+        if constexpr (RB > 1) {
+          c = ca[lt + 1];
+          fs *= c.y;
+          wave_reg_rot<1, RE>(a, c.x);
+        }
+        if constexpr (RB > 2) {
+          c = ca[lt + 2];
+          fs *= c.y;
+          wave_reg_rot<2, RE>(a, c.x);
+        }
+      };
+      if (code == pqs::kWLayerRy) layer(std::true_type{});
+      else layer(std::false_type{});
+      continue;
+    }
+    if (code == pqs::kWLayerRz) {
+      // one phase per amplitude: the lane bits' product, then the register bits'
+      const double2 *ca = mine_tab + ang;
+      double2 w{1.0, 0.0};
+#pragma unroll
+      for (int b = 0; b < 6; ++b)
+        if (b < lt) {
+          const double2 c = ca[b];
+          fs *= c.y;
+          const double t = ((l >> b) & 1) ? -c.x : c.x;
+          w = double2{fma(t, w.y, w.x), fma(-t, w.x, w.y)};
+        }
+      double2 ph[N];
+      ph[0] = w;
+#pragma unroll
+      for (int b = 0; b < RB; ++b) {
+        const double2 c = ca[lt + b];
+        fs *= c.y;
+#pragma unroll
+        for (int v = 0; v < (1 << b); ++v) {
+          const double2 y = ph[v];
+          ph[v] = double2{fma(c.x, y.y, y.x), fma(-c.x, y.x, y.y)};
+          ph[v | (1 << b)] = double2{fma(-c.x, y.y, y.x), fma(c.x, y.x, y.y)};
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < N; ++v) a[v] = cmul(a[v], ph[v]);
+      continue;
+    }
+    const uint32_t x = field(held[0].y, i), z = field(held[0].z, i);
+    const int c = int(field(held[0].w, i));
+    if (code == pqs::kWRefill) {
+      // ops before this one have read their angles (LDS in order)
+#pragma unroll
+      for (int m = 0; m < NANG; ++m) {
+        if (m * T < int(x)) {
+          double sn, cs;
+          sincos(0.5 * (poff[m] + pscale[m] * praw[m]), &sn, &cs);
+          if (fabs(cs) < cmin) cs = cs < 0.0 ? -cmin : cmin;
+          mine_tab[l + m * T] = double2{sn / cs, cs};
+        }
+      }
+      wave_fence();
+      ahead(c + int(x));
+      continue;
+    }
+    if (code == pqs::kWCheck) {
+      if (fabs(fs) < rescale) {
+#pragma unroll
+        for (int v = 0; v < N; ++v) a[v] = double2{a[v].x * fs, a[v].y * fs};
+        fs = 1.0;
+      }
+      continue;
+    }
+    const uint64_t zg = uint64_t(field(held[1].x, i)) | (uint64_t(field(held[1].y, i)) << 32);
+    if (code == pqs::kWMap) {
+      put();
+      // m(j): the masks of j's set bits, XORed
+      uint32_t from = 0;
+      auto mask = [&](int b) -> uint32_t {
+        const uint32_t w = b < 2 ? x : b < 4 ? z : b < 6 ? uint32_t(zg) : b < 8 ? uint32_t(zg >> 32) : uint32_t(c);
+        return b & 1 ? w >> 16 : w & 0xffff;
+      };
+#pragma unroll
+      for (int b = 0; b < 6; ++b)
+        if (b < lt) from ^= ((l >> b) & 1) ? mask(b) : 0u;
+      uint32_t rm[RB];
+#pragma unroll
+      for (int b = 0; b < RB; ++b) {
+        rm[b] = 0;
+#pragma unroll
+        for (int q = 0; q < pqs::kWaveTile; ++q)
+          if (q == lt + b) rm[b] = mask(q);
+      }
+#pragma unroll
+      for (int v = 0; v < N; ++v) {
+        uint32_t f = from;
+#pragma unroll
+        for (int b = 0; b < RB; ++b)
+          if ((v >> b) & 1) f ^= rm[b];
+        a[v] = tile[f];
+      }
+      continue;
+    }
+    const uint32_t xr = x >> lt, zl = z & uint32_t(T - 1), zr = z >> lt;
+    if (code == pqs::kWPhase) {
+      const double2 ca = mine_tab[ang];
+      fs *= ca.y;
+      const double t0 = sign_flip(ca.x, lane_parity(zl, zg) ^ uint32_t(c));
+#pragma unroll
+      for (int v = 0; v < N; ++v) {
+        const double t = sign_flip(t0, reg_parity(v, zr));
+        a[v] = double2{fma(t, a[v].y, a[v].x), fma(-t, a[v].x, a[v].y)};
+      }
+      continue;
+    }
+    if (code == pqs::kWCz) {
+      const bool lo = (uint32_t(l) & zl) == zl && (base & zg) == zg;
+#pragma unroll
+      for (int v = 0; v < N; ++v) {
+        const uint32_t neg = lo && (uint32_t(v) & zr) == zr ? 1u : 0u;
+        a[v] = double2{sign_flip(a[v].x, neg), sign_flip(a[v].y, neg)};
+      }
+      continue;
+    }
+    if (code == pqs::kWRotI || code == pqs::kWRotR) {
+      const double2 ca = mine_tab[ang];
+      double2 p[N];
+      put();
+      partner(p, x);
+      fs *= ca.y;
+      const double t0 = sign_flip(ca.x, lane_parity(zl, zg) ^ uint32_t(c));
+#pragma unroll
+      for (int v = 0; v < N; ++v) {
+        const double t = sign_flip(t0, reg_parity(v, zr));
+        // the imaginary form is the real one on (p.y, -p.x)
+        const double px = code == pqs::kWRotI ? p[v].y : p[v].x, py = code == pqs::kWRotI ? -p[v].x : p[v].y;
+        a[v] = double2{fma(t, px, a[v].x), fma(t, py, a[v].y)};
+      }
+      continue;
+    }
+    if (code == pqs::kWCx) {
+      double2 p[N];
+      put();
+      partner(p, x);
+      const bool on = (base & zg) != 0;
+#pragma unroll
+      for (int v = 0; v < N; ++v) {
+        a[v].x = on ? p[v].x : a[v].x;
+        a[v].y = on ? p[v].y : a[v].y;
+      }
+      continue;
+    }
+    if (code == pqs::kWMat1) {
+      const DevOp *d = dops + c;
+      double2 p[N];
+      put();
+      partner(p, x);
+      const uint32_t q = lane_parity(zl, zg);
+#pragma unroll
+      for (int v = 0; v < N; ++v) {
+        const bool b = (q ^ reg_parity(v, zr)) & 1;
+        const double2 md{b ? d->m[6] : d->m[0], b ? d->m[7] : d->m[1]};
+        const double2 mo{b ? d->m[4] : d->m[2], b ? d->m[5] : d->m[3]};
+        a[v] = cadd(cmul(md, a[v]), cmul(mo, p[v]));
+      }
+      continue;
+    }
+    const int tangent = int(field(held[1].z, i));
+    if (code == pqs::kWSum) {
+      const bool mine = in.tangent == tangent;
+      if (__ballot(mine && live)) {
+        const DevOp *d = dops + c;
+        const DevTerm *tm = terms + d->term0;
+        double2 acc[N];
+#pragma unroll
+        for (int v = 0; v < N; ++v) acc[v] = double2{0, 0};
+        put();
+#pragma unroll 1
+        for (int t = 0; t < d->nterms; ++t) {
+          const uint32_t tx = tm[t].xm, tz = tm[t].zm_tile;
+          double2 p[N];
+          partner(p, tx);
+          const uint32_t q = lane_parity(tz & uint32_t(T - 1), tm[t].zm_glob) ^ (uint32_t(__popc(tx & tz)) & 1);
+#pragma unroll
+          for (int v = 0; v < N; ++v) {
+            const uint32_t sg = q ^ reg_parity(v, tz >> lt);
+            acc[v] = cadd(acc[v], cmul(double2{sign_flip(tm[t].cre, sg), sign_flip(tm[t].cim, sg)}, p[v]));
+          }
+        }
+#pragma unroll
+        for (int v = 0; v < N; ++v) {
+          a[v].x = mine ? acc[v].x : a[v].x;
+          a[v].y = mine ? acc[v].y : a[v].y;
+        }
+      }
+      continue;
+    }
+    if (code == pqs::kWFsim || code == pqs::kWGenFsim) {
+      const bool mine = code == pqs::kWFsim || in.tangent == tangent;
+      const double2 ct = mine_tab[ang], cp = int(z) >= 0 ? mine_tab[z] : double2{0, 1};
+      double dg, of;
+      double2 ph;
+      fsim_coef(code == pqs::kWFsim ? 0 : dops[c].pauli, ct.x * ct.y, ct.y, cp.x * cp.y, cp.y, dg, of, ph);
+      double2 p[N];
+      put();
+      partner(p, x);
+      const uint32_t q = uint32_t(__popc(uint32_t(l) & x));  // l < T: the lane bits of x
+#pragma unroll
+      for (int v = 0; v < N; ++v) {
+        const uint32_t set = q + uint32_t(__builtin_popcount(uint32_t(v) & xr));  // 0, 1 or 2 of the two bits
+        const double2 odd{fma(dg, a[v].x, of * p[v].y), fma(dg, a[v].y, -of * p[v].x)};
+        const double2 both = cmul(a[v], ph);
+        const double nx = set == 1 ? odd.x : set == 2 ? both.x : a[v].x;
+        const double ny = set == 1 ? odd.y : set == 2 ? both.y : a[v].y;
+        a[v].x = mine ? nx : a[v].x;
+        a[v].y = mine ? ny : a[v].y;
+      }
+      continue;
+    }
+    {  // kWMat2
+      const DevOp *d = dops + c;
+      double2 y[N];
+#pragma unroll
+      for (int v = 0; v < N; ++v) y[v] = double2{0, 0};
+      put();
+#pragma unroll 1
+      for (int e = 0; e < 4; ++e) {  // column = row ^ e
+        double2 p[N];
+        partner(p, (e & 2 ? x : 0) | (e & 1 ? z : 0));
+#pragma unroll
+        for (int v = 0; v < N; ++v) {
+          const uint32_t j = uint32_t(l) | (uint32_t(v) << lt);
+          const int r = (j & x ? 2 : 0) | (j & z ? 1 : 0);
+          const double *m = d->m + 2 * (4 * r + (r ^ e));
+          y[v] = cadd(y[v], cmul(double2{m[0], m[1]}, p[v]));
+        }
+      }
+#pragma unroll
+      for (int v = 0; v < N; ++v) a[v] = y[v];
+    }
+  }
+  if (live) {
+#pragma unroll
+    for (int v = 0; v < N; ++v) dst[offset(v)] = double2{a[v].x * fs, a[v].y * fs};
+  }
+}
+
+template <int RB>
+__global__ __launch_bounds__(64, RB < 3 ? 3 : 2) void k_sweep_wave(const DevSweep sw, const pqs::WaveOp *__restrict__ stream,
+                                                   const pqs::WaveAngle *__restrict__ angles, int n_angles,
+                                                   const DevOp *__restrict__ ops, const DevTerm *__restrict__ terms,
+                                                   const InstDev *__restrict__ insts, int64_t n_active,
+                                                   const double2 *__restrict__ init_tab, int n, int s,
+                                                   int n_sweeps) {
+  __shared__ double2 lds[64 * (pqs::kWaveAngles + (1 << RB))];
+  const int lt = sw.k - RB;
+  const int64_t flat = (int64_t(blockIdx.x) << (6 - lt)) + (threadIdx.x >> lt);
+  const int64_t inst = flat / sw.n_tiles;
+  const bool live = inst < n_active;
+  const InstDev in = insts[live ? inst : n_active - 1];
+  wave_body<RB>(sw, stream, angles, n_angles, ops, terms, in, live, flat - inst * sw.n_tiles, init_tab, n, s, n_sweeps,
+                lds);
+}
+
 // ------------------------------------------------- launches that mix plans
 // A device record of a plan for launches that run instances of several
 // plans (uneven widths, depths) at once, and one work item per instance of
@@ -987,12 +1622,15 @@ struct PlanDev {
   const DevOp *ops;
   const DevTerm *terms;
   const DevPhase *phases;
+  const pqs::WaveOp *wave;  // wave executor plans: streams, angles, and where sweep s starts in each
+  const pqs::WaveAngle *angles;
   int32_t n_sweeps, n;
 };
 struct MultiItem {
   int64_t tile_begin;
   int32_t inst, plan;
   const void *init_tab;
+  int32_t wave0, angle0, n_angles, pad;  // of the item's sweep (wave executor)
 };
 
 __device__ __forceinline__ int find_item(const MultiItem *__restrict__ items, int n_items, int64_t b) {
@@ -1015,6 +1653,28 @@ __global__ __launch_bounds__(MAXT) void k_sweep_reg_multi(const PlanDev *__restr
   const InstDev in = insts[it.inst];
   sweep_reg_body<R, MAXT, LDSOPS>(pd.sweeps[s], pd.ops, pd.terms, pd.phases, in, b - it.tile_begin,
                                   static_cast<const typename CT<R>::V *>(it.init_tab), pd.n, s, pd.n_sweeps);
+}
+
+// One tile per wave: plans differ from block to block.
+__global__ __launch_bounds__(64) void k_sweep_wave_multi(const PlanDev *__restrict__ plans,
+                                                         const InstDev *__restrict__ insts,
+                                                         const MultiItem *__restrict__ items, int n_items, int s) {
+  __shared__ double2 lds[64 * (pqs::kWaveAngles + 8)];
+  const int64_t b = blockIdx.x;
+  const MultiItem it = items[find_item(items, n_items, b)];
+  const PlanDev pd = plans[it.plan];
+  const InstDev in = insts[it.inst];
+  const DevSweep &sw = pd.sweeps[s];
+  const int rb = pqs::wave_reg_bits(sw.k);
+  const bool live = threadIdx.x >> (sw.k - rb) == 0;
+  auto run = [&](auto r) {
+    wave_body<decltype(r)::value>(sw, pd.wave + it.wave0, pd.angles + it.angle0, it.n_angles, pd.ops, pd.terms, in,
+                                  live, b - it.tile_begin, static_cast<const double2 *>(it.init_tab), pd.n, s,
+                                  pd.n_sweeps, lds);
+  };
+  if (rb == 1) run(std::integral_constant<int, 1>{});
+  else if (rb == 2) run(std::integral_constant<int, 2>{});
+  else run(std::integral_constant<int, 3>{});
 }
 
 template <typename R, int BLOCK>
@@ -1929,9 +2589,11 @@ int plan_upload(pqs_ctx *ctx, pqs_plan *p, hipStream_t st) {
   const size_t tb = std::max<size_t>(1, p->dev_terms.size()) * sizeof(DevTerm);
   const size_t pb = std::max<size_t>(1, p->dev_phases.size()) * sizeof(pqs::DevPhase);
   const size_t sb = std::max<size_t>(1, p->dev_sweeps.size()) * sizeof(DevSweep);
-  void *d[4] = {nullptr, nullptr, nullptr, nullptr};
-  const size_t nb[4] = {ob, tb, pb, sb};
-  for (int i = 0; i < 4; ++i) {
+  const size_t wb = std::max<size_t>(1, p->dev_wave.size()) * sizeof(pqs::WaveOp);
+  const size_t ab = std::max<size_t>(1, p->dev_angles.size()) * sizeof(pqs::WaveAngle);
+  void *d[6] = {nullptr, nullptr, nullptr, nullptr, nullptr, nullptr};
+  const size_t nb[6] = {ob, tb, pb, sb, wb, ab};
+  for (int i = 0; i < 6; ++i) {
     const hipError_t e = hipMalloc(&d[i], nb[i]);
     if (e != hipSuccess) {
       for (int j = 0; j < i; ++j) (void)hipFree(d[j]);
@@ -1942,11 +2604,15 @@ int plan_upload(pqs_ctx *ctx, pqs_plan *p, hipStream_t st) {
   p->d_terms = d[1];
   p->d_phases = d[2];
   p->d_sweeps = d[3];
+  p->d_wave = d[4];
+  p->d_angles = d[5];
   p->dev_device = ctx->device;
   int rc = upload(ctx, p->d_ops, p->dev_ops.data(), p->dev_ops.size() * sizeof(DevOp), st);
   if (!rc) rc = upload(ctx, p->d_terms, p->dev_terms.data(), p->dev_terms.size() * sizeof(DevTerm), st);
   if (!rc) rc = upload(ctx, p->d_phases, p->dev_phases.data(), p->dev_phases.size() * sizeof(pqs::DevPhase), st);
   if (!rc) rc = upload(ctx, p->d_sweeps, p->dev_sweeps.data(), p->dev_sweeps.size() * sizeof(DevSweep), st);
+  if (!rc) rc = upload(ctx, p->d_wave, p->dev_wave.data(), p->dev_wave.size() * sizeof(pqs::WaveOp), st);
+  if (!rc) rc = upload(ctx, p->d_angles, p->dev_angles.data(), p->dev_angles.size() * sizeof(pqs::WaveAngle), st);
   if (rc) return rc;
   HIPCHECK(hipEventRecord((hipEvent_t)p->up_event, st));
   p->up_stream = (void *)st;
@@ -2012,24 +2678,35 @@ int jit_code_cached(const std::string &src, std::vector<char> &code, std::string
   return PQS_OK;
 }
 
-template <typename R, int BLOCK>
-int launch_sweep_t(pqs_ctx *ctx, pqs_plan *p, int s, const InstDev *d_insts, int64_t n_active,
-                   const void *init_tab, hipStream_t st) {
-  static bool attr_set[64] = {false};
+// complex64 tiles below 10 qubits: op by op, one wave per tile.
+int launch_sweep_ops(pqs_plan *p, int s, const InstDev *d_insts, int64_t n_active, const void *init_tab,
+                     hipStream_t st) {
   const DevSweep &sw = p->dev_sweeps[s];
-  size_t lds = (size_t(1) << sw.k) * sizeof(typename CT<R>::V);
-  if (int(lds) > ctx->max_lds) return fail(PQS_ERR_UNSUPPORTED, "tile does not fit in LDS");
-  auto kern = k_sweep<R, BLOCK>;
-  if (lds > 65536 && ctx->device < 64 && !attr_set[ctx->device]) {
-    HIPCHECK(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, ctx->max_lds));
-    attr_set[ctx->device] = true;
-  }
-  int64_t grid = sw.n_tiles * n_active;
+  const size_t lds = (size_t(1) << sw.k) * sizeof(float2);
+  const int64_t grid = sw.n_tiles * n_active;
   if (grid <= 0) return PQS_OK;
   if (grid > 0x7fffffff) return fail(PQS_ERR_UNSUPPORTED, "grid too large: split the batch");
-  hipLaunchKernelGGL(kern, dim3(unsigned(grid)), dim3(BLOCK), lds, st, sw, (const DevOp *)p->d_ops,
-                     (const DevTerm *)p->d_terms, d_insts, n_active,
-                     (const typename CT<R>::V *)init_tab, p->n, s, int(p->dev_sweeps.size()));
+  hipLaunchKernelGGL((k_sweep<float, 64>), dim3(unsigned(grid)), dim3(64), lds, st, sw, (const DevOp *)p->d_ops,
+                     (const DevTerm *)p->d_terms, d_insts, n_active, (const float2 *)init_tab, p->n, s,
+                     int(p->dev_sweeps.size()));
+  HIPCHECK(hipGetLastError());
+  return PQS_OK;
+}
+
+int launch_sweep_wave(pqs_plan *p, int s, const InstDev *d_insts, int64_t n_active, const void *init_tab,
+                      hipStream_t st) {
+  const DevSweep &sw = p->dev_sweeps[s];
+  if (n_active <= 0) return PQS_OK;
+  const int rb = pqs::wave_reg_bits(sw.k), per = 64 >> (sw.k - rb);  // tiles per wave
+  const int64_t grid = (sw.n_tiles * n_active + per - 1) / per;
+  if (grid > 0x7fffffff) return fail(PQS_ERR_UNSUPPORTED, "grid too large: split the batch");
+  const int a0 = p->angle_begin[size_t(s)], na = p->angle_begin[size_t(s) + 1] - a0;
+  auto kern = rb == 1 ? k_sweep_wave<1> : rb == 2 ? k_sweep_wave<2> : k_sweep_wave<3>;
+  hipLaunchKernelGGL(kern, dim3(unsigned(grid)), dim3(64), 0, st, sw,
+                     (const pqs::WaveOp *)p->d_wave + p->wave_begin[size_t(s)],
+                     (const pqs::WaveAngle *)p->d_angles + a0, na, (const DevOp *)p->d_ops,
+                     (const DevTerm *)p->d_terms, d_insts, n_active, (const double2 *)init_tab, p->n, s,
+                     int(p->dev_sweeps.size()));
   HIPCHECK(hipGetLastError());
   return PQS_OK;
 }
@@ -2086,22 +2763,10 @@ int launch_sweep_one(pqs_ctx *ctx, pqs_plan *p, int s, const InstDev *d_insts, i
                                    args, nullptr));
     return PQS_OK;
   }
-  if (p->reg_exec) {
-    if (p->dtype == PQS_C128) return launch_sweep_reg<double>(ctx, p, s, d_insts, n_active, init_tab, st);
-    return launch_sweep_reg<float>(ctx, p, s, d_insts, n_active, init_tab, st);
-  }
-  if (p->dtype == PQS_C128) {
-    switch (p->block) {
-      case 256: return launch_sweep_t<double, 256>(ctx, p, s, d_insts, n_active, init_tab, st);
-      case 512: return launch_sweep_t<double, 512>(ctx, p, s, d_insts, n_active, init_tab, st);
-      default: return launch_sweep_t<double, 1024>(ctx, p, s, d_insts, n_active, init_tab, st);
-    }
-  }
-  switch (p->block) {
-    case 256: return launch_sweep_t<float, 256>(ctx, p, s, d_insts, n_active, init_tab, st);
-    case 512: return launch_sweep_t<float, 512>(ctx, p, s, d_insts, n_active, init_tab, st);
-    default: return launch_sweep_t<float, 1024>(ctx, p, s, d_insts, n_active, init_tab, st);
-  }
+  if (p->wave_exec) return launch_sweep_wave(p, s, d_insts, n_active, init_tab, st);
+  if (!p->reg_exec) return launch_sweep_ops(p, s, d_insts, n_active, init_tab, st);
+  if (p->dtype == PQS_C128) return launch_sweep_reg<double>(ctx, p, s, d_insts, n_active, init_tab, st);
+  return launch_sweep_reg<float>(ctx, p, s, d_insts, n_active, init_tab, st);
 }
 
 // One sweep over n_active instances.  With a block cap on the context the
@@ -2238,6 +2903,8 @@ int pqs_plan_destroy(pqs_plan *p) {
     if (p->d_terms) (void)hipFree(p->d_terms);
     if (p->d_phases) (void)hipFree(p->d_phases);
     if (p->d_sweeps) (void)hipFree(p->d_sweeps);
+    if (p->d_wave) (void)hipFree(p->d_wave);
+    if (p->d_angles) (void)hipFree(p->d_angles);
     for (void *m : p->jit_modules) (void)hipModuleUnload((hipModule_t)m);
   }
   if (p->up_event) (void)hipEventDestroy((hipEvent_t)p->up_event);
@@ -2517,8 +3184,8 @@ int pqs_run_multi(pqs_ctx *ctx, pqs_plan *const *plans, int32_t n_plans, const p
   }
   const size_t ab = amp_bytes(dtype);
   // launch groups: register-phase plans by tile size (one block size per
-  // launch), the per-op LDS plans (tiles below 10 qubits) together
-  auto group_of = [&](const pqs_plan *p) { return p->reg_exec ? p->tile_bits : 0; };
+  // launch), smaller tiles together
+  auto group_of = [&](const pqs_plan *p) { return p->wave_exec ? -1 : p->reg_exec ? p->tile_bits : 0; };
   std::vector<InstDev> h(static_cast<size_t>(n_inst));
   size_t alt_rows_b = 0;
   std::vector<size_t> alt_off(size_t(n_inst), 0);
@@ -2574,6 +3241,11 @@ int pqs_run_multi(pqs_ctx *ctx, pqs_plan *const *plans, int32_t n_plans, const p
         it.inst = int32_t(i);
         it.plan = inst_plan[i];
         it.init_tab = init_tabs ? init_tabs[i] : nullptr;
+        if (p->wave_exec) {
+          it.wave0 = p->wave_begin[size_t(r)];
+          it.angle0 = p->angle_begin[size_t(r)];
+          it.n_angles = p->angle_begin[size_t(r) + 1] - it.angle0;
+        }
         items.push_back(it);
         L.tiles += sw.n_tiles;
         size_t lds = (size_t(1) << sw.k) * ab;
@@ -2589,7 +3261,8 @@ int pqs_run_multi(pqs_ctx *ctx, pqs_plan *const *plans, int32_t n_plans, const p
   for (int32_t k = 0; k < n_plans; ++k) {
     const pqs_plan *p = plans[k];
     pdv[size_t(k)] = PlanDev{(const DevSweep *)p->d_sweeps, (const DevOp *)p->d_ops, (const DevTerm *)p->d_terms,
-                             (const DevPhase *)p->d_phases, int32_t(p->dev_sweeps.size()), p->n};
+                             (const DevPhase *)p->d_phases, (const pqs::WaveOp *)p->d_wave,
+                             (const pqs::WaveAngle *)p->d_angles, int32_t(p->dev_sweeps.size()), p->n};
   }
   // workspace: [alt rows | instance table | plan records | items]
   auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
@@ -2652,12 +3325,11 @@ int pqs_run_multi(pqs_ctx *ctx, pqs_plan *const *plans, int32_t n_plans, const p
         auto kern = L.ldsops ? k_sweep_reg_multi<float, 1024, true> : k_sweep_reg_multi<float, 1024, false>;
         hipLaunchKernelGGL(kern, dim3(unsigned(L.tiles)), dim3(nthr), L.lds, st, d_pd, d_tab, its, ni, L.round);
       }
-    } else if (dtype == PQS_C128) {
-      hipLaunchKernelGGL((k_sweep_multi<double, 256>), dim3(unsigned(L.tiles)), dim3(256), L.lds, st, d_pd, d_tab,
-                         its, ni, L.round);
+    } else if (L.group_k < 0) {
+      hipLaunchKernelGGL(k_sweep_wave_multi, dim3(unsigned(L.tiles)), dim3(64), 0, st, d_pd, d_tab, its, ni, L.round);
     } else {
-      hipLaunchKernelGGL((k_sweep_multi<float, 256>), dim3(unsigned(L.tiles)), dim3(256), L.lds, st, d_pd, d_tab,
-                         its, ni, L.round);
+      hipLaunchKernelGGL((k_sweep_multi<float, 64>), dim3(unsigned(L.tiles)), dim3(64), L.lds, st, d_pd, d_tab, its,
+                         ni, L.round);
     }
     HIPCHECK(hipGetLastError());
   }

@@ -89,17 +89,9 @@ static void masks_of(int n, const pqs_op &o, qmask &active, qmask &diag) {
     }
     case PQS_OP_RX: case PQS_OP_RY: active |= bitq(o.q0); break;
     case PQS_OP_RZ: diag |= bitq(o.q0); break;
-    case PQS_OP_MAT2: {
-      bool d = true;
-      for (int r = 0; r < 4; ++r)
-        for (int c = 0; c < 4; ++c)
-          if (r != c && (o.m[2 * (4 * r + c)] != 0 || o.m[2 * (4 * r + c) + 1] != 0)) d = false;
-      (d ? diag : active) |= bitq(o.q0) | bitq(o.q1);
-      break;
-    }
     case PQS_OP_CX: diag |= bitq(o.q0); active |= bitq(o.q1); break;
     case PQS_OP_CZ: case PQS_OP_RZZ: diag |= bitq(o.q0) | bitq(o.q1); break;
-    case PQS_OP_RXX: case PQS_OP_RYY: case PQS_OP_FSIM: case PQS_OP_GEN_FSIM:
+    case PQS_OP_MAT2: case PQS_OP_RXX: case PQS_OP_RYY: case PQS_OP_FSIM: case PQS_OP_GEN_FSIM:
       active |= bitq(o.q0) | bitq(o.q1);
       break;
     case PQS_OP_GEN: {
@@ -109,6 +101,216 @@ static void masks_of(int n, const pqs_op &o, qmask &active, qmask &diag) {
       break;
     }
   }
+}
+
+// The op stream of one sweep for the wave executor.  Ops that commute past
+// the deferred ones are gathered into one record: equal rotations on distinct
+// qubits (a layer record, where they cover at least half of the tile), and
+// runs of CNOTs (one index map).  An angle refill covers the next kWaveAngles
+// angles per lane of a tile; ops refer to it by their position in it.  A
+// growth check every 10 rotations applies the accumulated scale early (the
+// scaled rotation form of the specialised kernels, with their bound).
+static void wave_stream(pqs_plan &p, const DevSweep &ds) {
+  p.wave_begin.push_back(int(p.dev_wave.size()));
+  p.angle_begin.push_back(int(p.dev_angles.size()));
+  const int k = ds.k, per_refill = kWaveAngles << (k - wave_reg_bits(k));
+  auto emit = [&](int code) -> WaveOp & {
+    WaveOp w{};
+    w.code = uint16_t(code);
+    w.tangent = -1;
+    p.dev_wave.push_back(w);
+    return p.dev_wave.back();
+  };
+  int n_ang = 0, refill_at = -1, refill_first = 0, rot = 0;
+  // room for `need` angles in the current refill
+  auto reserve = [&](int need) {
+    if (refill_at >= 0 && n_ang + need - refill_first <= per_refill) return;
+    refill_at = int(p.dev_wave.size());
+    refill_first = n_ang;
+    emit(kWRefill).c = n_ang;
+  };
+  auto angle = [&](double scale, double offset, int slot) {
+    WaveAngle w{};
+    w.scale = scale;
+    w.offset = offset;
+    w.slot = slot;
+    p.dev_angles.push_back(w);
+    ++n_ang;
+    p.dev_wave[size_t(refill_at)].x = uint32_t(n_ang - refill_first);
+    return uint16_t(n_ang - 1 - refill_first);
+  };
+  auto rotations = [&](int count) {  // at most 10 between two checks
+    if (rot + count > 10) {
+      emit(kWCheck);
+      rot = 0;
+    }
+    rot += count;
+  };
+  auto single = [&](int o) {
+    const DevOp &d = p.dev_ops[size_t(o)];
+    const uint32_t b0 = d.t0 >= 0 ? 1u << d.t0 : 0, b1 = d.t1 >= 0 ? 1u << d.t1 : 0;
+    const uint64_t h0 = d.t0 < 0 && d.g0 >= 0 ? uint64_t(1) << d.g0 : 0;
+    const uint64_t h1 = d.t1 < 0 && d.g1 >= 0 ? uint64_t(1) << d.g1 : 0;
+    // exp(-i a/2 P) = cos (1 - i t P), P = i^y (-1)^{(j ^ x).z} X^x on a[j ^ x]
+    auto rotation = [&](uint32_t x, uint32_t z, uint64_t zg, int y) {
+      rotations(1);
+      reserve(1);
+      const uint16_t a = angle(d.scale, d.offset, d.slot);
+      WaveOp &w = emit(!x ? kWPhase : y & 1 ? kWRotR : kWRotI);
+      w.ang = a;
+      w.x = x;
+      w.z = z;
+      w.zg = zg;
+      // -i i^y: -i (y = 0), 1 (y = 1), i (y = 2); times (-1)^{x.z}
+      w.c = (__builtin_popcount(x & z) & 1) ^ (y == 2 ? 1 : 0);
+    };
+    switch (d.kind) {
+      case PQS_OP_RX: rotation(b0, 0, 0, 0); break;
+      case PQS_OP_RY: rotation(b0, b0, 0, 1); break;
+      case PQS_OP_RZ: rotation(0, b0, h0, 0); break;
+      case PQS_OP_RZZ: rotation(0, b0 | b1, h0 | h1, 0); break;
+      case PQS_OP_RXX: rotation(b0 | b1, 0, 0, 0); break;
+      case PQS_OP_RYY: rotation(b0 | b1, b0 | b1, 0, 2); break;
+      case PQS_OP_CX: {
+        WaveOp &w = emit(kWCx);
+        w.x = b1;
+        w.zg = h0;
+        break;
+      }
+      case PQS_OP_CZ: {
+        WaveOp &w = emit(kWCz);
+        w.z = b0 | b1;
+        w.zg = h0 | h1;
+        break;
+      }
+      case PQS_OP_MAT1: {
+        const bool diag = d.m[2] == 0 && d.m[3] == 0 && d.m[4] == 0 && d.m[5] == 0;
+        WaveOp &w = emit(kWMat1);
+        w.x = diag ? 0 : b0;
+        w.z = b0;
+        w.zg = h0;
+        w.c = o;
+        break;
+      }
+      case kPauliSum: {
+        WaveOp &w = emit(kWSum);
+        w.c = o;
+        w.tangent = d.tangent;
+        break;
+      }
+      case PQS_OP_FSIM:
+      case PQS_OP_GEN_FSIM: {
+        reserve(2);
+        // doubled: the table holds (tan, cos) of half of each angle
+        const uint16_t a = angle(2 * d.scale, 2 * d.offset, d.slot);
+        const uint32_t f = d.slot2 >= 0 ? angle(2.0, 0.0, d.slot2) : 0xffffffffu;
+        WaveOp &w = emit(d.kind == PQS_OP_FSIM ? kWFsim : kWGenFsim);
+        w.ang = a;
+        w.x = b0 | b1;
+        w.z = f;
+        w.c = o;
+        w.tangent = d.tangent;
+        break;
+      }
+      default: {  // PQS_OP_MAT2
+        WaveOp &w = emit(kWMat2);
+        w.x = b0;
+        w.z = b1;
+        w.c = o;
+        break;
+      }
+    }
+  };
+  // qubits an op acts on, as positions: non-diagonally and at all
+  auto masks = [&](int o, uint64_t &act, uint64_t &all) {
+    const DevOp &d = p.dev_ops[size_t(o)];
+    const uint64_t b0 = d.g0 >= 0 ? uint64_t(1) << d.g0 : 0, b1 = d.g1 >= 0 ? uint64_t(1) << d.g1 : 0;
+    act = 0;
+    all = b0 | b1;
+    switch (d.kind) {
+      case PQS_OP_RZ: case PQS_OP_RZZ: case PQS_OP_CZ: break;
+      case PQS_OP_CX: act = b1; break;
+      case kPauliSum: act = all = ~uint64_t(0); break;  // a point that nothing passes
+      default: act = all; break;
+    }
+  };
+  auto in_tile = [&](const DevOp &d) { return d.t0 >= 0 && (d.g1 < 0 || d.t1 >= 0); };
+  std::vector<int> rem, rest, got;
+  for (int o = ds.op_begin; o < ds.op_end; ++o) rem.push_back(o);
+  while (!rem.empty()) {
+    const int kind = p.dev_ops[size_t(rem[0])].kind;
+    const bool layer = (kind == PQS_OP_RX || kind == PQS_OP_RY || kind == PQS_OP_RZ) &&
+                       in_tile(p.dev_ops[size_t(rem[0])]);
+    const bool map = kind == PQS_OP_CX && in_tile(p.dev_ops[size_t(rem[0])]);
+    got.assign(1, rem[0]);
+    rest.clear();
+    if (layer || map) {
+      uint64_t blocked_any = 0, blocked_act = 0;
+      uint32_t taken = layer ? 1u << p.dev_ops[size_t(rem[0])].t0 : 0;
+      for (size_t i = 1; i < rem.size(); ++i) {
+        const DevOp &d = p.dev_ops[size_t(rem[i])];
+        uint64_t act, all;
+        masks(rem[i], act, all);
+        const bool free = !(act & blocked_any) && !(all & blocked_act);
+        if (free && d.kind == kind && in_tile(d) && (map || !((taken >> d.t0) & 1))) {
+          got.push_back(rem[i]);
+          if (layer) taken |= 1u << d.t0;
+        } else {
+          rest.push_back(rem[i]);
+          blocked_any |= all;
+          blocked_act |= act;
+          if (blocked_act == ~uint64_t(0)) {  // nothing further can pass
+            rest.insert(rest.end(), rem.begin() + long(i) + 1, rem.end());
+            break;
+          }
+        }
+      }
+    } else {
+      rest.assign(rem.begin() + 1, rem.end());
+    }
+    if (layer && 2 * int(got.size()) >= k) {
+      rotations(k);
+      reserve(k);
+      int first = -1;
+      for (int t = 0; t < k; ++t) {
+        uint16_t a = 0;
+        bool found = false;
+        for (int o : got) {
+          const DevOp &d = p.dev_ops[size_t(o)];
+          if (d.t0 != t) continue;
+          a = angle(d.scale, d.offset, d.slot);
+          found = true;
+        }
+        if (!found) a = angle(0.0, 0.0, -1);
+        if (first < 0) first = a;
+      }
+      WaveOp &w = emit(kind == PQS_OP_RX ? kWLayerRx : kind == PQS_OP_RY ? kWLayerRy : kWLayerRz);
+      w.ang = uint16_t(first);
+    } else if (map) {
+      // a CNOT sets a'[j] = a[j ^ (bit c of j) << t]; a run of them, first
+      // one applied first: a'[j] = a[m_1(m_2(.. m_g(j)))]
+      uint16_t m[kWaveTile + 1];
+      for (int t = 0; t <= kWaveTile; ++t) m[t] = uint16_t(t < k ? 1u << t : 0);
+      for (int o : got) {
+        const DevOp &d = p.dev_ops[size_t(o)];
+        // append: m <- m . m_o, whose only changed column is the control's
+        m[d.t0] = uint16_t(m[d.t0] ^ m[d.t1]);
+      }
+      WaveOp &w = emit(kWMap);
+      auto pair = [&](int t) { return uint32_t(m[t]) | (uint32_t(m[t + 1]) << 16); };
+      w.x = pair(0);
+      w.z = pair(2);
+      w.zg = uint64_t(pair(4)) | (uint64_t(pair(6)) << 32);
+      w.c = int32_t(pair(8));
+    } else {
+      for (int o : got) single(o);
+    }
+    rem.swap(rest);
+  }
+  // whole blocks of 64 records, and one block more that is loaded ahead
+  do emit(kWEnd);
+  while ((p.dev_wave.size() - size_t(p.wave_begin.back())) % 64 != 0);
+  for (int i = 0; i < 64; ++i) emit(kWEnd);
 }
 
 int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_opts *opts) {
@@ -269,7 +471,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
         qmask touched = e.active | e.diag;
         bool dep = (touched & blocked_nd) || (e.active & blocked_any);
         bool ok = false;
-        if (n_angle >= kMaxSweepOps) dep = true;  // the sweep's LDS op table is full
+        if (n_angle >= kMaxSweepOps && k > kWaveTile) dep = true;  // the sweep's LDS op table is full
         if (!dep) {
           qmask need = e.active & ~T;
           if (popc(T | need) <= k) {
@@ -476,9 +678,18 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
     }
 
   // ---- register phases and device image
-  // Tiles of >= 11 qubits use the register-phase executor: 2^kRegBits
-  // amplitudes per thread, so at least one full wave per tile.
-  p.reg_exec = p.tile_bits >= kRegBits + 6;  // at least one full wave per tile
+  // Tiles of kRegBits + 6 qubits and more fill at least one wave with
+  // 2^kRegBits amplitudes per thread: the register-phase executor.  Smaller
+  // complex128 tiles go to the wave executor; smaller complex64 ones stay with
+  // the op-by-op executor (and complex64 two-qubit gates with LDS phases,
+  // below): another order of single-precision roundings would show in every
+  // QFIM and overlap of such states.
+  p.reg_exec = p.tile_bits >= kRegBits + 6;
+  p.wave_exec = !p.reg_exec && p.dtype == PQS_C128;
+  p.dev_wave.clear();
+  p.dev_angles.clear();
+  p.wave_begin.clear();
+  p.angle_begin.clear();
   p.dev_ops.clear();
   p.dev_terms.clear();
   p.dev_sweeps.clear();
@@ -543,6 +754,9 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
         const ExecOp &e = p.exec[ei];
         const int kind = e.kind;
         if (kind == kPauliSum) return e.n_src == 1 && ops[e.first].q1 < 0;  // one Pauli on one qubit
+        if (kind == PQS_OP_MAT2 || kind == PQS_OP_RXX || kind == PQS_OP_RYY || kind == PQS_OP_FSIM ||
+            kind == PQS_OP_GEN_FSIM)
+          return p.dtype == PQS_C128;  // both qubits become register bits
         return kind == PQS_OP_MAT1 || kind == PQS_OP_RX || kind == PQS_OP_RY || kind == PQS_OP_RZ ||
                kind == PQS_OP_CX || kind == PQS_OP_CZ || kind == PQS_OP_RZZ;
       };
@@ -1005,7 +1219,8 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
             return fail(PQS_ERR_UNSUPPORTED, "internal planner error: active qubit not in registers");
         }
         if (p.reg_exec && !ph.lds &&
-            (d.kind == PQS_OP_RX || d.kind == PQS_OP_RY || d.kind == PQS_OP_RZ || d.kind == PQS_OP_RZZ))
+            (d.kind == PQS_OP_RX || d.kind == PQS_OP_RY || d.kind == PQS_OP_RZ || d.kind == PQS_OP_RZZ ||
+             d.kind == PQS_OP_RXX || d.kind == PQS_OP_RYY))
           d.coef = n_coef++;
         if (d.kind == kPauliSum) {
           d.term0 = int(p.dev_terms.size());
@@ -1050,8 +1265,18 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
     ds.n_coef = 0;
     for (const PhaseSpec &ph : phases)
       if (ph.lds) ds.n_coef = 1;
+    for (int o = ds.op_begin; o < ds.op_end; ++o) {
+      const int kd = p.dev_ops[size_t(o)].kind;
+      if (kd == PQS_OP_MAT2 || kd == PQS_OP_RXX || kd == PQS_OP_RYY || kd == PQS_OP_FSIM || kd == PQS_OP_GEN_FSIM)
+        ds.n_coef = 1;
+    }
     (void)n_coef;
     p.dev_sweeps.push_back(ds);
+    if (p.wave_exec) wave_stream(p, ds);
+  }
+  if (p.wave_exec) {
+    p.wave_begin.push_back(int(p.dev_wave.size()));
+    p.angle_begin.push_back(int(p.dev_angles.size()));
   }
   return PQS_OK;
 }

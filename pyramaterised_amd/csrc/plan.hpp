@@ -57,7 +57,7 @@ struct alignas(16) DevTerm {
   double cre, cim;  // coefficient including i^{#Y}
 };
 
-// Register-phase executor: each thread holds 2^kRegBits amplitudes of the
+// Register-phase executors: each thread holds 2^kRegBits amplitudes of the
 // tile, over kRegBits tile bits chosen per phase.
 constexpr int kRegBits = 4;
 constexpr int kMaxSweepOps = 896;  // op records staged in LDS per sweep (28 KiB)
@@ -88,7 +88,7 @@ struct DevSweep {
   int32_t crun_pos[kMaxQubits], crun_len[kMaxQubits], crun_shift[kMaxQubits];
   int64_t n_tiles;
   int32_t phase_begin, phase_end;  // register phases (reg executor only)
-  int32_t n_coef;                  // 1: the sweep has LDS phases (dense 2q ops, generators)
+  int32_t n_coef;                  // 1: the sweep has LDS phases (Pauli sums) or dense two-qubit ops
   // Write layout (rolling plans): the tile is stored through a permutation
   // of its bits, store index bit i <-> tile bit sperm[i], ordered by
   // ascending write position wpos[sperm[i]]; complement (tile id) bit j is
@@ -101,6 +101,49 @@ struct DevSweep {
   // first (last) register phase, so the specialised kernel loads (stores)
   // that phase's registers directly, without staging the tile in LDS.
   int32_t direct_load, direct_store;
+};
+
+// ---- op stream of the wave executor (complex128 tiles below 10 qubits)
+// A tile of k qubits lies over 2^(k - r) lanes of a wave, 2^r amplitudes per
+// lane (wave_reg_bits); 64 >> (k - r) tiles share a wave, which walks one
+// stream per sweep.  Amplitude index j: lane part in the low bits, register
+// part in the top r.  Circuits come in layers, and so does the stream: one
+// record rotates every bit, or applies a whole run of CNOTs as one index map.
+// Every other op has the form a'[j] = D(j) a[j] + O(j) a[j ^ x] with D and O
+// depending on parities of j, so few codes cover all ops and bits are data.
+constexpr int kWaveTile = 9;    // largest tile of the wave executor
+constexpr int kWaveAngles = 4;  // angles per lane and refill
+constexpr int wave_reg_bits(int k) { return k == 1 ? 1 : k == 9 ? 3 : 2; }
+enum WaveCode : int32_t {
+  kWEnd = 0,
+  kWRefill,   // c: first angle, x: count
+  kWCheck,    // growth check of the scaled rotations
+  kWLayerRx,  // R_x on every bit, angles ang .. ang + k - 1 (identity: angle 0)
+  kWLayerRy,
+  kWLayerRz,
+  kWMap,      // a'[j] = a[m(j)], m linear: the masks of m on bits 0, 1, .. are the
+              // 16-bit halves of x, z, zg, c
+  kWRotI,     // a - (+) i t (-1)^{j.z} a[j ^ x] (c: 1 flips the sign)
+  kWRotR,     // a + (-) t (-1)^{j.z} a[j ^ x] (c: 1 flips the sign)
+  kWPhase,    // kWRotI with x = 0
+  kWCx,       // control outside the tile: a[j ^ x] where zg's bit is set
+  kWCz,       // -1 where all bits of z and zg are set
+  kWMat1,     // 2x2 of DevOp c on bit z (x = z, or 0 for a diagonal one)
+  kWSum,      // Pauli sum of DevOp c, for its tangent
+  kWFsim,     // on bits x: theta at ang, phi at z (-1: phi = 0)
+  kWGenFsim,  // as kWFsim, DevOp c, for its tangent
+  kWMat2      // 4x4 of DevOp c, q0 = bit x, q1 = bit z
+};
+struct alignas(16) WaveOp {
+  uint16_t code, ang;  // ang: index into the angles of the last refill
+  uint32_t x, z;       // masks over the tile index
+  int32_t c;
+  uint64_t zg;         // mask over the tile's global position bits, with z
+  int32_t tangent, pad;
+};
+struct alignas(8) WaveAngle {  // the rotation's angle: scale * params[slot] + offset
+  double scale, offset;
+  int32_t slot, pad;
 };
 
 std::string plan_error(); // last planner error (thread local)
@@ -131,7 +174,11 @@ struct pqs_plan {
   std::vector<pqs::DevTerm> dev_terms;
   std::vector<pqs::DevSweep> dev_sweeps;
   std::vector<pqs::DevPhase> dev_phases;
-  bool reg_exec = false;  // sweeps carry register phases
+  std::vector<pqs::WaveOp> dev_wave;      // wave executor: every sweep's stream
+  std::vector<pqs::WaveAngle> dev_angles; // and its angles
+  std::vector<int> wave_begin, angle_begin;  // per sweep (one entry more than sweeps)
+  bool reg_exec = false;   // sweeps carry register phases
+  bool wave_exec = false;  // the wave executor runs the sweeps
 
   // device copy (per plan, on the device of the first context that ran it)
   int dev_device = -1;
@@ -139,6 +186,8 @@ struct pqs_plan {
   void *d_terms = nullptr;
   void *d_phases = nullptr;
   void *d_sweeps = nullptr;  // DevSweep records (launches that mix plans)
+  void *d_wave = nullptr;    // wave executor: streams and angles
+  void *d_angles = nullptr;
   // the arrays are copied in stream order on the stream of the plan's first
   // launch; launches on other streams wait for this event until it has run
   void *up_event = nullptr;   // hipEvent_t
