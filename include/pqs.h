@@ -411,10 +411,11 @@ int pqs_abs2(pqs_ctx *ctx, const double *z_dev, int64_t n, double *out_dev, void
 int pqs_magic(pqs_ctx *ctx, int32_t dtype, const void *states_dev, int32_t n_qubits,
               int64_t batch, double alpha, double *out_dev, void *stream);
 
-/* Run-time specialisation (hiprtc) of the plan's sweeps: every sweep made of
- * one-qubit rotations, fixed one-qubit matrices, CNOT, CZ and R_zz gets its
- * own straight-line kernel with register and bit indices as constants; other
- * sweeps stay interpreted.  load = 0 compiles only (no device needed, used
+/* Run-time specialisation (hiprtc) of the plan's sweeps: every sweep (in
+ * complex64, every sweep made of one-qubit rotations, fixed one-qubit
+ * matrices, CNOT, CZ and R_zz) gets its own straight-line kernel with register
+ * and bit indices as constants; other sweeps, and tiles below 10 qubits, stay
+ * interpreted.  load = 0 compiles only (no device needed, used
  * to check generated code); load = 1 also loads the module on ctx's device,
  * after which pqs_run / pqs_run_batch / pqs_jacobian launch the specialised
  * kernels.  No reference counterpart (the reference has no kernels). */
