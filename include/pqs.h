@@ -348,6 +348,14 @@ int pqs_gram(pqs_ctx *ctx, int32_t dtype, const void *a_dev, int64_t lda, int64_
              const void *b_dev, int64_t ldb, int64_t n, int64_t dim,
              double *out_dev, void *stream);
 
+/* |<a_i|a_j>|^2 for i < j in the order (0, 1), (0, 2), .., (1, 2), .. of m >= 2
+ * rows of length dim, row stride ld (amplitudes), into out_dev (m (m - 1) / 2
+ * float64).  Replaces the pair loop of Measurements._gen_f_samples
+ * (measure.py:131-137): the upper triangle of the Gram, its squared moduli
+ * formed where its partial sums are added up. */
+int pqs_pair_fidelities(pqs_ctx *ctx, int32_t dtype, const void *states_dev, int64_t ld, int64_t m, int64_t dim,
+                        double *out_dev, void *stream);
+
 /* QFIM from a Jacobian and the state: F_pq = 4 Re(<J_p|J_q> - <J_p|psi><psi|J_q>)
  * into f_dev (P x P float64).  Replaces Measurements.get_QFI
  * (measure.py:33-71).  complex128 forms Re(J J^dag) = R R^T, R = J viewed as a

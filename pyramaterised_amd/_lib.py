@@ -76,6 +76,7 @@ SIGNATURES = {
     "pqs_inner": (C.c_int, [vp, i32, vp, i64, vp, vp, i64, vp, vp]),
     "pqs_mw": (C.c_int, [vp, i32, vp, i32, i64, vp, vp, vp]),
     "pqs_gram": (C.c_int, [vp, i32, vp, i64, i64, vp, i64, i64, i64, vp, vp]),
+    "pqs_pair_fidelities": (C.c_int, [vp, i32, vp, i64, i64, i64, vp, vp]),
     "pqs_qfim": (C.c_int, [vp, i32, vp, i64, vp, i64, vp, vp]),
     "pqs_expect_pauli": (C.c_int, [vp, i32, vp, i32, i64, vp, vp, vp, i32, vp, vp]),
     "pqs_histogram": (C.c_int, [vp, vp, i64, vp, i32, vp, vp]),

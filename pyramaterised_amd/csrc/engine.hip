@@ -1312,14 +1312,17 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
 #pragma unroll
     for (int v = 0; v < N; ++v) p[v] = tile[uint32_t(l | (v << lt)) ^ x];
   };
+  int block = 0;  // of 64 records, held
 #pragma unroll 1
   for (int o = 0;; ++o) {
     const int i = o & 63;
-    if (i == 0 && o) {  // streams are padded to whole blocks of 64 and one more
+    if ((o >> 6) != block) {  // streams are padded to whole blocks of 64 and one more
+      const bool step = (o >> 6) == block + 1;
+      block = o >> 6;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        held[h] = next[h];
-        next[h] = recs[2 * (o + 64 + lane) + h];
+        held[h] = step ? next[h] : recs[2 * (64 * block + lane) + h];
+        next[h] = recs[2 * (64 * block + 64 + lane) + h];
       }
     }
     const uint32_t w0 = field(held[0].x, i);
@@ -1398,6 +1401,10 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
     }
     const uint32_t x = field(held[0].y, i), z = field(held[0].z, i);
     const int c = int(field(held[0].w, i));
+    if (code == pqs::kWSkip) {
+      if (!__ballot(live && in.tangent >= int(z) && in.tangent <= c)) o += int(x);
+      continue;
+    }
     if (code == pqs::kWRefill) {
       // ops before this one have read their angles (LDS in order)
 #pragma unroll
@@ -1898,19 +1905,23 @@ __device__ __forceinline__ double2 syrk_ld2(const char *p) {
 // launch).  Every chunk is a whole number of ring turns (the host pads K),
 // so no step needs masking; the last turn's prefetches (never used) re-read
 // the chunk's first step instead of running past it.
-template <typename TIn, bool DIAG>
+// EDGE: a tile with fewer than 64 rows or columns left skips the 16 x 16 blocks
+// past them (na, nb blocks are left).
+template <typename TIn, bool DIAG, bool EDGE>
 __device__ __forceinline__ void syrk_wave_body(const TIn *R, const uint32_t (&oa)[4], const uint32_t (&ob)[4],
-                                               const TIn *psi, int64_t k0, int64_t k1, int g, int col,
+                                               const TIn *psi, int64_t k0, int64_t k1, int g, int col, int na, int nb,
                                                d4_t (&acc)[4][4], d4_t (&accb)[4]) {
   double2 A[SYRING][4], B[SYRING][4];
   auto load = [&](double2(&X)[4], double2(&Y)[4], int64_t kk) {
     const int64_t kl = kk < k1 ? kk : k0;
     const char *base = reinterpret_cast<const char *>(R + kl);
 #pragma unroll
-    for (int a = 0; a < 4; ++a) X[a] = syrk_ld2<TIn>(base + oa[a]);
+    for (int a = 0; a < 4; ++a)
+      if (!EDGE || a < na) X[a] = syrk_ld2<TIn>(base + oa[a]);
     if constexpr (!DIAG) {
 #pragma unroll
-      for (int b = 0; b < 4; ++b) Y[b] = syrk_ld2<TIn>(base + ob[b]);
+      for (int b = 0; b < 4; ++b)
+        if (!EDGE || b < nb) Y[b] = syrk_ld2<TIn>(base + ob[b]);
     } else {
       // the b vector's operand: column 0 pairs (Re, Im) of a row with
       // (Re psi, Im psi), column 1 with (Im psi, -Re psi), the rest zero
@@ -1925,23 +1936,25 @@ __device__ __forceinline__ void syrk_wave_body(const TIn *R, const uint32_t (&oa
     for (int a = 0; a < 4; ++a)
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        if (DIAG && a > b) continue;
+        if ((DIAG && a > b) || (EDGE && (a >= na || b >= nb))) continue;
         acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[a].x, DIAG ? X[b].x : Y[b].x, acc[a][b], 0, 0, 0);
       }
     if constexpr (DIAG) {
 #pragma unroll
-      for (int a = 0; a < 4; ++a) accb[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[a].x, Y[0].x, accb[a], 0, 0, 0);
+      for (int a = 0; a < 4; ++a)
+        if (!EDGE || a < na) accb[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[a].x, Y[0].x, accb[a], 0, 0, 0);
     }
 #pragma unroll
     for (int a = 0; a < 4; ++a)
 #pragma unroll
       for (int b = 0; b < 4; ++b) {
-        if (DIAG && a > b) continue;
+        if ((DIAG && a > b) || (EDGE && (a >= na || b >= nb))) continue;
         acc[a][b] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[a].y, DIAG ? X[b].y : Y[b].y, acc[a][b], 0, 0, 0);
       }
     if constexpr (DIAG) {
 #pragma unroll
-      for (int a = 0; a < 4; ++a) accb[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[a].y, Y[0].y, accb[a], 0, 0, 0);
+      for (int a = 0; a < 4; ++a)
+        if (!EDGE || a < na) accb[a] = __builtin_amdgcn_mfma_f64_16x16x4f64(X[a].y, Y[0].y, accb[a], 0, 0, 0);
     }
   };
 #pragma unroll
@@ -1955,6 +1968,14 @@ __device__ __forceinline__ void syrk_wave_body(const TIn *R, const uint32_t (&oa
   }
 }
 
+// Tile t of the upper triangle, row by row: row x starts at column step * x of
+// nt.
+__device__ __forceinline__ int2 upper_tile(int t, int nt, int step) {
+  int x = 0;
+  while (t >= nt - step * x) t -= nt - step * x++;
+  return int2{x, step * x + t};
+}
+
 // Work of one wave: the XCD-aware map from (block, wave).  The dispatcher
 // deals consecutive workgroups round-robin to the 8 XCDs, each with its own
 // L2.  Items (tile, K chunk) are numbered chunk-major and XCD x runs the
@@ -1964,7 +1985,7 @@ __device__ __forceinline__ void syrk_wave_body(const TIn *R, const uint32_t (&oa
 template <typename TIn>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SYWAVES))) void k_syrk_mfma(
     const TIn *__restrict__ R, int64_t ld, int64_t P, int64_t K, int64_t kchunk, int64_t n_items, int64_t per_xcd,
-    const int2 *__restrict__ tiles, int64_t T, const TIn *__restrict__ psi, int accum, double *__restrict__ part,
+    int nt, int64_t T, const TIn *__restrict__ psi, int accum, double *__restrict__ part,
     double2 *__restrict__ bpart) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, r16 = l & 15;
   const int64_t slot = int64_t(blockIdx.x >> 3) * 4 + w;
@@ -1972,7 +1993,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SYWAVES))) 
   const int64_t m = int64_t(blockIdx.x & 7) * per_xcd + slot;
   if (m >= n_items) return;
   const int64_t chunk = m / T;
-  const int2 tile = tiles[m - chunk * T];
+  const int2 tile = upper_tile(int(m - chunk * T), nt, 1);
   const int64_t i0 = int64_t(tile.x) * SYW, j0 = int64_t(tile.y) * SYW;
   const int64_t k0 = chunk * kchunk;
   if (k0 >= K) return;  // a narrower last column block has fewer chunks
@@ -1993,11 +2014,16 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SYWAVES))) 
   d4_t accb[4];
 #pragma unroll
   for (int a = 0; a < 4; ++a) accb[a] = d4_t{0.0, 0.0, 0.0, 0.0};
-  const bool diag = tile.x == tile.y;
-  if (diag)
-    syrk_wave_body<TIn, true>(R, oa, ob, psi, k0, k1, g, r16, acc, accb);
+  const bool diag = tile.x == tile.y, edge = j0 + SYW > P;  // i0 <= j0
+  const int na = P - i0 < SYW ? int(P - i0 + 15) >> 4 : 4, nb = P - j0 < SYW ? int(P - j0 + 15) >> 4 : 4;
+  if (diag && edge)
+    syrk_wave_body<TIn, true, true>(R, oa, ob, psi, k0, k1, g, r16, na, nb, acc, accb);
+  else if (diag)
+    syrk_wave_body<TIn, true, false>(R, oa, ob, psi, k0, k1, g, r16, na, nb, acc, accb);
+  else if (edge)
+    syrk_wave_body<TIn, false, true>(R, oa, ob, psi, k0, k1, g, r16, na, nb, acc, accb);
   else
-    syrk_wave_body<TIn, false>(R, oa, ob, psi, k0, k1, g, r16, acc, accb);
+    syrk_wave_body<TIn, false, false>(R, oa, ob, psi, k0, k1, g, r16, na, nb, acc, accb);
   double *out = part + chunk * P * P;
 #pragma unroll
   for (int a = 0; a < 4; ++a)
@@ -2037,7 +2063,7 @@ constexpr int CGM = 64, CGN = 32, CGK = 4;
 template <typename TIn>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SYWAVES))) void k_cgram_mfma(
     const TIn *__restrict__ A, int64_t lda, int64_t m, const TIn *__restrict__ B, int64_t ldb, int64_t nn, int64_t K,
-    int64_t kchunk, int64_t n_items, int64_t per_xcd, const int2 *__restrict__ tiles, int64_t T, int accum,
+    int64_t kchunk, int64_t n_items, int64_t per_xcd, int tn, int sym, int64_t T, int accum,
     double2 *__restrict__ part) {
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63, g = l >> 4, r16 = l & 15;
   const int64_t slot = int64_t(blockIdx.x >> 3) * 4 + w;
@@ -2045,7 +2071,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(SYWAVES))) 
   const int64_t mi = int64_t(blockIdx.x & 7) * per_xcd + slot;
   if (mi >= n_items) return;
   const int64_t chunk = mi / T;
-  const int2 tile = tiles[mi - chunk * T];
+  // A = B: only the tiles that meet the upper triangle (row x of them starts
+  // at column 2 x)
+  const int2 tile = upper_tile(int(mi - chunk * T), tn, sym ? CGM / CGN : 0);
   const int64_t i0 = int64_t(tile.x) * CGM, j0 = int64_t(tile.y) * CGN;
   const int64_t k0 = chunk * kchunk;
   if (k0 >= K) return;
@@ -2144,6 +2172,23 @@ __global__ void k_cgram_reduce(const double2 *__restrict__ part, int64_t m, int6
   out[e] = lower ? double2{a.x, -a.y} : sym && i == j ? double2{a.x, 0.0} : a;
 }
 
+// |G_ij|^2 for i < j in the order (0, 1), (0, 2), .., (1, 2), ..; G_ij the sum
+// over the split of part[z][i][j].
+__global__ __launch_bounds__(256) void k_pair_fidelities(const double2 *__restrict__ part, int64_t m, int64_t ks,
+                                                         double *__restrict__ out) {
+  const int64_t j = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  for (int64_t i = blockIdx.y; i < m; i += gridDim.y) {
+    if (j <= i || j >= m) continue;
+    double2 a{0, 0};
+    for (int64_t z = 0; z < ks; ++z) {
+      const double2 p = part[(z * m + i) * m + j];
+      a.x += p.x;
+      a.y += p.y;
+    }
+    out[i * m - i * (i + 1) / 2 + (j - i - 1)] = a.x * a.x + a.y * a.y;
+  }
+}
+
 // dst[r][0, w) = src[r][0, w) for P rows (16-byte units, row strides lds and
 // ldd): a column block of the Jacobian into a compact buffer.
 __global__ void k_copy_cols(const uint4 *__restrict__ src, int64_t lds, uint4 *__restrict__ dst, int64_t ldd,
@@ -2164,18 +2209,6 @@ __global__ void k_pad_cols(const T *__restrict__ src, int64_t lds, T *__restrict
   dst[u] = c < lds ? src[r * lds + c] : T(0);
 }
 
-// Column-major C[i + j P] = sum over the split of part[z][i][j], for the
-// upper triangle i <= j (every such entry lies in a computed block).
-__global__ void k_syrk_reduce(const double *__restrict__ part, int64_t P, int64_t ks, double *__restrict__ C) {
-  const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= P * P) return;
-  const int64_t i = e / P, j = e - i * P;
-  if (i > j) return;
-  double a = 0;
-  for (int64_t z = 0; z < ks; ++z) a += part[z * P * P + e];
-  C[i + j * P] = a;
-}
-
 __global__ void k_gram_reduce(const double2 *__restrict__ part, int64_t mn, int64_t ks, double2 *__restrict__ out) {
   const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (e >= mn) return;
@@ -2187,16 +2220,60 @@ __global__ void k_gram_reduce(const double2 *__restrict__ part, int64_t mn, int6
   out[e] = a;
 }
 
-// F from the upper triangle of the real Gram C = Re(J J^dag) (column-major,
-// C[p + q P] for p <= q) and b_p = <psi|J_p>.
-__global__ void k_qfim_combine_sym(const double *__restrict__ C, const double2 *__restrict__ bvec, int64_t P,
-                                   double *__restrict__ F) {
-  const int64_t e = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (e >= P * P) return;
-  const int64_t p = e / P, q = e - p * P;
-  const int64_t lo = p < q ? p : q, hi = p < q ? q : p;
-  const double2 bp = bvec[p], bq = bvec[q];
-  F[e] = 4 * (C[lo + hi * P] - (bp.x * bq.x + bp.y * bq.y));
+// F = 4 (Re(J J^dag) - Re(b b^dag)) from the split's partials (upper triangle)
+// and those of b_p = <psi|J_p>: a block sums one 16 x 16 tile with p <= q,
+// four threads per entry over the split, and the b of its rows and columns,
+// and writes the tile and its mirror image.
+constexpr int QF = 16, QFZ = 4;
+__global__ __launch_bounds__(QF *QF *QFZ) void k_qfim_finish(const double *__restrict__ part,
+                                                             const double2 *__restrict__ bpart, int64_t P, int64_t ks,
+                                                             int nt, double *__restrict__ F) {
+  __shared__ double g[QFZ][QF][QF + 1];
+  __shared__ double2 bs[QFZ * 8][2 * QF];
+  const int2 tile = upper_tile(int(blockIdx.x), nt, 1);
+  const int64_t p0 = int64_t(tile.x) * QF, q0 = int64_t(tile.y) * QF;
+  const int tid = threadIdx.x, zi = tid >> 8, pi = (tid >> 4) & 15, qi = tid & 15;
+  {  // 32 rows of b, 32 threads each over the split
+    const int r = tid & 31, z0 = tid >> 5;
+    const int64_t row = r < QF ? p0 + r : q0 + r - QF;
+    double2 x{0, 0};
+    if (row < P)
+#pragma unroll 8
+      for (int64_t z = z0; z < ks; z += 32) {
+        const double2 y = bpart[z * P + row];
+        x.x += y.x;
+        x.y += y.y;
+      }
+    bs[z0][r] = x;
+  }
+  const int64_t p = p0 + pi, q = q0 + qi;
+  double x = 0;
+  if (p < P && q < P && p <= q)
+#pragma unroll 8
+    for (int64_t z = zi; z < ks; z += QFZ) x += part[(z * P + p) * P + q];
+  g[zi][pi][qi] = x;
+  __syncthreads();
+  if (tid < 2 * QF) {
+    double2 y = bs[0][tid];
+    for (int z = 1; z < 32; ++z) {
+      y.x += bs[z][tid].x;
+      y.y += bs[z][tid].y;
+    }
+    bs[0][tid] = y;
+  }
+  __syncthreads();
+  if (zi == 0 && p < P && q < P && p <= q) {
+    const double c = ((g[0][pi][qi] + g[1][pi][qi]) + g[2][pi][qi]) + g[3][pi][qi];
+    const double2 bp = bs[0][pi], bq = bs[0][QF + qi];
+    const double f = 4 * (c - (bp.x * bq.x + bp.y * bq.y));
+    F[p * P + q] = f;
+    g[0][pi][qi] = f;
+  }
+  __syncthreads();
+  if (zi == 0) {  // the mirror image, its rows along the lanes
+    const int64_t pm = p0 + qi, qm = q0 + pi;
+    if (pm < P && qm < P && pm < qm) F[qm * P + pm] = g[0][qi][pi];
+  }
 }
 
 struct PauliTerm {
@@ -3655,8 +3732,9 @@ int gram_impl(pqs_ctx *ctx, int32_t dtype, const void *a, int64_t lda, int64_t m
 // without touching the stream, for shapes it does not take: a K that is not
 // a whole number of load-ring steps (fewer than 8 amplitudes) or operands
 // whose rows cannot be addressed in 32 bits nor copied in 16-byte units.
+// With `fid` (A = B) it writes the pair fidelities there instead of G.
 int cgram_mfma(pqs_ctx *ctx, int32_t dtype, const void *a, int64_t lda, int64_t m, const void *b, int64_t ldb,
-               int64_t nn, int64_t dim, double2 *out, hipStream_t st) {
+               int64_t nn, int64_t dim, double2 *out, hipStream_t st, double *fid = nullptr) {
   const int64_t cb = dtype == PQS_C128 ? 16 : 8;  // bytes per amplitude
   const int64_t ring = SYRING * CGK;
   if (dim % ring != 0) return PQS_ERR_UNSUPPORTED;
@@ -3676,23 +3754,24 @@ int cgram_mfma(pqs_ctx *ctx, int32_t dtype, const void *a, int64_t lda, int64_t 
   if (size_t(m) * size_t(la) * size_t(cb) >= (size_t(1) << 32) || size_t(nn) * size_t(lb) * size_t(cb) >= (size_t(1) << 32))
     return PQS_ERR_UNSUPPORTED;
   const int64_t tm = (m + CGM - 1) / CGM, tn = (nn + CGN - 1) / CGN;
-  std::vector<int2> tl;
-  for (int64_t x = 0; x < tm; ++x)
-    for (int64_t y = 0; y < tn; ++y)
-      if (!sym || CGM * x <= CGN * y + CGN - 1) tl.push_back(int2{int(x), int(y)});
-  const int64_t T = int64_t(tl.size());
-  // the K split that leaves the fewest wave slots idle over whole rounds
-  // (chunks of at least 256 amplitudes, partials within 2 GiB)
+  const int64_t T = sym ? tm * tn - tm * (tm - 1) : tm * tn;
+  // The split over K: a 4-wide step of 8 blocks takes one wave about 1 us, and
+  // every chunk's partials are written and read once (half of them for A =
+  // B).  The split with the least sum of the two (chunks of at least two ring
+  // turns, partials within 2 GiB); the first of them at a tie.  Measured, 1000
+  // states of 12 qubits: 320 us for the product in 15 chunks and 95 us for
+  // their sum, 330 and 12 us in 7.
   const int64_t slots = 4 * SYWAVES * int64_t(ctx->n_cu);
   const int64_t ks_max = std::max<int64_t>(
-      1, std::min<int64_t>({Kc / 256, int64_t(64), int64_t((size_t(2) << 30) / (size_t(m) * size_t(nn) * 16))}));
+      1, std::min<int64_t>({Kc / (2 * ring), int64_t(64), int64_t((size_t(2) << 30) / (size_t(m) * size_t(nn) * 16))}));
   int64_t ks = 1;
-  double best = -1;
+  double best = 1e300;
   for (int64_t k = 1; k <= ks_max; ++k) {
-    const int64_t items = T * k, rounds = (items + slots - 1) / slots;
-    const double fill = double(items) / double(rounds * slots);
-    if (fill > best + 0.01) {
-      best = fill;
+    const int64_t per_simd = (T * k + slots / 2 - 1) / (slots / 2);
+    const int64_t chunk = ((Kc + k - 1) / k + ring - 1) / ring * ring;
+    const double us = double(chunk / CGK * per_simd) + double(k) * double(m) * double(nn) * (sym ? 16 : 32) / 4e6;
+    if (us < best) {
+      best = us;
       ks = k;
     }
   }
@@ -3703,17 +3782,13 @@ int cgram_mfma(pqs_ctx *ctx, int32_t dtype, const void *a, int64_t lda, int64_t 
   const int64_t grid = 8 * ((per_xcd + 3) / 4);
   if (grid > 0x7fffffff) return PQS_ERR_UNSUPPORTED;
   const size_t al = 255;
-  const size_t off_t = (size_t(ks) * size_t(m) * size_t(nn) * sizeof(double2) + al) & ~al;
-  const size_t off_a = (off_t + tl.size() * sizeof(int2) + al) & ~al;
+  const size_t off_a = (size_t(ks) * size_t(m) * size_t(nn) * sizeof(double2) + al) & ~al;
   const size_t off_b = (off_a + (staged ? size_t(m) * size_t(Ks) * size_t(cb) : 0) + al) & ~al;
   const size_t end = off_b + (staged && !sym ? size_t(nn) * size_t(Ks) * size_t(cb) : 0);
   int rc = ws_reserve(ctx, end, st);
   if (rc) return rc;
   char *ws = (char *)ctx->ws;
   double2 *part = (double2 *)ws;
-  int2 *d_tiles = (int2 *)(ws + off_t);
-  rc = upload(ctx, d_tiles, tl.data(), tl.size() * sizeof(int2), st);
-  if (rc) return rc;
   for (int64_t c0 = 0; c0 < dim; c0 += Kc) {
     const int64_t w = std::min(Kc, dim - c0);
     const void *pa = (const char *)a + size_t(c0) * size_t(cb), *pb = (const char *)b + size_t(c0) * size_t(cb);
@@ -3735,14 +3810,19 @@ int cgram_mfma(pqs_ctx *ctx, int32_t dtype, const void *a, int64_t lda, int64_t 
     const int accum = c0 > 0;
     if (dtype == PQS_C128)
       hipLaunchKernelGGL(k_cgram_mfma<double>, dim3(unsigned(grid)), dim3(256), 0, st, (const double *)pa, la, m,
-                         (const double *)pb, lb, nn, w, kchunk, n_items, per_xcd, d_tiles, T, accum, part);
+                         (const double *)pb, lb, nn, w, kchunk, n_items, per_xcd, int(tn), int(sym), T, accum, part);
     else
       hipLaunchKernelGGL(k_cgram_mfma<float>, dim3(unsigned(grid)), dim3(256), 0, st, (const float *)pa, la, m,
-                         (const float *)pb, lb, nn, w, kchunk, n_items, per_xcd, d_tiles, T, accum, part);
+                         (const float *)pb, lb, nn, w, kchunk, n_items, per_xcd, int(tn), int(sym), T, accum, part);
     HIPCHECK(hipGetLastError());
   }
-  hipLaunchKernelGGL(k_cgram_reduce, dim3(grid_for(m * nn, 256)), dim3(256), 0, st, (const double2 *)part, m, nn, ks,
-                     int(sym), out);
+  if (fid) {
+    hipLaunchKernelGGL(k_pair_fidelities, dim3(grid_for(nn, 256), unsigned(std::min<int64_t>(m, 65535))), dim3(256), 0,
+                       st, (const double2 *)part, m, ks, fid);
+  } else {
+    hipLaunchKernelGGL(k_cgram_reduce, dim3(grid_for(m * nn, 256)), dim3(256), 0, st, (const double2 *)part, m, nn, ks,
+                       int(sym), out);
+  }
   HIPCHECK(hipGetLastError());
   return PQS_OK;
 }
@@ -3767,6 +3847,28 @@ int pqs_gram(pqs_ctx *ctx, int32_t dtype, const void *a, int64_t lda, int64_t m,
   return gram_impl(ctx, dtype, a, lda, m, b, ldb, nn, dim, (double2 *)out, (double2 *)ctx->ws, st);
 }
 
+int pqs_pair_fidelities(pqs_ctx *ctx, int32_t dtype, const void *states, int64_t ld, int64_t m, int64_t dim,
+                        double *out, void *stream) {
+  Range rg_("pqs_pair_fidelities");
+  if (!ctx || !states || !out) return fail(PQS_ERR_ARG, "NULL argument");
+  if (m < 2 || dim <= 0 || ld < dim) return fail(PQS_ERR_ARG, "bad sizes");
+  DeviceGuard g(ctx->device);
+  hipStream_t st = (hipStream_t)stream;
+  int rc = cgram_mfma(ctx, dtype, states, ld, m, states, ld, m, dim, nullptr, st, out);
+  if (rc != PQS_ERR_UNSUPPORTED) return rc;  // else: shapes the matrix-core path does not take
+  // G, then its partials
+  const size_t g_b = (size_t(m) * size_t(m) * sizeof(double2) + 255) & ~size_t(255);
+  rc = ws_reserve(ctx, g_b + gram_part_bytes(ctx, m, m, dim), st);
+  if (rc) return rc;
+  char *ws = (char *)ctx->ws;
+  rc = gram_impl(ctx, dtype, states, ld, m, states, ld, m, dim, (double2 *)ws, (double2 *)(ws + g_b), st);
+  if (rc) return rc;
+  hipLaunchKernelGGL(k_pair_fidelities, dim3(grid_for(m, 256), unsigned(std::min<int64_t>(m, 65535))), dim3(256), 0, st,
+                     (const double2 *)ws, m, int64_t(1), out);
+  HIPCHECK(hipGetLastError());
+  return PQS_OK;
+}
+
 int pqs_qfim(pqs_ctx *ctx, int32_t dtype, const void *jac, int64_t P, const void *psi, int64_t dim, double *F,
              void *stream) {
   Range rg_("pqs_qfim");
@@ -3782,11 +3884,7 @@ int pqs_qfim(pqs_ctx *ctx, int32_t dtype, const void *jac, int64_t P, const void
     // to double in registers: the same products and sums.
     const int64_t K = 2 * dim;
     const size_t esz = dtype == PQS_C128 ? sizeof(double) : sizeof(float);
-    const int64_t nt = (P + SYW - 1) / SYW;
-    std::vector<int2> tl;
-    for (int64_t a = 0; a < nt; ++a)
-      for (int64_t b = a; b < nt; ++b) tl.push_back(int2{int(a), int(b)});
-    const int64_t T = int64_t(tl.size());
+    const int64_t nt = (P + SYW - 1) / SYW, T = nt * (nt + 1) / 2;
     // A Jacobian above 1 GiB is taken in column blocks of at most 512 MiB,
     // each copied to a compact P x Kc buffer first: rows of 2^20 amplitudes
     // and more lie 16 MiB apart, and every load of the product kernel
@@ -3803,24 +3901,40 @@ int pqs_qfim(pqs_ctx *ctx, int32_t dtype, const void *jac, int64_t P, const void
       Kc = int64_t(kQfimBlockBytes / (size_t(P) * esz)) / ring * ring;
       Kc = std::max<int64_t>(ring, std::min<int64_t>(Kc, K));
     }
-    // one item per wave slot (a single round), chunks of at least 1024 k, a
-    // multiple of the load ring
+    // The split over K.  With at least 1024 k per chunk in every wave slot:
+    // one round of all slots.  Shorter products are bound by the length of a
+    // chunk (an 8-wide step of 16 blocks takes one wave about 1 us) until the
+    // partials' traffic and their sum (30 ns a chunk) outweigh it: the split
+    // with the least total, chunks of at least two ring turns.  Measured, P =
+    // 160, K = 512 (8 qubits): product and sums 87 us unsplit, 15 us in 16
+    // chunks; P = 20, K = 8192: 147 us in 8
+    // chunks, 20 us in 128.
     const int64_t slots = 4 * SYWAVES * int64_t(ctx->n_cu);
-    int64_t ks = std::max<int64_t>(1, std::min<int64_t>(slots / T, Kc / 1024));
-    int64_t kchunk = (Kc + ks - 1) / ks;
-    kchunk = (kchunk + ring - 1) / ring * ring;
+    int64_t ks = std::max<int64_t>(1, slots / T), kchunk = 0;
+    auto chunk_of = [&](int64_t k) { return ((Kc + k - 1) / k + ring - 1) / ring * ring; };
+    if (Kc / 1024 < ks) {
+      const int64_t most = std::max<int64_t>(1, std::min<int64_t>(ks, Kc / (2 * ring)));
+      double best = 1e300;
+      for (int64_t k = 1; k <= most; ++k) {
+        const int64_t waves = T * k, per_simd = (waves + slots / 2 - 1) / (slots / 2);
+        const double us = double(chunk_of(k) / SYK * per_simd) +
+                          double(k) * (0.03 + double(P) * double(P) * 16 / 4e6);
+        if (us < best) {
+          best = us;
+          ks = k;
+        }
+      }
+    }
+    kchunk = chunk_of(ks);
     ks = (Kc + kchunk - 1) / kchunk;
     const int64_t n_items = T * ks, per_xcd = (n_items + 7) / 8;
     const int64_t grid = 8 * ((per_xcd + 3) / 4);
     if (grid > 0x7fffffff) return fail(PQS_ERR_UNSUPPORTED, "QFIM too large");
-    // workspace: [partials ks P^2 | C P^2 | b P | b partials ks P | tiles |
-    // staged block (P Kc) | padded psi (Kc, short Jacobians only)]
+    // workspace: [partials ks P^2 | b partials ks P | staged block (P Kc) |
+    // padded psi (Kc, short Jacobians only)]
     const size_t al = 255;
-    const size_t off_c = (size_t(ks * P * P) * sizeof(double) + al) & ~al;
-    const size_t off_b = (off_c + size_t(P * P) * sizeof(double) + al) & ~al;
-    const size_t off_bp = (off_b + size_t(P) * sizeof(double2) + al) & ~al;
-    const size_t off_t = (off_bp + size_t(ks * P) * sizeof(double2) + al) & ~al;
-    const size_t off_s = (off_t + tl.size() * sizeof(int2) + al) & ~al;
+    const size_t off_bp = (size_t(ks * P * P) * sizeof(double) + al) & ~al;
+    const size_t off_s = (off_bp + size_t(ks * P) * sizeof(double2) + al) & ~al;
     // staged rows are Kc + 32 elements apart: a power-of-two row stride
     // would put the 16 rows of every load on one L2 channel
     const int64_t Ks = Kc + 32;
@@ -3830,13 +3944,8 @@ int pqs_qfim(pqs_ctx *ctx, int32_t dtype, const void *jac, int64_t P, const void
     int rc = ws_reserve(ctx, off_ps + (pad ? size_t(Kc) * esz : 0), st);
     if (rc) return rc;
     char *ws = (char *)ctx->ws;
-    double *C = (double *)(ws + off_c);
-    double2 *bv = (double2 *)(ws + off_b);
     double2 *bpart = (double2 *)(ws + off_bp);
-    int2 *d_tiles = (int2 *)(ws + off_t);
     void *stage = ws + off_s;
-    rc = upload(ctx, d_tiles, tl.data(), tl.size() * sizeof(int2), st);
-    if (rc) return rc;
     // column blocks after the first add to the partials (same stream, in
     // order); the diagonal tiles' waves also form b = <J_p|psi>
     for (int64_t c0 = 0; c0 < K; c0 += Kc) {
@@ -3872,17 +3981,16 @@ int pqs_qfim(pqs_ctx *ctx, int32_t dtype, const void *jac, int64_t P, const void
       const int accum = c0 > 0;
       if (dtype == PQS_C128)
         hipLaunchKernelGGL(k_syrk_mfma<double>, dim3(unsigned(grid)), dim3(256), 0, st, (const double *)src, ld, P, w,
-                           kchunk, n_items, per_xcd, d_tiles, T, (const double *)ps, accum, (double *)ws, bpart);
+                           kchunk, n_items, per_xcd, int(nt), T, (const double *)ps, accum, (double *)ws, bpart);
       else
         hipLaunchKernelGGL(k_syrk_mfma<float>, dim3(unsigned(grid)), dim3(256), 0, st, (const float *)src, ld, P, w,
-                           kchunk, n_items, per_xcd, d_tiles, T, (const float *)ps, accum, (double *)ws, bpart);
+                           kchunk, n_items, per_xcd, int(nt), T, (const float *)ps, accum, (double *)ws, bpart);
       HIPCHECK(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_syrk_reduce, dim3(grid_for(P * P, 256)), dim3(256), 0, st, (const double *)ws, P, ks, C);
-    HIPCHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_gram_reduce, dim3(grid_for(P, 256)), dim3(256), 0, st, bpart, P, ks, bv);
-    HIPCHECK(hipGetLastError());
-    hipLaunchKernelGGL(k_qfim_combine_sym, dim3(grid_for(P * P, 256)), dim3(256), 0, st, C, bv, P, F);
+    const int64_t nf = (P + QF - 1) / QF, tf = nf * (nf + 1) / 2;
+    if (tf > 0x7fffffff) return fail(PQS_ERR_UNSUPPORTED, "QFIM too large");
+    hipLaunchKernelGGL(k_qfim_finish, dim3(unsigned(tf)), dim3(QF * QF * QFZ), 0, st, (const double *)ws,
+                       (const double2 *)bpart, P, ks, int(nf), F);
     HIPCHECK(hipGetLastError());
     return PQS_OK;
   }

@@ -139,6 +139,24 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
     p.dev_wave[size_t(refill_at)].x = uint32_t(n_ang - refill_first);
     return uint16_t(n_ang - 1 - refill_first);
   };
+  // a generator's record; a run of them is headed by a record that skips them
+  // all where the wave holds no tangent of theirs
+  int skip_at = -1;
+  auto generator = [&](int code, int tangent) -> WaveOp & {
+    if (skip_at < 0 || skip_at + int(p.dev_wave[size_t(skip_at)].x) + 1 != int(p.dev_wave.size())) {
+      skip_at = int(p.dev_wave.size());
+      WaveOp &h = emit(kWSkip);
+      h.z = uint32_t(tangent);
+      h.c = tangent;
+    }
+    WaveOp &h = p.dev_wave[size_t(skip_at)];
+    ++h.x;
+    h.z = std::min(h.z, uint32_t(tangent));
+    h.c = std::max(h.c, tangent);
+    WaveOp &w = emit(code);
+    w.tangent = tangent;
+    return w;
+  };
   auto rotations = [&](int count) {  // at most 10 between two checks
     if (rot + count > 10) {
       emit(kWCheck);
@@ -192,24 +210,18 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
         w.c = o;
         break;
       }
-      case kPauliSum: {
-        WaveOp &w = emit(kWSum);
-        w.c = o;
-        w.tangent = d.tangent;
-        break;
-      }
+      case kPauliSum: generator(kWSum, d.tangent).c = o; break;
       case PQS_OP_FSIM:
       case PQS_OP_GEN_FSIM: {
         reserve(2);
         // doubled: the table holds (tan, cos) of half of each angle
         const uint16_t a = angle(2 * d.scale, 2 * d.offset, d.slot);
         const uint32_t f = d.slot2 >= 0 ? angle(2.0, 0.0, d.slot2) : 0xffffffffu;
-        WaveOp &w = emit(d.kind == PQS_OP_FSIM ? kWFsim : kWGenFsim);
+        WaveOp &w = d.kind == PQS_OP_FSIM ? emit(kWFsim) : generator(kWGenFsim, d.tangent);
         w.ang = a;
         w.x = b0 | b1;
         w.z = f;
         w.c = o;
-        w.tangent = d.tangent;
         break;
       }
       default: {  // PQS_OP_MAT2
@@ -221,6 +233,9 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
       }
     }
   };
+  uint64_t tpos[kMaxTileBits];  // position bit of every tile bit
+  for (int r = 0; r < ds.nruns; ++r)
+    for (int b = 0; b < ds.run_len[r]; ++b) tpos[ds.run_shift[r] + b] = uint64_t(1) << (ds.run_pos[r] + b);
   // qubits an op acts on, as positions: non-diagonally and at all
   auto masks = [&](int o, uint64_t &act, uint64_t &all) {
     const DevOp &d = p.dev_ops[size_t(o)];
@@ -230,7 +245,19 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
     switch (d.kind) {
       case PQS_OP_RZ: case PQS_OP_RZZ: case PQS_OP_CZ: break;
       case PQS_OP_CX: act = b1; break;
-      case kPauliSum: act = all = ~uint64_t(0); break;  // a point that nothing passes
+      case kPauliSum: {
+        all = 0;
+        for (int t = d.term0; t < d.term0 + d.nterms; ++t) {
+          const DevTerm &m = p.dev_terms[size_t(t)];
+          for (int b = 0; b < k; ++b) {
+            if ((m.xm >> b) & 1) act |= tpos[b];
+            if ((m.zm_tile >> b) & 1) all |= tpos[b];
+          }
+          all |= m.zm_glob;
+        }
+        all |= act;
+        break;
+      }
       default: act = all; break;
     }
   };

@@ -118,6 +118,7 @@ enum WaveCode : int32_t {
   kWEnd = 0,
   kWRefill,   // c: first angle, x: count
   kWCheck,    // growth check of the scaled rotations
+  kWSkip,     // the next x records are generators of tangents z .. c
   kWLayerRx,  // R_x on every bit, angles ang .. ang + k - 1 (identity: angle 0)
   kWLayerRy,
   kWLayerRz,

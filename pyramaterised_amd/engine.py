@@ -734,6 +734,18 @@ def gram(a, b):
     return out
 
 
+def pair_fidelities(states):
+    """|<s_a|s_b>|^2 over combinations(range(S), 2) of the rows of an (S, dim)
+    tensor (S >= 2) -> float64 (S (S - 1) / 2,)."""
+    ctx = context()
+    states = states.contiguous()
+    S, dim = states.shape
+    out = torch.empty(S * (S - 1) // 2, dtype=torch.float64, device=states.device)
+    check(L.lib().pqs_pair_fidelities(ctx.handle, dtype_code(states.dtype), ptr(states), dim, S, dim, ptr(out),
+                                      stream_ptr()))
+    return out
+
+
 def qfim(J, psi):
     """F = 4 Re(J J^dag - (J psi^*)(psi J^dag)) -> float64 (P, P)."""
     ctx = context()

@@ -112,10 +112,7 @@ class Measurements:
         S = states.shape[0]
         if S < 2:
             return torch.empty(0, dtype=torch.float64, device=states.device)
-        G = E.gram(states, states)
-        a, b = pair_indices(S)
-        idx = torch.as_tensor(a * S + b, device=states.device)
-        return E.abs2(G.reshape(-1)[idx])
+        return E.pair_fidelities(states)
 
     def fidelities_pairs(self, states_a, states_b):
         """|<a_i|b_i>|^2 for paired rows."""

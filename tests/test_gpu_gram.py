@@ -86,3 +86,37 @@ def test_all_pairs_fidelities_vs_oracle(pyqc_mod):
 def pyqc_mod():
     import pyramaterised_amd
     return pyramaterised_amd
+
+
+@pytest.mark.parametrize("S,dim,dtype", [(2, 2, "complex128"), (3, 4, "complex64"), (2, 16, "complex128"),
+                                         (65, 32, "complex128"), (257, 1024, "complex64"), (300, 4096, "complex128")])
+def test_pair_fidelities_order_and_shapes(S, dim, dtype):
+    """Every pair in combinations order, with and without the matrix cores
+    (below 8 amplitudes), one and several K chunks; states of norm 1, so
+    double sums of dim products are within 1e-13."""
+    from pyramaterised_amd import engine as E
+    g = torch.Generator(device="cuda").manual_seed(S + dim)
+    s = _rand(g, S, dim, torch.complex128)
+    s = (s / torch.linalg.norm(s, dim=1, keepdim=True)).to(getattr(torch, dtype))
+    G = _ref(s, s).cpu().numpy()
+    a, b = np.triu_indices(S, k=1)
+    assert np.max(np.abs(E.pair_fidelities(s).cpu().numpy() - np.abs(G[a, b]) ** 2)) < 1e-13
+
+
+@pytest.mark.parametrize("P,dim,dtype", [(1, 2, "complex128"), (15, 8, "complex128"), (17, 256, "complex64"),
+                                         (20, 4096, "complex128"), (64, 64, "complex128"), (65, 1024, "complex128"),
+                                         (160, 256, "complex128"), (200, 2048, "complex64")])
+def test_qfim_shapes(P, dim, dtype):
+    """QFIM product at the edges of its 64-row tiles and 16-row blocks, for
+    one and many K chunks, against the formula in complex128 (rel-Frobenius
+    1e-12; rows of norm 1, so no cancellation beyond F's own size)."""
+    from pyramaterised_amd import engine as E
+    g = torch.Generator(device="cuda").manual_seed(P * 3 + dim)
+    J = _rand(g, P, dim, getattr(torch, dtype))
+    psi = _rand(g, 1, dim, getattr(torch, dtype))[0]
+    F = E.qfim(J, psi)
+    j, p = J.to(torch.complex128), psi.to(torch.complex128)
+    b = j.conj() @ p
+    ref = 4 * ((j.conj() @ j.T) - b[:, None] * b.conj()[None, :]).real
+    assert (torch.linalg.norm(F - ref) / torch.linalg.norm(ref)).item() < 1e-12
+    assert torch.equal(F, F.T)
