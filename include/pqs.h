@@ -71,7 +71,12 @@ enum pqs_op_kind {
   /* fSim-family derivative matrices as the reference writes them
    * (gates.py:609-648, 719-737): pauli selects 1 = d_theta, 2 = d_phi,
    * 3 = fixed_fSim d_theta; angles from slot / slot2 as for PQS_OP_FSIM. */
-  PQS_OP_GEN_FSIM = 12
+  PQS_OP_GEN_FSIM = 12,
+  /* Measurement of a pair of states: the plan's state is [a; b], qubit 0
+   * selecting the half, and no other op touches qubit 0.  At this point of the
+   * circuit Re(coef <a|P|b>), P and coef as for PQS_OP_GEN on qubits >= 1, goes
+   * to output i (the i-th such op of the list).  pqs_adjoint runs such plans. */
+  PQS_OP_MEAS = 13
 };
 
 typedef struct pqs_op {
@@ -391,6 +396,18 @@ int pqs_apply_pauli(pqs_ctx *ctx, int32_t dtype, const void *x_dev, int32_t n_qu
 int pqs_pauli_transition(pqs_ctx *ctx, int32_t dtype, const void *bra_dev, const void *ket_dev, int32_t n_qubits,
                          const uint64_t *xmask_host, const uint64_t *zmask_host, const double *coef_host,
                          int32_t n_terms, double *out_dev, void *stream);
+
+/* Evolve the pair [a; b] at pair_dev (left unchanged; 2^N amplitudes, qubit 0
+ * the half) through a plan with PQS_OP_MEAS ops and write every measurement
+ * to out_dev (one double each, in op order).  With a = H^dag psi, b = psi and
+ * the inverse gates of a circuit this is its whole adjoint backward pass:
+ * each sweep carries both states once and measures its parameters in
+ * registers (reference Measurements.get_gradient_vector, measure.py:461-471,
+ * and pqs_pauli_transition's passes per point).  complex128; tiles of 10
+ * qubits and more need specialised sweeps (pqs_plan_jit, else
+ * PQS_ERR_UNSUPPORTED). */
+int pqs_adjoint(pqs_ctx *ctx, pqs_plan *plan, const double *params_dev, const void *pair_dev, double *out_dev,
+                void *stream);
 
 /* Histogram of values into n_bins int64 counts over the n_bins + 1 ascending
  * edges (device array, e.g. numpy.linspace(0, 1, n_bins + 1)) with

@@ -22,7 +22,7 @@ PQS_PLAN_GREEDY_PHASES = 128
 PQS_PLAN_NO_EXCHANGE = 256
 
 (OP_MAT1, OP_RX, OP_RY, OP_RZ, OP_MAT2, OP_CX, OP_CZ, OP_RXX, OP_RYY, OP_RZZ,
- OP_FSIM, OP_GEN, OP_GEN_FSIM) = range(13)
+ OP_FSIM, OP_GEN, OP_GEN_FSIM, OP_MEAS) = range(14)
 
 
 class Op(C.Structure):
@@ -73,6 +73,7 @@ SIGNATURES = {
     "pqs_run_multi": (C.c_int, [vp, vp, i32, vp, vp, vp, i64, vp]),
     "pqs_run_batch_noalloc": (C.c_int, [vp, vp, vp, i64, i64, vp, i64, i32, vp, vp, vp, vp]),
     "pqs_jacobian": (C.c_int, [vp, vp, vp, i32, vp, vp, vp, vp, vp]),
+    "pqs_adjoint": (C.c_int, [vp, vp, vp, vp, vp, vp]),
     "pqs_inner": (C.c_int, [vp, i32, vp, i64, vp, vp, i64, vp, vp]),
     "pqs_mw": (C.c_int, [vp, i32, vp, i32, i64, vp, vp, vp]),
     "pqs_gram": (C.c_int, [vp, i32, vp, i64, i64, vp, i64, i64, i64, vp, vp]),

@@ -10,14 +10,18 @@ circuit.py:149-192).  Here, with psi = U_G..U_1 psi0 and lambda = H^dag psi,
 
 where g is the gate of parameter p, D_p its generator (d U_g = D_p U_g) and
 lambda_g, psi_g are lambda and psi carried back to the point right after
-gate g (U_{g+1}^dag .. U_G^dag applied to both).  The backward pass walks
-the gates in reverse: parameters whose generators commute with every gate
+gate g (U_{g+1}^dag .. U_G^dag applied to both).  [lambda; psi] is one state of
+n + 1 qubits whose first qubit no gate touches, so the whole backward pass is
+one plan of the inverse gates with a measurement op per generator term
+(``pqs_adjoint``): every sweep carries the pair once and measures in
+registers.  Memory: the pair, its evolved copy and that copy's second buffer.
+
+Without that plan (complex64, or specialised kernels not wanted yet) the pass
+goes point by point: parameters whose generators commute with every gate
 between them are measured at one point (a whole rotation layer of a
-hardware-efficient ansatz at once), and between measurement points the pair
-(lambda, psi) is evolved by a small plan of inverse ops (one batched run of
-two instances).  Each measurement is one ``pqs_pauli_transition`` launch
-over the group's Pauli terms.  Memory: the two states plus the workspace of
-one small plan, against P states for the Jacobian route.
+hardware-efficient ansatz at once) by one ``pqs_pauli_transition`` launch,
+and between points the pair is evolved by a small plan of inverse ops (one
+batched run of two instances).
 """
 import ctypes as C
 
@@ -138,9 +142,28 @@ class AdjointProgram:
         self.dtype = dt
         self.P = qc.n_true_params
         self.step_ops = steps  # (inverse ops, group) per step, before planning
-        self.steps = []
-        for ops, grp in steps:
-            plan = E.Plan(self.n, ops, dtype=dt, tile_bits=min(12, self.n), low_bits=3) if ops else None
+        self.owner = np.array([slot for _, grp in steps for slot, terms in grp for _ in terms], dtype=np.int64)
+        self.n_terms = len(self.owner)
+        self._steps = None
+        self._fused = None
+        self._uses = 0
+        # as for the circuit's own plans: specialised kernels at once for
+        # large states, else from the third pass on
+        self._want_jit = qc._want_jit(1)
+        self._may_jit = qc.jit == "auto" and qc._jit_env() is None
+
+    @property
+    def steps(self):
+        """[(plan or None, n_terms, xmasks, zmasks, coefs, owner slots)]: the
+        point-by-point form."""
+        if self._steps is None:
+            self._steps = self._plan_steps()
+        return self._steps
+
+    def _plan_steps(self):
+        out = []
+        for ops, grp in self.step_ops:
+            plan = E.Plan(self.n, ops, dtype=self.dtype, tile_bits=min(12, self.n), low_bits=3) if ops else None
             xs, zs, cs, owner = [], [], [], []
             for slot, terms in grp:
                 for c, x, z in terms:
@@ -149,33 +172,93 @@ class AdjointProgram:
                     cs += [c.real, c.imag]
                     owner.append(slot)
             nt = len(xs)
-            self.steps.append((plan, nt, (C.c_uint64 * max(1, nt))(*xs), (C.c_uint64 * max(1, nt))(*zs),
-                               (C.c_double * max(2, 2 * nt))(*cs), np.array(owner, dtype=np.int64)))
-        self.n_terms = sum(s[1] for s in self.steps)
+            out.append((plan, nt, (C.c_uint64 * max(1, nt))(*xs), (C.c_uint64 * max(1, nt))(*zs),
+                        (C.c_double * max(2, 2 * nt))(*cs), np.array(owner, dtype=np.int64)))
+        return out
+
+    # partials of the measurements (one per tile and term) above this many
+    # bytes: the point-by-point form
+    FUSED_PARTIAL_BYTES = 4 << 30
+
+    def fused_ops(self):
+        """The backward pass as one op list on n + 1 qubits (qubit 0: lambda
+        or psi): the inverse gates, and a measurement op per generator term,
+        in the order of ``owner``."""
+        out = []
+
+        def shifted(o):
+            c = L.Op.from_buffer_copy(o)
+            c.q0 = o.q0 + 1
+            c.q1 = o.q1 + 1 if o.q1 >= 0 else o.q1
+            return c
+
+        for ops, grp in self.step_ops:
+            out += [shifted(o) for o in ops]
+            for _, terms in grp:
+                for c, x, z in terms:
+                    qs = [q for q in range(self.n) if ((x | z) >> q) & 1]
+                    m = L.Op(kind=L.OP_MEAS, q0=qs[0] + 1 if qs else 1, q1=qs[1] + 1 if len(qs) > 1 else -1,
+                             slot=-1, slot2=-1, tangent=-1, pauli=(1 if x and not z else 2 if x else 3) if qs else 0)
+                    m.m[0], m.m[1] = c.real, c.imag
+                    out.append(m)
+        return out
+
+    def fused_plan(self):
+        """The plan of ``fused_ops`` if this pass runs fused, else None.
+        12-bit tiles (11 qubits and the pair's), 20 qubits, 40 layers: 19
+        sweeps in 1.08 ms; 11-bit 1.22 ms, 13-bit 1.87, 10-bit 1.35.  At 13-16
+        qubits 11-bit tiles are 6% faster."""
+        if self._fused is None and self.dtype == L.PQS_C128 and self.n_terms:
+            k = min(12, self.n + 1)
+            self._uses += 1
+            if k >= 10 and not (self._want_jit or (self._may_jit and self._uses >= PASSES_BEFORE_JIT)):
+                return None
+            if k >= 4 and (k < 10 or (8 * self.n_terms << (self.n + 1 - k)) <= self.FUSED_PARTIAL_BYTES):
+                self._fused = E.Plan(self.n + 1, self.fused_ops(), dtype=self.dtype, tile_bits=k, low_bits=min(3, k),
+                                     flags=L.PQS_PLAN_ROLLING)
+                if k >= 10:
+                    self._fused.jit()
+            else:
+                self._fused = False
+        return self._fused or None
 
     def gradient(self, psi, lam, params):
         """Energy gradient 2 Re <psi|H|d_p psi> from psi = U psi0 and lambda =
         H^dag psi (both (2^N,) tensors, left unchanged).  Returns a float64
         numpy array of P values."""
+        return self.gradient_of_pair(torch.stack([lam.reshape(-1), psi.reshape(-1)]).contiguous(), params)
+
+    def gradient_of_pair(self, pair, params):
+        """``gradient`` for [lambda; psi] as one contiguous (2, 2^N) tensor,
+        which this may overwrite."""
         ctx = E.context()
-        pair = torch.stack([lam.reshape(-1), psi.reshape(-1)]).contiguous()
-        out = torch.empty((max(1, self.n_terms), 2), dtype=torch.float64, device=pair.device)
         th = E._params_tensor(params, pair.device)
-        off = 0
-        for plan, nt, xs, zs, cs, _ in self.steps:
-            if plan is not None:
-                E.run_rows(plan, th, pair)
-            E.check(L.lib().pqs_pauli_transition(ctx.handle, self.dtype, E.ptr(pair[0]), E.ptr(pair[1]), self.n,
-                                                 xs, zs, cs, nt, E.ptr(out[off:off + nt]), E.stream_ptr()))
-            off += nt
-        vals = out[:off].cpu().numpy()
+        plan = self.fused_plan()
+        if plan is not None:
+            vals = torch.empty(self.n_terms, dtype=torch.float64, device=pair.device)
+            E.check(L.lib().pqs_adjoint(ctx.handle, plan.handle, E.ptr(th), E.ptr(pair), E.ptr(vals), E.stream_ptr()))
+            E._keepalive(th, pair)
+            real = vals.cpu().numpy()
+        else:
+            out = torch.empty((max(1, self.n_terms), 2), dtype=torch.float64, device=pair.device)
+            off = 0
+            for step, nt, xs, zs, cs, _ in self.steps:
+                if step is not None:
+                    E.run_rows(step, th, pair)
+                E.check(L.lib().pqs_pauli_transition(ctx.handle, self.dtype, E.ptr(pair[0]), E.ptr(pair[1]), self.n,
+                                                     xs, zs, cs, nt, E.ptr(out[off:off + nt]), E.stream_ptr()))
+                off += nt
+            real = out[:off].cpu().numpy()[:, 0]
         grad = np.zeros(self.P)
-        owner = np.concatenate([s[5] for s in self.steps]) if self.steps else np.zeros(0, dtype=np.int64)
-        np.add.at(grad, owner, 2 * vals[:, 0])
+        np.add.at(grad, self.owner, 2 * real)
         return grad
 
 
-def apply_hamiltonian(H, psi, n, adjoint=False):
+# passes of one circuit before its fused plan is specialised (PQC.JIT_AFTER_USES)
+PASSES_BEFORE_JIT = 3
+
+
+def apply_hamiltonian(H, psi, n, adjoint=False, out=None):
     """H psi (or H^dag psi) for a PauliSum H on one state tensor."""
     ctx = E.context()
     terms = H.terms()
@@ -185,7 +268,7 @@ def apply_hamiltonian(H, psi, n, adjoint=False):
     cs = [complex(t[0]).conjugate() if adjoint else complex(t[0]) for t in terms]
     cf = (C.c_double * max(2, 2 * nt))(*[v for c in cs for v in (c.real, c.imag)])
     x = psi.reshape(-1).contiguous()
-    out = torch.empty_like(x)
+    out = torch.empty_like(x) if out is None else out
     E.check(L.lib().pqs_apply_pauli(ctx.handle, E.dtype_code(x.dtype), E.ptr(x), n, xm, zm, cf, nt, E.ptr(out),
                                     E.stream_ptr()))
     return out
@@ -201,17 +284,23 @@ def program(qc):
     return p
 
 
-def energy_and_gradient(qc, params, H=None):
+def energy_and_gradient(qc, params, H=None, psi=None):
     """(<psi|H|psi>, dE/dtheta) at ``params`` by the adjoint pass (H: the
-    circuit's Hamiltonian as a PauliSum by default)."""
+    circuit's Hamiltonian as a PauliSum by default; psi: the circuit's state
+    at ``params`` where the caller has it already)."""
     from .qobj import PauliSum
     prog = program(qc)
     if H is None:
         H = qc.hamiltonian()
     elif not isinstance(H, PauliSum):
         H = PauliSum.from_dense(H)
-    psi = E.run(qc.plan(), params, qc.init())[0]
     # lambda = H^dag psi, so that <lambda|d psi> = <psi|H|d psi> for any H
-    lam = apply_hamiltonian(H, psi, qc.n_qubits, adjoint=True)
-    energy = complex(E.inner(psi, lam).item()).real
-    return energy, prog.gradient(psi, lam, params)
+    pair = torch.empty((2, 1 << qc.n_qubits), dtype=E.CDTYPE[prog.dtype], device=E.device())
+    if psi is None:
+        E.run(qc.plan(), params, qc.init(), out=pair[1:2])
+    else:
+        pair[1].copy_(psi.reshape(-1))
+    apply_hamiltonian(H, pair[1], qc.n_qubits, adjoint=True, out=pair[0])
+    energy = E.inner(pair[1], pair[0])
+    grad = prog.gradient_of_pair(pair, params)
+    return complex(energy.item()).real, grad

@@ -192,11 +192,88 @@ template <int LB> __device__ __forceinline__ void lswap(V &x, V &y) {
 }
 )PQS";
 
+// Measurement plans: sums of per-lane values over the wave.
+static const char *kMeasPrelude = R"PQS(
+template <int LB> __device__ __forceinline__ void dswap(double &x, double &y) {
+  unsigned xs[2], ys[2];
+  __builtin_memcpy(xs, &x, 8);
+  __builtin_memcpy(ys, &y, 8);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if constexpr (LB == 5) {
+      const auto r = __builtin_amdgcn_permlane32_swap(xs[i], ys[i], false, false);
+      xs[i] = r[0];
+      ys[i] = r[1];
+    } else {
+      const auto r = __builtin_amdgcn_permlane16_swap(xs[i], ys[i], false, false);
+      xs[i] = r[0];
+      ys[i] = r[1];
+    }
+  }
+  __builtin_memcpy(&x, xs, 8);
+  __builtin_memcpy(&y, ys, 8);
+}
+template <int B> __device__ __forceinline__ double dxor(double x) {
+  int w[2];
+  __builtin_memcpy(w, &x, 8);
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    if constexpr (B == 3) w[i] = __builtin_amdgcn_update_dpp(0, w[i], 0x128, 0xf, 0xf, true);
+    else if constexpr (B == 2) {
+      w[i] = __builtin_amdgcn_update_dpp(0, w[i], 0x141, 0xf, 0xf, true);
+      w[i] = __builtin_amdgcn_update_dpp(0, w[i], 0x1b, 0xf, 0xf, true);
+    } else if constexpr (B == 1) w[i] = __builtin_amdgcn_update_dpp(0, w[i], 0x4e, 0xf, 0xf, true);
+    else w[i] = __builtin_amdgcn_update_dpp(0, w[i], 0xb1, 0xf, 0xf, true);
+  }
+  __builtin_memcpy(&x, w, 8);
+  return x;
+}
+// Totals over the wave of M values per lane (a power of two up to 16): each
+// step hands half of them to the lane across bit B; lane l ends with value
+// mfirst<M>(l) in v[0].
+template <int M, int B = 5> __device__ __forceinline__ void mfold(double *v, int lane) {
+  if constexpr (B >= 0) {
+    if constexpr (M > 1) {
+      constexpr int H = M / 2;
+      const bool up = (lane >> B) & 1;
+#pragma unroll
+      for (int i = 0; i < H; ++i) {
+        if constexpr (B >= 4) {
+          dswap<B>(v[i], v[i + H]);
+          v[i] += v[i + H];
+        } else {
+          const double keep = up ? v[i + H] : v[i], send = up ? v[i] : v[i + H];
+          v[i] = keep + dxor<B>(send);
+        }
+      }
+      mfold<H, B - 1>(v, lane);
+    } else {
+      if constexpr (B >= 4) {
+        double y = v[0];
+        dswap<B>(v[0], y);
+        v[0] += y;
+      } else {
+        v[0] += dxor<B>(v[0]);
+      }
+      mfold<1, B - 1>(v, lane);
+    }
+  }
+}
+template <int M> __device__ __forceinline__ int mfirst(int lane) {
+  int f = 0;
+#pragma unroll
+  for (int m = M / 2, b = 5; m > 0; m >>= 1, --b) f += ((lane >> b) & 1) * m;
+  return f;
+}
+)PQS";
+
 static constexpr int NA_() { return 1 << kRegBits; }
 // cmin, K and T of the scaled rotation form (comment at the top of this file)
 static double cos_min(const pqs_plan &p) { return p.dtype == PQS_C128 ? 1e-20 : 1e-7; }
-static int rot_per_check(const pqs_plan &p) { return p.dtype == PQS_C128 ? 10 : 4; }
-static double rescale_below(const pqs_plan &p) { return p.dtype == PQS_C128 ? 1e-100 : 1e-9; }
+// Measurements take products of two scaled amplitudes times f^2, so their
+// plans keep |f| >= 1e-60 * 1e-80: f^2 stays a normal number.
+static int rot_per_check(const pqs_plan &p) { return p.dtype != PQS_C128 || p.n_meas ? 4 : 10; }
+static double rescale_below(const pqs_plan &p) { return p.n_meas ? 1e-60 : p.dtype == PQS_C128 ? 1e-100 : 1e-9; }
 static int swz_host(int j) { return j ^ (((j >> 4) ^ (j >> 8) ^ (j >> 12)) & 15); }
 
 static std::string dbl(double v) {
@@ -232,7 +309,7 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o);
 
 static std::string prelude(const pqs_plan &p) {
   std::string t = p.dtype == PQS_C128 ? "typedef double R;\ntypedef double2 V;\n" : "typedef float R;\ntypedef float2 V;\n";
-  return t + kPrelude;
+  return t + kPrelude + (p.n_meas ? kMeasPrelude : "");
 }
 
 std::string jit_source_sweep(const pqs_plan &p, int s) {
@@ -320,7 +397,17 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
     // and writes the tile's share of <psi_2i|psi_2i+1> to pov[b].  Both
     // instances end in the same register / lane layout, so each thread pairs
     // its own amplitudes.
-    const bool emit_pair = s == S_total - 1 && !persist && p.n_tangents == 0;
+    const bool emit_pair = s == S_total - 1 && !persist && p.n_tangents == 0 && !p.n_meas;
+    // measurements of this sweep, in op order: output indices
+    std::vector<int> meas;
+    for (int i = ds.op_begin; i < ds.op_end; ++i)
+      if (p.dev_ops[i].kind == PQS_OP_MEAS) meas.push_back(p.dev_ops[i].term0);
+    const int nm = int(meas.size()), nwaves = std::max(1, nthr / 64);
+    if (nm) {
+      o << "__device__ const int MI" << s << "[" << nm << "] = {";
+      for (int i = 0; i < nm; ++i) o << (i ? "," : "") << meas[i];
+      o << "};\n";
+    }
   for (int pm = 0; pm < (emit_pair ? 2 : 1); ++pm) {
     const bool pair = pm == 1;
     // Block b processes flat tile b (flat tile = instance * n_tiles + tile).
@@ -330,10 +417,11 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
     // compute when only one block fits per CU.
     o << "extern \"C\" __global__ __launch_bounds__(" << nthr << ") void " << (pair ? "pqs_jit_pair_" : "pqs_jit_sweep_")
       << s << "(const InstDev *__restrict__ insts, long long n_active, const V *__restrict__ init_tab"
-      << (pair ? ", double2 *__restrict__ pov" : "") << ") {\n";
+      << (pair ? ", double2 *__restrict__ pov" : p.n_meas ? ", double *__restrict__ mpart" : "") << ") {\n";
     o << "  __shared__ V tile[" << S << "];\n";
     o << "  __shared__ double2 tf[" << (na > 0 ? na : 1) << "];\n";
     o << "  const int tid = threadIdx.x;\n";
+    if (nm) o << "  __shared__ double mred[" << nm * nwaves << "];\n";
     if (pair) {
       o << "  __shared__ double2 pred[" << std::max(1, nthr / 64) << "];\n";
       o << "  const long long total = (n_active >> 1) << " << (p.n - k) << ";\n";
@@ -487,6 +575,8 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
       return v;
     };
     std::vector<int> next_pre;
+    int n_meas_done = 0;  // measurements whose wave totals are in mred
+    int mg = 0;           // groups emitted (names)
     bool carry = false;
     int nrot = 0;  // rotations since the last check of the accumulated scale
     // phases
@@ -561,10 +651,32 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
           fl[r] = false;
         }
       };
+      // Measurements: each leaves a per-thread value; up to 16 of them are
+      // summed over the wave together.  conj(a) b per pair of amplitudes is
+      // not changed by diagonal gates (both halves turn alike) and serves
+      // every Z string until the next non-diagonal op ("wz<id>", "wt<id>").
+      std::vector<std::string> mvals;
+      int wz_id = -1, wz_count = 0;
+      int wz_parts = 0;  // 1: real products there, 2: imaginary ones
+      bool wz_total[2] = {false, false};
+      auto flush_meas = [&]() {
+        if (mvals.empty()) return;
+        int M = 1;
+        while (M < int(mvals.size())) M *= 2;
+        o << "    { double mv[" << M << "] = {";
+        for (int j = 0; j < M; ++j) o << (j ? ", " : "") << (j < int(mvals.size()) ? mvals[size_t(j)] : "0.0");
+        o << "};\n      const int ln = ptid & 63;\n      mfold<" << M << ">(mv, ln);\n      const int f = mfirst<" << M
+          << ">(ln);\n      if ((ln & " << (64 / M - 1) << ") == 0 && f < " << mvals.size() << ") mred[(ptid >> 6) * "
+          << nm << " + " << n_meas_done << " + f] = mv[0]; }\n";
+        n_meas_done += int(mvals.size());
+        ++mg;
+        mvals.clear();
+      };
       for (int i = P.op_begin; i < P.op_end; ++i) {
         const DevOp &d = p.dev_ops[i];
         const int ai = ang[i - ds.op_begin];
         const bool r0 = d.r0 >= 0, r1 = d.r1 >= 0;
+        if (d.kind != PQS_OP_MEAS && d.kind != PQS_OP_RZ && d.kind != PQS_OP_RZZ && d.kind != PQS_OP_CZ) wz_id = -1;
         if (is_rot(d.kind)) {
           if (nrot == rot_per_check(p)) {
             o << "    if (fabs(fs) < " << dbl(rescale_below(p)) << ") { rscale(a, R(fs)); fs = 1.0; }\n";
@@ -606,6 +718,89 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
             } else
               o << "    { const double2 c = " << aexpr(ai) << "; fs *= c.y; pall(a, (" << cbit_expr(d, 0) << " ^ "
                 << cbit_expr(d, 1) << ") ? R(-c.x) : R(c.x)); }\n";
+            break;
+          }
+          case PQS_OP_MEAS: {
+            // Re(c <a|P|b>): (P b)[j] = (-1)^{z.(j ^ x)} b[j ^ x], i^{#Y} in c
+            int top = -1;  // register bit of the pair's qubit
+            for (int r = 0; r < kRegBits; ++r)
+              if (P.rb[r] == ds.pair_bit) top = r;
+            const bool xx = d.pauli == 1 || d.pauli == 2, zz = d.pauli == 2 || d.pauli == 3;
+            int xr = 0, zr = 0;
+            std::string sign;  // the lane's part of the sign, as a bit expression
+            auto add_sign = [&](const std::string &e) { sign += sign.empty() ? e : " ^ " + e; };
+            for (int w = 0; w < (d.g1 >= 0 ? 2 : 1); ++w) {
+              const int r = w ? d.r1 : d.r0;
+              if (xx) xr |= 1 << r;
+              if (!zz) continue;
+              if (r >= 0) {
+                zr |= 1 << r;
+                if (fl[r]) add_sign(xf(r));
+              } else {
+                add_sign(cbit_expr(d, w));
+              }
+            }
+            const bool want[2] = {d.m[0] != 0, d.m[1] != 0};
+            const std::string id = std::to_string(ph - ds.phase_begin) + "_" + std::to_string(i - ds.op_begin);
+            auto prod = [&](int part, int v) {  // conj(a) (P b) without the sign, one part
+              const std::string A = "a[" + std::to_string(v) + "]", B = "a[" + std::to_string((v ^ xr) | (1 << top)) + "]";
+              return part == 0 ? "fma(" + A + ".x, " + B + ".x, " + A + ".y * " + B + ".y)"
+                               : "fma(" + A + ".x, " + B + ".y, -" + A + ".y * " + B + ".x)";
+            };
+            o << "    double me" << id << " = 0.0;\n";
+            for (int part = 0; part < 2; ++part) {
+              if (!want[part]) continue;
+              const std::string c = dbl(part == 0 ? d.m[0] : -d.m[1]);
+              if (!xx) {
+                // products shared by the Z strings of this point, true scale
+                if (wz_id < 0) {
+                  wz_id = wz_count++;
+                  wz_parts = 0;
+                  wz_total[0] = wz_total[1] = false;
+                }
+                const std::string nm_ = std::to_string(ph - ds.phase_begin) + "_" + std::to_string(wz_id) + "_" + std::to_string(part);
+                if (!((wz_parts >> part) & 1)) {
+                  o << "    double wz" << nm_ << "[8]; { const double f2 = fs * fs;\n";
+                  int q = 0;
+                  for (int v = 0; v < NA_(); ++v)
+                    if (!((v >> top) & 1)) o << "      wz" << nm_ << "[" << q++ << "] = (" << prod(part, v) << ") * f2;\n";
+                  o << "    }\n";
+                  wz_parts |= 1 << part;
+                }
+                std::string sum;
+                if (zr == 0) {
+                  if (!wz_total[part]) {
+                    o << "    const double wt" << nm_ << " = ((wz" << nm_ << "[0] + wz" << nm_ << "[1]) + (wz" << nm_
+                      << "[2] + wz" << nm_ << "[3])) + ((wz" << nm_ << "[4] + wz" << nm_ << "[5]) + (wz" << nm_
+                      << "[6] + wz" << nm_ << "[7]));\n";
+                    wz_total[part] = true;
+                  }
+                  sum = "wt" + nm_;
+                } else {
+                  int q = 0;
+                  for (int v = 0; v < NA_(); ++v) {
+                    if ((v >> top) & 1) continue;
+                    sum += (__builtin_popcount(unsigned(v & zr)) & 1 ? " - wz" : q ? " + wz" : "wz") + nm_ + "[" + std::to_string(q) + "]";
+                    ++q;
+                  }
+                }
+                o << "    me" << id << " += " << c << " * (" << sum << ");\n";
+              } else {
+                o << "    { double t = 0.0;\n";
+                for (int v = 0; v < NA_(); ++v) {
+                  if ((v >> top) & 1) continue;
+                  const bool neg = __builtin_popcount(unsigned((v ^ xr) & zr)) & 1;
+                  const std::string A = "a[" + std::to_string(v) + "]", B = "a[" + std::to_string((v ^ xr) | (1 << top)) + "]";
+                  const std::string sA = (neg ? "-" : "") + A, nA = (neg ? "" : "-") + A;
+                  if (part == 0) o << "      t = fma(" << sA << ".x, " << B << ".x, fma(" << sA << ".y, " << B << ".y, t));\n";
+                  else o << "      t = fma(" << sA << ".x, " << B << ".y, fma(" << nA << ".y, " << B << ".x, t));\n";
+                }
+                o << "      me" << id << " += " << c << " * t * fs * fs; }\n";
+              }
+            }
+            if (!sign.empty()) o << "    if (" << sign << ") me" << id << " = -me" << id << ";\n";
+            mvals.push_back("me" + id);
+            if (mvals.size() == 16) flush_meas();
             break;
           }
           case PQS_OP_RXX:  // X flips commute with X(x)X
@@ -727,6 +922,7 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
             break;
         }
       }
+      flush_meas();
       // Exchange into the next phase: its layout is this one with register
       // bits traded against lane bits 5 / 4, so the amplitudes move with
       // cross-lane swaps and stay in registers (no LDS round trip, no
@@ -847,6 +1043,11 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
       o << "  }\n";
     }
     if (!pair) {
+      if (nm) {
+        o << "  __syncthreads();\n  for (int i = tid; i < " << nm << "; i += " << nthr << ") {\n    double x = mred[i];\n";
+        for (int w = 1; w < nwaves; ++w) o << "    x += mred[" << w * nm << " + i];\n";
+        o << "    mpart[t * " << p.n_meas << "ll + MI" << s << "[i]] = x;\n  }\n";
+      }
       o << "  }\n}\n";
       continue;
     }

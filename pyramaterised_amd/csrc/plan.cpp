@@ -59,9 +59,9 @@ static int validate(int n, const pqs_op &o, int idx) {
     std::snprintf(buf, sizeof buf, "op %d (kind %d): %s", idx, o.kind, what);
     return fail(PQS_ERR_ARG, buf);
   };
-  if (o.kind < PQS_OP_MAT1 || o.kind > PQS_OP_GEN_FSIM) return bad("unknown kind");
+  if (o.kind < PQS_OP_MAT1 || o.kind > PQS_OP_MEAS) return bad("unknown kind");
   if (o.q0 < 0 || o.q0 >= n) return bad("q0 out of range");
-  bool two = is_two_qubit(o.kind) || (o.kind == PQS_OP_GEN && o.q1 >= 0);
+  bool two = is_two_qubit(o.kind) || ((o.kind == PQS_OP_GEN || o.kind == PQS_OP_MEAS) && o.q1 >= 0);
   if (two) {
     if (o.q1 < 0 || o.q1 >= n) return bad("q1 out of range");
     if (o.q1 == o.q0) return bad("q0 == q1");
@@ -72,6 +72,8 @@ static int validate(int n, const pqs_op &o, int idx) {
     if (o.kind == PQS_OP_GEN && (o.pauli < 0 || o.pauli > 3)) return bad("pauli must be 0..3");
     if (o.kind == PQS_OP_GEN_FSIM && (o.pauli < 1 || o.pauli > 3)) return bad("fSim derivative selector must be 1..3");
     if (o.kind == PQS_OP_GEN_FSIM && o.pauli != 3 && o.slot2 < 0) return bad("fSim derivative without a phi slot");
+  } else if (o.kind == PQS_OP_MEAS && (o.pauli < 0 || o.pauli > 3)) {
+    return bad("pauli must be 0..3");
   } else if (o.tangent >= 0) {
     return bad("only derivative ops carry a tangent index");
   }
@@ -94,7 +96,7 @@ static void masks_of(int n, const pqs_op &o, qmask &active, qmask &diag) {
     case PQS_OP_MAT2: case PQS_OP_RXX: case PQS_OP_RYY: case PQS_OP_FSIM: case PQS_OP_GEN_FSIM:
       active |= bitq(o.q0) | bitq(o.q1);
       break;
-    case PQS_OP_GEN: {
+    case PQS_OP_GEN: case PQS_OP_MEAS: {
       qmask qs = bitq(o.q0) | (o.q1 >= 0 ? bitq(o.q1) : 0);
       if (o.pauli == 1 || o.pauli == 2) active |= qs;
       else if (o.pauli == 3) diag |= qs;
@@ -224,6 +226,14 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
         w.c = o;
         break;
       }
+      case PQS_OP_MEAS: {
+        WaveOp &w = emit(kWMeas);
+        w.x = d.pauli == 1 || d.pauli == 2 ? b0 | b1 : 0;
+        w.z = d.pauli == 2 || d.pauli == 3 ? b0 | b1 : 0;
+        w.c = o;
+        w.tangent = d.term0;
+        break;
+      }
       default: {  // PQS_OP_MAT2
         WaveOp &w = emit(kWMat2);
         w.x = b0;
@@ -245,6 +255,7 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
     switch (d.kind) {
       case PQS_OP_RZ: case PQS_OP_RZZ: case PQS_OP_CZ: break;
       case PQS_OP_CX: act = b1; break;
+      case PQS_OP_MEAS: act = d.pauli == 1 || d.pauli == 2 ? all : 0; break;
       case kPauliSum: {
         all = 0;
         for (int t = d.term0; t < d.term0 + d.nterms; ++t) {
@@ -367,11 +378,23 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
   p.sweeps.clear();
   p.n_tangents = 0;
   p.n_sub = 0;
+  p.n_meas = 0;
 
+  bool pair_touched = false;
   for (int i = 0; i < n_ops; ++i) {
     int rc = validate(n, ops[i], i);
     if (rc) return rc;
+    if (ops[i].kind == PQS_OP_MEAS) ++p.n_meas;
+    pair_touched = pair_touched || ops[i].q0 == 0 || (is_two_qubit(ops[i].kind) && ops[i].q1 == 0) ||
+                   ((ops[i].kind == PQS_OP_GEN || ops[i].kind == PQS_OP_MEAS) && ops[i].q1 == 0);
     if (ops[i].tangent >= 0) p.n_tangents = std::max(p.n_tangents, ops[i].tangent + 1);
+  }
+
+  if (p.n_meas) {
+    if (pair_touched) return fail(PQS_ERR_ARG, "with measurements, no op acts on qubit 0 (the pair)");
+    if (p.n_tangents) return fail(PQS_ERR_ARG, "measurements and derivative ops in one plan");
+    if (p.dtype != PQS_C128) return fail(PQS_ERR_UNSUPPORTED, "measurement plans are complex128");
+    if (k < std::min(n, 4)) return fail(PQS_ERR_UNSUPPORTED, "measurement plans need tiles of 4 qubits");
   }
 
   // Merge consecutive generator terms of one tangent into a Pauli sum.  A sum
@@ -458,6 +481,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
       i = j;
     } else {
       e.kind = ops[i].kind;
+      if (e.kind == PQS_OP_MEAS) e.need = bitq(0);
       if (e.kind == PQS_OP_GEN_FSIM) e.tangent = part_tangent(ops[i].tangent, true);
       ++i;
     }
@@ -473,6 +497,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
 
   // Positions: pos(q) = n-1-q.  Forced low positions 0..low-1 = qubits n-1..n-low.
   qmask forced = 0;
+  const qmask always = p.n_meas ? bitq(0) : 0;  // the pair's qubit: in every tile
   for (int b = 0; b < low; ++b) forced |= bitq(n - 1 - b);
   qmask all = (n == 64) ? ~qmask(0) : ((qmask(1) << n) - 1);
 
@@ -488,7 +513,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
                       std::vector<int> &rest) {
     run.clear();
     for (int attempt = 0; attempt < 2 && run.empty(); ++attempt) {
-      T = (n <= k) ? all : (attempt == 0 ? want : 0);
+      T = (n <= k) ? all : ((attempt == 0 ? want : 0) | always);
       run.clear();
       rest.clear();
       qmask blocked_any = 0, blocked_nd = 0;
@@ -547,7 +572,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
                         std::vector<int> &run, std::vector<int> &rest) {
     plan_one(rem, want, T, run, rest);
     if (!run.empty() && p.rolling && rest.empty() && (T & forced) != forced &&
-        popc(want | forced) <= k) {
+        popc(want | forced | always) <= k) {
       // the last sweep writes the standard layout: keep its lowest qubits in
       // the tile (a shorter last sweep and one more are cheaper than a
       // scattered final write)
@@ -606,8 +631,8 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
   // fewest sweeps (a full look-ahead was both slower and worse), so the
   // partition is built for horizons 1, 2 and 3 and the one with the fewest
   // sweeps is kept.
-  const bool search = p.rolling && !(o.flags & PQS_PLAN_GREEDY_SWEEPS) && low < k;
-  const int win = k - low;
+  const bool search = p.rolling && !(o.flags & PQS_PLAN_GREEDY_SWEEPS) && low + popc(always) < k;
+  const int win = k - low - popc(always);
   auto partition = [&](int horizon, std::vector<Sweep> &out) {
     out.clear();
     std::vector<int> rem(p.exec.size());
@@ -625,7 +650,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
         qmask T2;
         std::vector<int> run2, rest2;
         for (int s0 = 0; s0 + win <= n; ++s0) {
-          const qmask W = want | (((qmask(1) << win) - 1) << s0);
+          const qmask W = want | always | (((qmask(1) << win) - 1) << s0);
           if (popc(W) > k) continue;
           sweep_from(W, prevT, rem, T2, run2, rest2);
           if (run2.empty() || (!first && popc(T2 & prevT) < low)) continue;
@@ -704,6 +729,10 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
       if (tg >= 0 && p.tangent_sweep[tg] < 0) p.tangent_sweep[tg] = int(s);
     }
 
+  std::vector<int> meas_index(size_t(n_ops), 0);  // ordinal of a PQS_OP_MEAS
+  for (int i = 0, m = 0; i < n_ops; ++i)
+    if (ops[i].kind == PQS_OP_MEAS) meas_index[size_t(i)] = m++;
+
   // ---- register phases and device image
   // Tiles of kRegBits + 6 qubits and more fill at least one wave with
   // 2^kRegBits amplitudes per thread: the register-phase executor.  Smaller
@@ -753,6 +782,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
       return nr;
     };
     ds.k = int(tpos.size());
+    ds.pair_bit = p.n_meas ? tile_index[0] : -1;
     ds.nruns = runs(tpos, ds.run_pos, ds.run_len, ds.run_shift);
     ds.cnruns = runs(cpos, ds.crun_pos, ds.crun_len, ds.crun_shift);
     ds.n_tiles = int64_t(1) << cpos.size();
@@ -784,7 +814,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
         if (kind == PQS_OP_MAT2 || kind == PQS_OP_RXX || kind == PQS_OP_RYY || kind == PQS_OP_FSIM ||
             kind == PQS_OP_GEN_FSIM)
           return p.dtype == PQS_C128;  // both qubits become register bits
-        return kind == PQS_OP_MAT1 || kind == PQS_OP_RX || kind == PQS_OP_RY || kind == PQS_OP_RZ ||
+        return kind == PQS_OP_MEAS || kind == PQS_OP_MAT1 || kind == PQS_OP_RX || kind == PQS_OP_RY || kind == PQS_OP_RZ ||
                kind == PQS_OP_CX || kind == PQS_OP_CZ || kind == PQS_OP_RZZ;
       };
       qmask tmask = 0;  // qubits of this sweep's tile
@@ -816,11 +846,12 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
             const qmask soft = ((e.kind == PQS_OP_CX || e.kind == PQS_OP_CZ) && !(p.flags & PQS_PLAN_NO_SOFT_REGS))
                                    ? (e.diag & tmask)
                                    : 0;
-            if (!dep && popc(R | e.active | soft) <= kRegBits) {
-              R |= e.active | soft;
+            const qmask hold = e.active | e.need;
+            if (!dep && popc(R | hold | soft) <= kRegBits) {
+              R |= hold | soft;
               run.push_back(ei);
-            } else if (!dep && popc(R | e.active) <= kRegBits) {
-              R |= e.active;
+            } else if (!dep && popc(R | hold) <= kRegBits) {
+              R |= hold;
               run.push_back(ei);
             } else {
               rest.push_back(ei);
@@ -869,8 +900,10 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
             PhAhead best = greedy_phases(rest);
             qmask R2;
             std::vector<int> run2, rest2;
-            for (int q0 = 0; q0 + kRegBits <= n; ++q0) {
-              const qmask W = ((qmask(1) << kRegBits) - 1) << q0;
+            // (with measurements: their qubit and kRegBits - 1 more)
+            const int wbits = kRegBits - popc(always);
+            for (int q0 = popc(always); q0 + wbits <= n; ++q0) {
+              const qmask W = always | (((qmask(1) << wbits) - 1) << q0);
               if ((W & tmask) != W) continue;
               phase_from(rem, W, R2, run2, rest2);
               if (run2.empty()) continue;
@@ -1239,6 +1272,16 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
         d.r0 = d.t0 >= 0 ? reg_index[d.t0] : -1;
         d.r1 = d.t1 >= 0 ? reg_index[d.t1] : -1;
         d.coef = -1;
+        if (e.kind == PQS_OP_MEAS) {
+          // output index, and the coefficient with i^{#Y}
+          d.term0 = meas_index[size_t(e.first)];
+          d.slot = d.slot2 = -1;
+          for (int y = so.pauli == 2 ? (so.q1 >= 0 ? 2 : 1) : 0; y > 0; --y) {
+            const double t2 = d.m[0];
+            d.m[0] = -d.m[1];
+            d.m[1] = t2;
+          }
+        }
         if (p.reg_exec && !ph.lds) {
           const qmask act = e.active;
           if (((act >> so.q0) & 1) && d.r0 < 0) return fail(PQS_ERR_UNSUPPORTED, "internal planner error: active qubit not in registers");

@@ -24,6 +24,7 @@ struct ExecOp {
   qmask active = 0;      // qubits the op acts on non-diagonally
   qmask diag = 0;        // qubits the op acts on diagonally (block-diagonal)
   int tangent = -1;      // derivative ops: tangent (or sub-tangent) index
+  qmask need = 0;        // further qubits held in the tile and in registers
 };
 constexpr int kPauliSum = 100;
 // A one-term, one-qubit generator (coef * Pauli on q0, applied only by the
@@ -101,6 +102,7 @@ struct DevSweep {
   // first (last) register phase, so the specialised kernel loads (stores)
   // that phase's registers directly, without staging the tile in LDS.
   int32_t direct_load, direct_store;
+  int32_t pair_bit;  // measurement plans: tile bit of qubit 0
 };
 
 // ---- op stream of the wave executor (complex128 tiles below 10 qubits)
@@ -133,7 +135,8 @@ enum WaveCode : int32_t {
   kWSum,      // Pauli sum of DevOp c, for its tangent
   kWFsim,     // on bits x: theta at ang, phi at z (-1: phi = 0)
   kWGenFsim,  // as kWFsim, DevOp c, for its tangent
-  kWMat2      // 4x4 of DevOp c, q0 = bit x, q1 = bit z
+  kWMat2,     // 4x4 of DevOp c, q0 = bit x, q1 = bit z
+  kWMeas      // PQS_OP_MEAS of DevOp c, masks x and z, output `tangent`
 };
 struct alignas(16) WaveOp {
   uint16_t code, ang;  // ang: index into the angles of the last refill
@@ -164,6 +167,7 @@ struct pqs_plan {
   // the first runs as a sub-tangent n_tangents.. whose state is summed into
   // its parent's row at the end of a run.  n_sub counts all of them.
   int n_sub = 0;
+  int n_meas = 0;  // PQS_OP_MEAS ops: qubit 0 is then in every tile
   std::vector<int> tangent_parent;  // per tangent / sub-tangent: caller tangent
   std::vector<pqs_op> src_ops;
   std::vector<pqs::ExecOp> exec;

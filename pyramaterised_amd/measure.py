@@ -318,7 +318,7 @@ class Measurements:
         self._grad_states = None
         try:
             from . import adjoint
-            _, g = adjoint.energy_and_gradient(self.QC, self.QC._params_vec())
+            _, g = adjoint.energy_and_gradient(self.QC, self.QC._params_vec(), psi=self.QC.state.t)
             return list(g)
         except NotImplementedError:
             pass

@@ -109,3 +109,47 @@ def test_gradient_vector_and_autograd_use_the_adjoint(pyqc):
     gf = pyqc.measure.Measurements(qf).get_gradient_vector(list(thf))
     _, gf_ref = _oracle(ogf, thf, 6, qf.hamiltonian().full(), OC.half_filled(6))
     assert np.max(np.abs(np.array(gf) - gf_ref)) < 1e-12
+
+
+@pytest.mark.parametrize("which", ["hea", "tfim", "xxz", "mixed"])
+@pytest.mark.parametrize("n", [4, 8, 9, 10, 11, 13])
+def test_fused_pass_matches_point_by_point(pyqc, which, n):
+    """The one-plan backward pass (pqs_adjoint: the wave executor up to 8
+    qubits, one specialised tile up to 11, several with rolling layouts
+    beyond) against the point-by-point pass, and pi-rotations in it.  Both
+    round each amplitude by a few eps per gate, so gradients of size <= 4
+    agree to 1e-12."""
+    from pyramaterised_amd import adjoint
+    from pyramaterised_amd import templates as T
+    if which == "xxz" and n % 2:
+        pytest.skip("the XXZ template couples pairs of an even ring")
+    qc = pyqc.PQC(n)
+    if which == "mixed":
+        layer = [pyqc.R_x(q, n) for q in range(n)] + [pyqc.CHAIN(pyqc.CZ, n), pyqc.H(0, n), pyqc.S(1, n)]
+        layer += [pyqc.R_yy([0, n - 1], n), pyqc.R_xx([1, 2], n), pyqc.sqrtiSWAP([0, 2], n), pyqc.R_zz([n - 1, 1], n)]
+        layer += [pyqc.R_z(q, n) for q in range(n)] + [pyqc.CNOT([n - 1, 0], n), pyqc.R_y(n - 1, n)]
+        layers = [layer, layer]
+    else:
+        layers = {"hea": lambda: T.clifford_HE_layers(3, n), "tfim": lambda: T.TFIM_layers(2, n),
+                  "xxz": lambda: T.XXZ_layers(2, n)}[which]()
+    for l in layers:
+        qc.add_layer(l)
+    th = np.random.default_rng(n).random(qc.n_true_params) * 2 * np.pi
+    th[::4] = np.pi
+    H = _hamiltonian(pyqc, n)
+    prog = adjoint.program(qc)
+    prog._want_jit = False
+    prog._may_jit = False
+    prog.FUSED_PARTIAL_BYTES = -1 if n + 1 >= 10 else prog.FUSED_PARTIAL_BYTES
+    prog._fused = False  # point by point
+    e0, g0 = adjoint.energy_and_gradient(qc, th, H)
+    prog._fused, prog._want_jit, prog.FUSED_PARTIAL_BYTES = None, True, 1 << 32
+    print(f"fused adjoint {which} n={n}", flush=True)
+    e1, g1 = adjoint.energy_and_gradient(qc, th, H)
+    assert prog.fused_plan() is not None
+    assert abs(e0 - e1) < 1e-12
+    assert np.max(np.abs(g0 - g1)) < 1e-12
+    psi = qc.run(list(th))
+    e2, g2 = adjoint.energy_and_gradient(qc, th, H, psi=psi.t)  # the state in hand, left as it is
+    assert np.max(np.abs(g2 - g1)) < 1e-12
+    assert abs(psi.norm() - 1) < 1e-12
