@@ -334,7 +334,7 @@ class PQC:
     # circuit into segments of local gates, each run as its own plan, with
     # the dense operator applied on the GPU in between (pqs_apply_dense).
     def has_dense(self):
-        return any(getattr(g, "dense", False) for g in self.gates)
+        return any([getattr(g, "dense", False) for g in self.gates])
 
     def _segments(self):
         """[(local gates, dense gate or None)] in gate order."""

@@ -2525,7 +2525,7 @@ static __device__ __align__(256) unsigned char scratch[kNoallocMaxBatch * sizeof
 // Instance table of a strided batch, written on the device (no host copy).
 __global__ __launch_bounds__(256) void k_fill_batch_table(InstDev *__restrict__ tab, char *states, int64_t state_bytes,
                                                           int64_t batch, const double *params, int64_t param_stride,
-                                                          int32_t init, const void *src, char *alt,
+                                                          int32_t init, const void *src, char *alt, int64_t alt_bytes,
                                                           int32_t pingpong) {
   const int64_t i = int64_t(blockIdx.x) * 256 + threadIdx.x;
   if (i >= batch) return;
@@ -2533,7 +2533,7 @@ __global__ __launch_bounds__(256) void k_fill_batch_table(InstDev *__restrict__ 
   d.state = states + i * state_bytes;
   d.src = src;
   d.params = params ? params + i * param_stride : nullptr;
-  d.alt = pingpong ? alt + i * state_bytes : nullptr;
+  d.alt = pingpong ? alt + i * alt_bytes : nullptr;
   d.tangent = -1;
   d.init = init;
   d.start_sweep = 0;
@@ -2634,6 +2634,27 @@ __global__ void k_upload1(const unsigned char *__restrict__ src, unsigned char *
     dst[i] = src[i];
 }
 
+// Small uploads travel in the launch's argument block: the runtime copies the
+// arguments when the kernel is queued, so no staging buffer is held and no
+// event recorded or queried for it (a 4-qubit state, whose call makes two such
+// uploads: 62 -> 58 us).
+constexpr size_t kArgUpload = 2048;
+struct alignas(16) ArgBlob {
+  unsigned char b[kArgUpload];
+};
+__global__ __launch_bounds__(128) void k_upload_arg(const ArgBlob blob, unsigned char *__restrict__ dst, int bytes) {
+  // the first argument in place, read through the argument segment (indexing
+  // the parameter itself would copy it to scratch memory)
+  const auto *src = (const unsigned char *)__builtin_amdgcn_kernarg_segment_ptr();
+  const int i = threadIdx.x * 16;
+  if (((uintptr_t(dst) | unsigned(bytes)) & 15) == 0) {
+    if (i < bytes)
+      *reinterpret_cast<uint4 *>(dst + i) = *reinterpret_cast<const uint4 *>(src + i);
+  } else {
+    for (int j = i; j < i + 16 && j < bytes; ++j) dst[j] = src[j];
+  }
+}
+
 // true once the event's work has run; false while it is pending (the
 // not-ready status is cleared so that a later launch check does not see it)
 bool event_done(hipEvent_t ev) {
@@ -2643,10 +2664,18 @@ bool event_done(hipEvent_t ev) {
   return false;
 }
 
-// Copy host bytes to device memory in stream order: into a pinned staging
-// buffer now, then by a copy kernel on `st`, which reads the pinned buffer.
+// Copy host bytes to device memory in stream order: small ones as a launch's
+// argument, others into a pinned staging buffer now, then by a copy kernel on
+// `st`, which reads the pinned buffer.
 int upload(pqs_ctx *ctx, void *dst, const void *src, size_t bytes, hipStream_t st) {
   if (bytes == 0) return PQS_OK;
+  if (bytes <= kArgUpload) {
+    ArgBlob blob;
+    std::memcpy(blob.b, src, bytes);
+    hipLaunchKernelGGL(k_upload_arg, dim3(1), dim3(128), 0, st, blob, (unsigned char *)dst, int(bytes));
+    HIPCHECK(hipGetLastError());
+    return PQS_OK;
+  }
   auto &pins = ctx->pins;
   const int n_slots = int(pins.size());
   int k = -1;
@@ -2685,16 +2714,29 @@ int upload(pqs_ctx *ctx, void *dst, const void *src, size_t bytes, hipStream_t s
   }
   ctx->pin_next = (k + 1) % int(pins.size());
   pqs_ctx::PinSlot &sl = pins[size_t(k)];
-  std::memcpy(sl.host, src, bytes);
+  // In pieces, so that the host copies one while the kernel fetches the one
+  // before it; 64 blocks keep the link busy, and more only crowd it (1.28 MB:
+  // 70 us as one piece of 313 blocks, 51 us in two; 36 against 42 us for the
+  // kernel alone).
+  constexpr size_t kPiece = size_t(512) << 10;
   const bool wide = (reinterpret_cast<uintptr_t>(dst) & 15) == 0 && (bytes & 15) == 0;
-  const int64_t n = wide ? int64_t(bytes >> 4) : int64_t(bytes);
-  const int64_t blocks = std::min<int64_t>((n + 255) / 256, 1024);
-  if (wide)
-    hipLaunchKernelGGL(k_upload16, dim3(unsigned(blocks)), dim3(256), 0, st, (const uint4 *)sl.host, (uint4 *)dst, n);
-  else
-    hipLaunchKernelGGL(k_upload1, dim3(unsigned(blocks)), dim3(256), 0, st, (const unsigned char *)sl.host,
-                       (unsigned char *)dst, n);
-  HIPCHECK(hipGetLastError());
+  for (size_t o = 0; o < bytes; o += kPiece) {
+    const size_t c = std::min(kPiece, bytes - o);
+    unsigned char *host = (unsigned char *)sl.host + o, *to = (unsigned char *)dst + o;
+    std::memcpy(host, (const unsigned char *)src + o, c);
+    const int64_t n = wide ? int64_t(c >> 4) : int64_t(c);
+    const int64_t blocks = std::min<int64_t>((n + 255) / 256, wide ? 64 : 1024);
+    if (wide)
+      hipLaunchKernelGGL(k_upload16, dim3(unsigned(blocks)), dim3(256), 0, st, (const uint4 *)host, (uint4 *)to, n);
+    else
+      hipLaunchKernelGGL(k_upload1, dim3(unsigned(blocks)), dim3(256), 0, st, host, to, n);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+      // pieces already queued still read the buffer
+      if (o && hipEventRecord(sl.event, st) == hipSuccess) sl.pending = true;
+      return hip_fail(e, "upload");
+    }
+  }
   HIPCHECK(hipEventRecord(sl.event, st));
   sl.pending = true;
   return PQS_OK;
@@ -3067,6 +3109,57 @@ static int launch_add_rows(pqs_plan *p, const AccRow *d_acc, const void *const *
   return PQS_OK;
 }
 
+// Partials per pair of a batch's overlaps (0: none wanted): per last-sweep tile
+// where the last sweep's pair kernel forms them (fused), else per chunk.
+static int64_t pair_chunks(const pqs_ctx *ctx, const pqs_plan *p, bool pairs, bool &fused) {
+  const int S = int(p->dev_sweeps.size());
+  fused = pairs && S > 0 && p->jit_pair_fn && p->jit_module && p->dev_device == ctx->device &&
+          S - 1 < int(p->jit_fn.size()) && p->jit_fn[size_t(S - 1)];
+  if (!pairs) return 0;
+  return fused ? p->dev_sweeps[size_t(S - 1)].n_tiles : ((int64_t(1) << p->n) + kInnerChunk - 1) / kInnerChunk;
+}
+
+// Every sweep over the n_all instances of the table, the first n_main of them
+// the caller's; with pair_out also the overlaps of their pairs (states from
+// `first`, `stride` amplitudes apart, where they are read back).
+static int launch_sweeps(pqs_ctx *ctx, pqs_plan *p, const InstDev *d_tab, int64_t n_all, int64_t n_main, const void *first,
+                         int64_t stride, const void *init_tab, hipStream_t st, bool fused, int64_t n_chunks, double2 *pov,
+                         double *pair_out) {
+  const int S_sw = int(p->dev_sweeps.size());
+  const int64_t n_pairs = pair_out ? n_main / 2 : 0;
+  for (int s = 0; s < S_sw; ++s) {
+    if (fused && s == S_sw - 1) {
+      if (n_pairs == 0) break;
+      const DevSweep &sw = p->dev_sweeps[size_t(s)];
+      const int nthr = (1 << sw.k) >> pqs::kRegBits;
+      const int64_t grid = n_pairs * sw.n_tiles;
+      if (grid > 0x7fffffff) return fail(PQS_ERR_UNSUPPORTED, "grid too large: split the batch");
+      long long na = (long long)n_all;
+      void *args[] = {(void *)&d_tab, (void *)&na, (void *)&init_tab, (void *)&pov};
+      HIPCHECK(hipModuleLaunchKernel((hipFunction_t)p->jit_pair_fn, unsigned(grid), 1, 1, unsigned(nthr), 1, 1, 0, st,
+                                     args, nullptr));
+      break;
+    }
+    const int rc = launch_sweep(ctx, p, s, d_tab, n_all, init_tab, st);
+    if (rc) return rc;
+  }
+  if (n_pairs == 0) return PQS_OK;
+  if (!fused) {
+    const int64_t dim = int64_t(1) << p->n, grid = n_pairs * n_chunks;
+    if (grid > 0x7fffffff) return fail(PQS_ERR_UNSUPPORTED, "too many pairs x chunks");
+    if (p->dtype == PQS_C128)
+      hipLaunchKernelGGL(k_pair_partial<double>, dim3(unsigned(grid)), dim3(RB), 0, st, (const double2 *)first, stride,
+                         dim, n_chunks, pov);
+    else
+      hipLaunchKernelGGL(k_pair_partial<float>, dim3(unsigned(grid)), dim3(RB), 0, st, (const float2 *)first, stride,
+                         dim, n_chunks, pov);
+    HIPCHECK(hipGetLastError());
+  }
+  hipLaunchKernelGGL(k_sum_rows, dim3(unsigned(n_pairs)), dim3(RB), 0, st, pov, n_chunks, (double2 *)pair_out);
+  HIPCHECK(hipGetLastError());
+  return PQS_OK;
+}
+
 // Run instances h of plan p (pqs_run, pqs_run_batch).
 //  - An instance whose tangent's generator was split into parts gets one
 //    extra instance per further part, evolving a workspace row from the same
@@ -3114,14 +3207,9 @@ static int run_instances(pqs_ctx *ctx, pqs_plan *p, std::vector<InstDev> &h, con
   }
   const size_t acc_off = al(tab_off + n_all * sizeof(InstDev));
   const size_t src_off = al(acc_off + acc.size() * sizeof(AccRow));
-  const int S_sw = int(p->dev_sweeps.size());
   const int64_t n_pairs = int64_t(n_main / 2);
-  const bool fused = pair_out && S_sw > 0 && parts.empty() && p->jit_pair_fn && p->jit_module &&
-                     p->dev_device == ctx->device && S_sw - 1 < int(p->jit_fn.size()) && p->jit_fn[S_sw - 1];
-  // partials: per pair and last-sweep tile (fused), else per pair and chunk
-  const int64_t n_chunks = !pair_out ? 0
-                           : fused   ? p->dev_sweeps[size_t(S_sw - 1)].n_tiles
-                                     : ((int64_t(1) << p->n) + kInnerChunk - 1) / kInnerChunk;
+  bool fused;
+  const int64_t n_chunks = pair_chunks(ctx, p, pair_out && parts.empty(), fused);
   const size_t pov_off = al(src_off + srcs.size() * sizeof(void *));
   const size_t total = pov_off + size_t(n_pairs * n_chunks) * sizeof(double2);
   int rc = ws_reserve(ctx, total, st);
@@ -3170,46 +3258,60 @@ static int run_instances(pqs_ctx *ctx, pqs_plan *p, std::vector<InstDev> &h, con
   }
   rc = upload(ctx, ws + tab_off, blob.data(), blob.size(), st);
   if (rc) return rc;
-  const InstDev *d_tab = (const InstDev *)(ws + tab_off);
-  double2 *pov = (double2 *)(ws + pov_off);
-  for (int s = 0; s < S_sw; ++s) {
-    if (fused && s == S_sw - 1) {
-      if (n_pairs == 0) break;
-      const DevSweep &sw = p->dev_sweeps[size_t(s)];
-      const int nthr = (1 << sw.k) >> pqs::kRegBits;
-      const int64_t grid = n_pairs * sw.n_tiles;
-      if (grid > 0x7fffffff) return fail(PQS_ERR_UNSUPPORTED, "grid too large: split the batch");
-      long long na = (long long)h.size();
-      void *args[] = {(void *)&d_tab, (void *)&na, (void *)&init_tab, (void *)&pov};
-      HIPCHECK(hipModuleLaunchKernel((hipFunction_t)p->jit_pair_fn, unsigned(grid), 1, 1, unsigned(nthr), 1, 1, 0,
-                                     st, args, nullptr));
-      break;
-    }
-    rc = launch_sweep(ctx, p, s, d_tab, int64_t(h.size()), init_tab, st);
+  // (a strided batch where overlaps are wanted: pair i at h[2i].state)
+  const int64_t stride =
+      pair_out && n_main > 1 ? int64_t(((const char *)h[1].state - (const char *)h[0].state) / ptrdiff_t(amp_bytes(p->dtype)))
+                             : 0;
+  rc = launch_sweeps(ctx, p, (const InstDev *)(ws + tab_off), int64_t(h.size()), int64_t(n_main), h[0].state, stride,
+                     init_tab, st, fused, n_chunks, (double2 *)(ws + pov_off), pair_out);
+  if (rc) return rc;
+  return launch_add_rows(p, (const AccRow *)(ws + acc_off), (const void *const *)(ws + src_off), int64_t(acc.size()),
+                         st);
+}
+
+// pqs_run_batch and pqs_run_batch_pairs.  A plain batch (no tangents, input not
+// among its own rows) has a table that follows from its strides: a kernel
+// writes it, with no list to build and copy, from the size on where the list
+// would no longer travel as a launch's argument (2000 8-qubit states: 158 ->
+// 150 us; below that the two are one launch each).
+static int run_strided(pqs_ctx *ctx, pqs_plan *p, void *states, int64_t state_stride, int64_t batch,
+                       const double *params, int64_t param_stride, const int32_t *tangents, int32_t init,
+                       const void *src, const void *init_tab, hipStream_t st, double *pair_out) {
+  const size_t ab = amp_bytes(p->dtype), row = size_t(state_stride) * ab;
+  const char *lo = (const char *)states, *hi = lo + size_t(batch) * row;
+  const bool own_input = init == 0 && (!src || ((const char *)src >= lo && (const char *)src < hi));
+  if (!tangents && !own_input && size_t(batch) * sizeof(InstDev) > kArgUpload) {
+    const size_t sb = (size_t(1) << p->n) * ab;
+    auto al = [](size_t x) { return (x + 255) & ~size_t(255); };
+    const size_t tab_off = al(p->rolling ? size_t(batch) * sb : 0);
+    const size_t pov_off = al(tab_off + size_t(batch) * sizeof(InstDev));
+    bool fused;
+    const int64_t n_chunks = pair_chunks(ctx, p, pair_out != nullptr, fused);
+    int rc = ws_reserve(ctx, pov_off + size_t(batch / 2 * n_chunks) * sizeof(double2), st);
     if (rc) return rc;
-  }
-  rc = launch_add_rows(p, (const AccRow *)(ws + acc_off), (const void *const *)(ws + src_off),
-                       int64_t(acc.size()), st);
-  if (rc || !pair_out || n_pairs == 0) return rc;
-  if (!fused) {
-    // overlaps read back from the states: instance i's state is h[i].state
-    // (a strided batch: pair i at h[2i].state, stride h[1].state - h[0].state)
-    const int64_t dim = int64_t(1) << p->n;
-    const size_t ab = amp_bytes(p->dtype);
-    const int64_t stride = int64_t(((const char *)h[1].state - (const char *)h[0].state) / ptrdiff_t(ab));
-    const int64_t grid = n_pairs * n_chunks;
-    if (grid > 0x7fffffff) return fail(PQS_ERR_UNSUPPORTED, "too many pairs x chunks");
-    if (p->dtype == PQS_C128)
-      hipLaunchKernelGGL(k_pair_partial<double>, dim3(unsigned(grid)), dim3(RB), 0, st, (const double2 *)h[0].state,
-                         stride, dim, n_chunks, pov);
-    else
-      hipLaunchKernelGGL(k_pair_partial<float>, dim3(unsigned(grid)), dim3(RB), 0, st, (const float2 *)h[0].state,
-                         stride, dim, n_chunks, pov);
+    char *ws = (char *)ctx->ws;
+    InstDev *tab = (InstDev *)(ws + tab_off);
+    hipLaunchKernelGGL(k_fill_batch_table, dim3(grid_for(batch, 256)), dim3(256), 0, st, tab, (char *)states,
+                       int64_t(row), batch, params, param_stride, init, src, ws, int64_t(sb), p->rolling ? 1 : 0);
     HIPCHECK(hipGetLastError());
+    return launch_sweeps(ctx, p, tab, batch, batch, states, state_stride, init_tab, st, fused, n_chunks,
+                         (double2 *)(ws + pov_off), pair_out);
   }
-  hipLaunchKernelGGL(k_sum_rows, dim3(unsigned(n_pairs)), dim3(RB), 0, st, pov, n_chunks, (double2 *)pair_out);
-  HIPCHECK(hipGetLastError());
-  return PQS_OK;
+  std::vector<InstDev> h((size_t)batch);
+  for (int64_t i = 0; i < batch; ++i) {
+    InstDev &d = h[(size_t)i];
+    d.state = (char *)states + size_t(i) * row;
+    d.src = src;
+    d.params = params ? params + i * param_stride : nullptr;
+    d.alt = nullptr;
+    d.tangent = tangents ? tangents[i] : -1;
+    if (d.tangent >= p->n_tangents) return fail(PQS_ERR_ARG, "tangent index beyond the plan's tangents");
+    if (d.tangent < 0) d.tangent = -1;
+    d.init = init;
+    d.start_sweep = 0;
+    d.pingpong = 0;
+  }
+  return run_instances(ctx, p, h, init_tab, st, pair_out);
 }
 
 int pqs_run(pqs_ctx *ctx, pqs_plan *p, const pqs_instance *insts, int64_t n_inst, const void *init_tab,
@@ -3255,24 +3357,13 @@ int pqs_run_batch(pqs_ctx *ctx, pqs_plan *p, void *states, int64_t state_stride,
   if (init == 2 && !init_tab) return fail(PQS_ERR_ARG, "product init needs an init table");
   DeviceGuard g(ctx->device);
   hipStream_t st = (hipStream_t)stream;
-  const size_t ab = amp_bytes(p->dtype);
-  std::vector<InstDev> h((size_t)batch);
-  for (int64_t i = 0; i < batch; ++i) {
-    InstDev &d = h[(size_t)i];
-    d.state = (char *)states + size_t(i) * size_t(state_stride) * ab;
-    d.src = src;
-    d.params = params ? params + i * param_stride : nullptr;
-    d.alt = nullptr;
-    d.tangent = tangents ? tangents[i] : -1;
-    if (d.tangent >= p->n_tangents) return fail(PQS_ERR_ARG, "tangent index beyond the plan's tangents");
-    if (d.tangent < 0) d.tangent = -1;
-    d.init = init;
-    d.start_sweep = 0;
-    d.pingpong = 0;
-  }
-  int rc = plan_upload(ctx, p, st);
+  if (tangents)
+    for (int64_t i = 0; i < batch; ++i)
+      if (tangents[i] >= p->n_tangents) return fail(PQS_ERR_ARG, "tangent index beyond the plan's tangents");
+  const int rc = plan_upload(ctx, p, st);
   if (rc) return rc;
-  return run_instances(ctx, p, h, init_tab, st);
+  return run_strided(ctx, p, states, state_stride, batch, params, param_stride, tangents, init, src, init_tab, st,
+                     nullptr);
 }
 
 int pqs_run_batch_pairs(pqs_ctx *ctx, pqs_plan *p, void *states, int64_t state_stride, int64_t batch,
@@ -3287,22 +3378,10 @@ int pqs_run_batch_pairs(pqs_ctx *ctx, pqs_plan *p, void *states, int64_t state_s
   if (init == 2 && !init_tab) return fail(PQS_ERR_ARG, "product init needs an init table");
   DeviceGuard g(ctx->device);
   hipStream_t st = (hipStream_t)stream;
-  const size_t ab = amp_bytes(p->dtype);
-  std::vector<InstDev> h((size_t)batch);
-  for (int64_t i = 0; i < batch; ++i) {
-    InstDev &d = h[(size_t)i];
-    d.state = (char *)states + size_t(i) * size_t(state_stride) * ab;
-    d.src = src;
-    d.params = params ? params + i * param_stride : nullptr;
-    d.alt = nullptr;
-    d.tangent = -1;
-    d.init = init;
-    d.start_sweep = 0;
-    d.pingpong = 0;
-  }
-  int rc = plan_upload(ctx, p, st);
+  const int rc = plan_upload(ctx, p, st);
   if (rc) return rc;
-  return run_instances(ctx, p, h, init_tab, st, overlaps);
+  return run_strided(ctx, p, states, state_stride, batch, params, param_stride, nullptr, init, src, init_tab, st,
+                     overlaps);
 }
 
 int pqs_run_multi(pqs_ctx *ctx, pqs_plan *const *plans, int32_t n_plans, const pqs_instance *insts,
@@ -3550,7 +3629,7 @@ int pqs_run_batch_noalloc(pqs_ctx *ctx, pqs_plan *p, void *states, int64_t state
   InstDev *tab = static_cast<InstDev *>(ctx->scratch);
   const int64_t sbytes = state_stride * int64_t(amp_bytes(p->dtype));
   hipLaunchKernelGGL(k_fill_batch_table, dim3(grid_for(batch, 256)), dim3(256), 0, st, tab, (char *)states, sbytes,
-                     batch, params, param_stride, init, src, (char *)alt, p->rolling ? 1 : 0);
+                     batch, params, param_stride, init, src, (char *)alt, sbytes, p->rolling ? 1 : 0);
   HIPCHECK(hipGetLastError());
   for (int s = 0; s < int(p->dev_sweeps.size()); ++s) {
     const int rc = launch_sweep(ctx, p, s, tab, batch, init_tab, st);

@@ -119,3 +119,73 @@ def test_plan_first_launched_on_another_stream(E):
         want = OS.run(og, th, n)
         for out in (out_a, out_b, out_b2):
             assert infidelity(out.cpu().numpy().ravel(), want) < 1e-12, jit
+
+
+@pytest.mark.parametrize("off", [0, 8, 3])
+def test_upload_sizes_at_the_path_edges(E, off):
+    """Largest argument upload (2048 bytes), the smallest staged one, and the
+    edges of the staged pieces (512 KB): every byte, and none beyond."""
+    from pyramaterised_amd import _lib as L
+    lib = L.lib()
+    rng = np.random.default_rng(7)
+    piece = 512 << 10
+    buf = torch.zeros(3 * piece, dtype=torch.uint8, device="cuda")
+    ctx = E.context().handle
+    for nb in (15, 16, 2032, 2047, 2048, 2049, 2064, piece - 16, piece, piece + 1, piece + 16, 2 * piece + 48):
+        src = rng.integers(1, 256, nb, dtype=np.uint8)
+        buf.zero_()
+        E.check(lib.pqs_upload(ctx, C.c_void_p(buf.data_ptr() + off), C.c_void_p(src.ctypes.data), nb,
+                               E.stream_ptr()))
+        want = src.copy()
+        src.fill(0)  # the caller reuses its array at once
+        got = buf.cpu().numpy()
+        assert np.array_equal(got[off:off + nb], want), (off, nb)
+        assert not got[:off].any() and not got[off + nb:].any(), (off, nb)
+
+
+@pytest.mark.parametrize("rolling", [False, True])
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+def test_device_written_batch_tables(E, dtype, rolling):
+    """Batches whose instance table a kernel writes (beyond 2048 bytes: 43
+    instances) equal the same rows run alone, bit for bit: every initial
+    state, shared parameters, padded rows, rows evolved in place
+    (their input inside the batch's own rows), and pairs."""
+    import pyramaterised_amd as pyqc
+    from pyramaterised_amd import templates as T
+    from pyramaterised_amd import _lib as L
+    lib = L.lib()
+    n, B = 7, 60
+    rng = np.random.default_rng(11)
+    qc = pyqc.PQC(n)
+    for layer in T.clifford_HE_layers(3, n):
+        qc.add_layer(layer)
+    plan = E.Plan(n, qc.ops(), dtype=dtype, tile_bits=5, low_bits=2, flags=L.PQS_PLAN_ROLLING if rolling else 0)
+    P, dim, cdt = qc.n_true_params, 1 << n, E.CDTYPE[plan.dtype]
+    th = rng.random((B, P)) * 2 * np.pi
+    vec = rng.normal(size=dim) + 1j * rng.normal(size=dim)
+    vec /= np.linalg.norm(vec)
+    prod = [v / np.linalg.norm(v) for v in rng.normal(size=(n, 2)) + 1j * rng.normal(size=(n, 2))]
+    for init in (E.Init.zero(), E.Init.product(prod), E.Init.from_vector(vec)):
+        got = E.run(plan, th, init)
+        for b in (0, 1, 41, 42, B - 1):
+            assert torch.equal(got[b], E.run(plan, th[b], init)[0]), (init.kind, b)
+    rows = torch.as_tensor(rng.normal(size=(B, dim)) + 1j * rng.normal(size=(B, dim))).to(cdt).cuda()
+    want = [E.run_rows(plan, th[b], rows[b:b + 1].clone())[0] for b in range(B)]
+    got = E.run_rows(plan, th, rows.clone())
+    assert all(torch.equal(got[b], want[b]) for b in range(B))
+    # one shared parameter vector, rows 2^n + 5 amplitudes apart, from |0..0>
+    p = E.to_device(th[3])
+    pad = torch.full((B, dim + 5), 7.0, dtype=cdt, device="cuda")
+    E.check(lib.pqs_run_batch(E.context().handle, plan.handle, E.ptr(pad), dim + 5, B, E.ptr(p), 0, None, 1, None,
+                              None, E.stream_ptr()))
+    one = E.run(plan, th[3], E.Init.zero())[0]
+    assert all(torch.equal(pad[b, :dim], one) for b in range(B)) and bool((pad[:, dim:] == 7.0).all())
+    # pairs of the padded rows
+    ov = torch.zeros(B // 2, dtype=torch.complex128, device="cuda")
+    pt = E.to_device(th)
+    E.check(lib.pqs_run_batch_pairs(E.context().handle, plan.handle, E.ptr(pad), dim + 5, B, E.ptr(pt), P, 1,
+                                    None, None, E.ptr(ov), E.stream_ptr()))
+    st = E.run(plan, th, E.Init.zero()).to(torch.complex128).cpu()
+    ref = (st[0:B:2].conj() * st[1:B:2]).sum(1)
+    # 2^7 products of unit vectors: 128 roundings of at most 2^-53 each
+    assert float((ov.cpu() - ref).abs().max()) < 128 * 2.0 ** -53
