@@ -141,6 +141,14 @@ __device__ __forceinline__ double op_angle(const DevOp *op, const double *params
   return a;
 }
 
+// (sin, cos) of half a rotation's angle for the instance of the tangent that
+// it carries: those of the angle plus pi (kNoShift); the caller scales by s/2.
+__device__ __forceinline__ void half_turn(double &s, double &c) {
+  const double t = s;
+  s = c;
+  c = -t;
+}
+
 // 2x2 complex matrix in double: m[0..3] = m00 m01 m10 m11
 struct M2 {
   double2 m[4];
@@ -820,6 +828,8 @@ __device__ __forceinline__ void sweep_reg_body(const DevSweep &sw, const DevOp *
     if (d->coef >= 0) {
       double sn, cs;
       sincos(0.5 * op_angle(d, params), &sn, &cs);
+      const bool turned = d->shift == in.tangent;
+      if (turned) half_turn(sn, cs);
       if (fabs(cs) >= fabs(sn)) {
         r.t = sn / cs;
         r.f = cs;
@@ -828,6 +838,7 @@ __device__ __forceinline__ void sweep_reg_body(const DevSweep &sw, const DevOp *
         r.f = sn;
         r.regs |= 1 << 16;
       }
+      if (turned) r.f *= 0.5 * d->scale;
     }
     rops[o - sw.op_begin] = r;
   }
@@ -1249,15 +1260,18 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
 
   // parameters of the next refill, loaded ahead
   double praw[NANG], pscale[NANG], poff[NANG];
+  int pshift[NANG];
   auto ahead = [&](int a0) {
 #pragma unroll
     for (int m = 0; m < NANG; ++m) {
       const int i = a0 + l + m * T;
       praw[m] = pscale[m] = poff[m] = 0.0;
+      pshift[m] = pqs::kNoShift;
       if (live && i < n_angles) {
         const pqs::WaveAngle &w = angles[i];
         pscale[m] = w.scale;
         poff[m] = w.offset;
+        pshift[m] = w.shift;
         if (w.slot >= 0) praw[m] = params[w.slot];
       }
     }
@@ -1412,8 +1426,13 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
         if (m * T < int(x)) {
           double sn, cs;
           sincos(0.5 * (poff[m] + pscale[m] * praw[m]), &sn, &cs);
+          double f = 1.0;
+          if (pshift[m] == in.tangent) {
+            half_turn(sn, cs);
+            f = 0.5 * pscale[m];
+          }
           if (fabs(cs) < cmin) cs = cs < 0.0 ? -cmin : cmin;
-          mine_tab[l + m * T] = double2{sn / cs, cs};
+          mine_tab[l + m * T] = double2{sn / cs, f * cs};
         }
       }
       wave_fence();

@@ -345,9 +345,11 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
     struct Angle {
       int slot;
       double scale, offset;
+      int shift;
     };
     std::vector<int> ang(ds.op_end - ds.op_begin, -1);
     std::vector<Angle> aops;
+    bool shifts = false;  // rotations that carry their derivatives
     auto is_rot = [](int kd) {
       return kd == PQS_OP_RX || kd == PQS_OP_RY || kd == PQS_OP_RZ || kd == PQS_OP_RZZ || kd == PQS_OP_RXX ||
              kd == PQS_OP_RYY;
@@ -356,11 +358,12 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
       const DevOp &d = p.dev_ops[i];
       if (is_rot(d.kind)) {
         ang[i - ds.op_begin] = int(aops.size());
-        aops.push_back({d.slot, d.scale, d.offset});
+        aops.push_back({d.slot, d.scale, d.offset, d.shift});
+        if (d.shift >= 0) shifts = true;
       } else if (d.kind == PQS_OP_FSIM || d.kind == PQS_OP_GEN_FSIM) {
         ang[i - ds.op_begin] = int(aops.size());
-        aops.push_back({d.slot, 2 * d.scale, 2 * d.offset});
-        if (d.slot2 >= 0) aops.push_back({d.slot2, 2.0, 0.0});
+        aops.push_back({d.slot, 2 * d.scale, 2 * d.offset, kNoShift});
+        if (d.slot2 >= 0) aops.push_back({d.slot2, 2.0, 0.0, kNoShift});
       }
     }
     const int na = int(aops.size());
@@ -388,6 +391,11 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
       o << "};\n__device__ const double OF" << s << "[" << na << "] = {";
       for (int a = 0; a < na; ++a) o << (a ? "," : "") << dbl(aops[a].offset);
       o << "};\n";
+      if (shifts) {
+        o << "__device__ const int SH" << s << "[" << na << "] = {";
+        for (int a = 0; a < na; ++a) o << (a ? "," : "") << aops[a].shift;
+        o << "};\n";
+      }
     }
     const bool persist = (p.flags & PQS_PLAN_JIT_PERSISTENT) != 0;
     // The last sweep of a plan also comes as a pair kernel (pqs_jit_pair_<s>)
@@ -538,9 +546,15 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
       o << "    double sn, cs;\n";
       o << "    const int sl = SL" << s << "[i];\n";
       o << "    sincos(0.5 * (OF" << s << "[i] + (sl >= 0 ? SC" << s << "[i] * params[sl] : 0.0)), &sn, &cs);\n";
+      if (shifts) {
+        // the derivative's instance: the angle plus pi, and half its scale
+        o << "    double f = 1.0;\n";
+        o << "    if (SH" << s << "[i] == in.tangent) { const double u = sn; sn = cs; cs = -u; f = 0.5 * SC" << s
+          << "[i]; }\n";
+      }
       o << "    if (fabs(cs) < " << dbl(cos_min(p)) << ") cs = cs < 0.0 ? -" << dbl(cos_min(p)) << " : "
         << dbl(cos_min(p)) << ";\n";
-      o << "    tf[i] = double2{sn / cs, cs};\n  }\n";
+      o << "    tf[i] = double2{sn / cs, " << (shifts ? "f * cs" : "cs") << "};\n  }\n";
     }
     o << "  __syncthreads();\n";
     // fs: the accumulated scale of the rotations (uniform over the block

@@ -131,11 +131,12 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
     refill_first = n_ang;
     emit(kWRefill).c = n_ang;
   };
-  auto angle = [&](double scale, double offset, int slot) {
+  auto angle = [&](double scale, double offset, int slot, int shift) {
     WaveAngle w{};
     w.scale = scale;
     w.offset = offset;
     w.slot = slot;
+    w.shift = shift;
     p.dev_angles.push_back(w);
     ++n_ang;
     p.dev_wave[size_t(refill_at)].x = uint32_t(n_ang - refill_first);
@@ -175,7 +176,7 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
     auto rotation = [&](uint32_t x, uint32_t z, uint64_t zg, int y) {
       rotations(1);
       reserve(1);
-      const uint16_t a = angle(d.scale, d.offset, d.slot);
+      const uint16_t a = angle(d.scale, d.offset, d.slot, d.shift);
       WaveOp &w = emit(!x ? kWPhase : y & 1 ? kWRotR : kWRotI);
       w.ang = a;
       w.x = x;
@@ -217,8 +218,8 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
       case PQS_OP_GEN_FSIM: {
         reserve(2);
         // doubled: the table holds (tan, cos) of half of each angle
-        const uint16_t a = angle(2 * d.scale, 2 * d.offset, d.slot);
-        const uint32_t f = d.slot2 >= 0 ? angle(2.0, 0.0, d.slot2) : 0xffffffffu;
+        const uint16_t a = angle(2 * d.scale, 2 * d.offset, d.slot, kNoShift);
+        const uint32_t f = d.slot2 >= 0 ? angle(2.0, 0.0, d.slot2, kNoShift) : 0xffffffffu;
         WaveOp &w = d.kind == PQS_OP_FSIM ? emit(kWFsim) : generator(kWGenFsim, d.tangent);
         w.ang = a;
         w.x = b0 | b1;
@@ -316,10 +317,10 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
         for (int o : got) {
           const DevOp &d = p.dev_ops[size_t(o)];
           if (d.t0 != t) continue;
-          a = angle(d.scale, d.offset, d.slot);
+          a = angle(d.scale, d.offset, d.slot, d.shift);
           found = true;
         }
-        if (!found) a = angle(0.0, 0.0, -1);
+        if (!found) a = angle(0.0, 0.0, -1, kNoShift);
         if (first < 0) first = a;
       }
       WaveOp &w = emit(kind == PQS_OP_RX ? kWLayerRx : kind == PQS_OP_RY ? kWLayerRy : kWLayerRz);
@@ -422,6 +423,25 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
     p.tangent_parent.push_back(t);
     return p.n_sub++;
   };
+  // the generator right after a rotation, alone in its run, that is exactly
+  // the rotation's derivative (kNoShift)
+  auto derivative_of = [&](int i) {
+    if (p.dtype != PQS_C128 || i + 1 >= n_ops) return false;
+    const pqs_op &r = ops[i], &g = ops[i + 1];
+    int pauli;
+    switch (r.kind) {
+      case PQS_OP_RX: case PQS_OP_RXX: pauli = 1; break;
+      case PQS_OP_RY: case PQS_OP_RYY: pauli = 2; break;
+      case PQS_OP_RZ: case PQS_OP_RZZ: pauli = 3; break;
+      default: return false;
+    }
+    if (g.kind != PQS_OP_GEN || g.pauli != pauli) return false;
+    if (i + 2 < n_ops && ops[i + 2].kind == PQS_OP_GEN && ops[i + 2].tangent == g.tangent) return false;
+    if (is_two_qubit(r.kind) ? !((g.q0 == r.q0 && g.q1 == r.q1) || (g.q0 == r.q1 && g.q1 == r.q0))
+                             : !(g.q0 == r.q0 && g.q1 < 0))
+      return false;
+    return r.scale != 0.0 && g.m[0] == 0.0 && g.m[1] == -0.5 * r.scale;
+  };
   for (int i = 0; i < n_ops;) {
     ExecOp e;
     e.first = i;
@@ -483,6 +503,11 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
       e.kind = ops[i].kind;
       if (e.kind == PQS_OP_MEAS) e.need = bitq(0);
       if (e.kind == PQS_OP_GEN_FSIM) e.tangent = part_tangent(ops[i].tangent, true);
+      if (derivative_of(i)) {
+        e.shift = part_tangent(ops[i + 1].tangent, true);
+        e.n_src = 2;
+        ++i;
+      }
       ++i;
     }
     if (popc(e.active) > k) {
@@ -725,7 +750,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
   p.tangent_sweep.assign(p.n_sub, -1);
   for (size_t s = 0; s < p.sweeps.size(); ++s)
     for (int ei : p.sweeps[s].ops) {
-      const int tg = p.exec[ei].tangent;
+      const int tg = p.exec[ei].shift >= 0 ? p.exec[ei].shift : p.exec[ei].tangent;
       if (tg >= 0 && p.tangent_sweep[tg] < 0) p.tangent_sweep[tg] = int(s);
     }
 
@@ -1259,6 +1284,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
         DevOp d{};
         d.kind = e.kind == kPauliSum ? ((p.reg_exec && !ph.lds) ? kGen1 : kPauliSum) : so.kind;
         d.tangent = e.tangent;
+        d.shift = e.shift;
         d.slot = so.slot;
         d.slot2 = so.slot2;
         d.pauli = so.pauli;
@@ -1412,9 +1438,17 @@ int pqs_plan_sweep(const pqs_plan *p, int32_t s, int32_t *tile_qubits, int32_t *
   if (n_tile) *n_tile = int32_t(sw.tile_qubits.size());
   if (tile_qubits)
     for (size_t i = 0; i < sw.tile_qubits.size(); ++i) tile_qubits[i] = sw.tile_qubits[i];
-  if (n_op) *n_op = int32_t(sw.ops.size());
-  if (op_index)
-    for (size_t i = 0; i < sw.ops.size(); ++i) op_index[i] = p->exec[sw.ops[i]].first;
+  int32_t n = 0;
+  for (int ei : sw.ops) {
+    const pqs::ExecOp &e = p->exec[size_t(ei)];
+    if (op_index) op_index[n] = e.first;
+    ++n;
+    if (e.shift >= 0) {  // a rotation and its generator
+      if (op_index) op_index[n] = e.first + 1;
+      ++n;
+    }
+  }
+  if (n_op) *n_op = n;
   return PQS_OK;
 }
 

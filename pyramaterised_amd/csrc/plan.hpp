@@ -16,6 +16,16 @@ constexpr int kMaxTileBits = 14; // 2^14 complex64 = 128 KiB of LDS
 // A 64-bit qubit mask: bit q set <=> qubit q.
 using qmask = uint64_t;
 
+// A rotation's derivative is the rotation itself, turned by pi more:
+// -i s/2 P exp(-i a/2 P) = s/2 exp(-i (a + pi)/2 P), a = s p + offset.  Where a
+// rotation's own generator follows it (complex128), the pair is one op: the
+// instance of that tangent reads (-sin, cos) for (cos, sin) of half the angle
+// and scales by s/2, and the sweep has no generator ops to place, to step over
+// in every other instance and to order the gates around (16 qubits, 20 HEA
+// layers, 640 parameters: the Jacobian 3.4 -> 2.0 ms).  complex64 plans keep the generators:
+// their rounding is part of double results made from their states.
+constexpr int kNoShift = -2;
+
 // One executable op after generator-term merging.
 struct ExecOp {
   int kind = 0;          // pqs_op_kind, or kPauliSum for a merged PQS_OP_GEN
@@ -25,6 +35,7 @@ struct ExecOp {
   qmask diag = 0;        // qubits the op acts on diagonally (block-diagonal)
   int tangent = -1;      // derivative ops: tangent (or sub-tangent) index
   qmask need = 0;        // further qubits held in the tile and in registers
+  int shift = kNoShift;  // rotations: (sub-)tangent whose derivative is this rotation by pi more
 };
 constexpr int kPauliSum = 100;
 // A one-term, one-qubit generator (coef * Pauli on q0, applied only by the
@@ -46,6 +57,7 @@ struct alignas(16) DevOp {
   int32_t term0, nterms;
   int32_t pauli, coef;  // coef: index of (cos, sin) in the sweep's table, -1 none
   int32_t r0, r1;       // register index of q0 / q1 in the op's phase, -1 if not
+  int32_t shift;        // rotations: tangent whose derivative it carries, or kNoShift
   double scale, offset;
   double m[32];
 };
@@ -147,7 +159,7 @@ struct alignas(16) WaveOp {
 };
 struct alignas(8) WaveAngle {  // the rotation's angle: scale * params[slot] + offset
   double scale, offset;
-  int32_t slot, pad;
+  int32_t slot, shift;  // shift: as in DevOp
 };
 
 std::string plan_error(); // last planner error (thread local)
