@@ -149,137 +149,125 @@ __device__ __forceinline__ void half_turn(double &s, double &c) {
   c = -t;
 }
 
-// 2x2 complex matrix in double: m[0..3] = m00 m01 m10 m11
-struct M2 {
-  double2 m[4];
-};
-struct M4 {
-  double2 m[16];
-};
-
-__device__ void mat1_of(const DevOp *op, const double *params, M2 &M) {
-  const int kind = op->kind;
-  if (kind == PQS_OP_MAT1) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) M.m[i] = double2{op->m[2 * i], op->m[2 * i + 1]};
-    return;
-  }
-  double s, c;
-  sincos(0.5 * op_angle(op, params), &s, &c);
-  if (kind == PQS_OP_RX) {
-    M.m[0] = double2{c, 0};
-    M.m[1] = double2{0, -s};
-    M.m[2] = double2{0, -s};
-    M.m[3] = double2{c, 0};
-  } else if (kind == PQS_OP_RY) {
-    M.m[0] = double2{c, 0};
-    M.m[1] = double2{-s, 0};
-    M.m[2] = double2{s, 0};
-    M.m[3] = double2{c, 0};
-  } else {  // RZ
-    M.m[0] = double2{c, -s};
-    M.m[1] = double2{0, 0};
-    M.m[2] = double2{0, 0};
-    M.m[3] = double2{c, s};
-  }
-}
-
-__device__ void mat2_of(const DevOp *op, const double *params, M4 &M) {
-  const int kind = op->kind;
-  if (kind == PQS_OP_MAT2) {
-#pragma unroll
-    for (int i = 0; i < 16; ++i) M.m[i] = double2{op->m[2 * i], op->m[2 * i + 1]};
-    return;
-  }
-#pragma unroll
-  for (int i = 0; i < 16; ++i) M.m[i] = double2{0, 0};
-  if (kind == PQS_OP_RXX || kind == PQS_OP_RYY) {
-    double s, c;
-    sincos(0.5 * op_angle(op, params), &s, &c);
-    for (int r = 0; r < 4; ++r) M.m[5 * r] = double2{c, 0};
-    // X(x)X: 00<->11, 01<->10 with +1; Y(x)Y: 00<->11 with -1, 01<->10 with +1
-    double sa = kind == PQS_OP_RXX ? 1.0 : -1.0;
-    M.m[3] = double2{0, -s * sa};
-    M.m[12] = double2{0, -s * sa};
-    M.m[6] = double2{0, -s};
-    M.m[9] = double2{0, -s};
-    return;
-  }
-  // fSim family (gates.py:598-606, 619-627, 640-648, 708-716, 729-737)
-  double th = op_angle(op, params);
-  double ph = op->slot2 >= 0 ? params[op->slot2] : 0.0;
-  double st, ct, sp, cp;
-  sincos(th, &st, &ct);
-  sincos(ph, &sp, &cp);
-  M.m[0] = double2{1, 0};
-  int sel = kind == PQS_OP_FSIM ? 0 : op->pauli;
-  if (sel == 1 || sel == 3) {  // d_theta as written by the reference
-    M.m[5] = double2{-st, 0};
-    M.m[6] = double2{0, -ct};
-    M.m[9] = double2{0, -ct};
-    M.m[10] = double2{-st, 0};
-  } else {
-    M.m[5] = double2{ct, 0};
-    M.m[6] = double2{0, -st};
-    M.m[9] = double2{0, -st};
-    M.m[10] = double2{ct, 0};
-  }
-  if (sel == 3) {
-    M.m[15] = double2{1, 0};
-  } else if (sel == 2) {  // -i e^{-i phi}
-    M.m[15] = double2{-sp, -cp};
-  } else {  // e^{-i phi}
-    M.m[15] = double2{cp, -sp};
-  }
-}
-
+// What an op's angles come to: cos and sin of half a rotation's angle, or of
+// fSim's theta and phi.  Computed once per block and op, in double, and
+// rounded to the state's precision.
 template <typename R>
-__device__ __forceinline__ typename CT<R>::V cvt(double2 a) {
-  return typename CT<R>::V{R(a.x), R(a.y)};
+struct LdsCoef {
+  R c, s, cp, sp;
+};
+template <typename R>
+__device__ __forceinline__ LdsCoef<R> lds_coef(const DevOp *op, const double *params) {
+  double s = 0.0, c = 1.0, sp = 0.0, cp = 1.0;
+  switch (op->kind) {
+    case PQS_OP_RX: case PQS_OP_RY: case PQS_OP_RZ: case PQS_OP_RXX: case PQS_OP_RYY: case PQS_OP_RZZ:
+      sincos(0.5 * op_angle(op, params), &s, &c);
+      break;
+    case PQS_OP_FSIM: case PQS_OP_GEN_FSIM:
+      sincos(op_angle(op, params), &s, &c);
+      sincos(op->slot2 >= 0 ? params[op->slot2] : 0.0, &sp, &cp);
+      break;
+    default: break;
+  }
+  return LdsCoef<R>{R(c), R(s), R(cp), R(sp)};
+}
+// x a + y b and x a - y b with every product and sum rounded by itself: what
+// the products of a matrix with real or imaginary entries come to.
+template <typename R>
+__device__ __forceinline__ R mul_add(R x, R a, R y, R b) {
+#pragma clang fp contract(off)
+  return x * a + y * b;
+}
+// m a, with the rounding written out: results in single precision stay what
+// they are whatever the compiler would fuse.
+template <typename V>
+__device__ __forceinline__ V cmul_at(V m, V a) {
+  return V{fma(a.x, m.x, -(a.y * m.y)), fma(a.x, m.y, a.y * m.x)};
 }
 
 __device__ __forceinline__ int swz(int j) { return j ^ (((j >> 4) ^ (j >> 8) ^ (j >> 12)) & 15); }
 
+// One op on a tile in LDS.  Rotations and fSim act through the entries of
+// their matrices that are not zero.
 template <typename R, int MAXPER, bool SWZ>
-__device__ __forceinline__ void apply_lds_op(typename CT<R>::V *tile, const int S, const DevOp *op,
-                                             const uint64_t base, const double *params,
+__device__ __forceinline__ void apply_lds_op(typename CT<R>::V *tile, const int S, const DevOp *op, const int kind,
+                                             const int t0, const int t1, const LdsCoef<R> cf, const uint64_t base,
                                              const DevTerm *terms, const int tid, const int nthr) {
   using V = typename CT<R>::V;
-  const int kind = op->kind;
-  const int t0 = op->t0, t1 = op->t1;
   auto IX = [](int j) { return SWZ ? swz(j) : j; };
+  const R c = cf.c, s = cf.s;
+  auto pairs = [&](auto f) {  // f on both amplitudes of every pair over q0's bit
+    for (int u = tid; u < (S >> 1); u += nthr) {
+      const int j0 = ins0(u, t0), j1 = j0 | (1 << t0);
+      V a = tile[IX(j0)], b = tile[IX(j1)];
+      f(a, b);
+      tile[IX(j0)] = a;
+      tile[IX(j1)] = b;
+    }
+  };
+  auto quads = [&](auto f) {  // f on the four amplitudes over the bits of q0 (high) and q1
+    const int lo = t0 < t1 ? t0 : t1, hi = t0 < t1 ? t1 : t0;
+    for (int u = tid; u < (S >> 2); u += nthr) {
+      const int j = ins0(ins0(u, lo), hi);
+      const int jj[4] = {j, j | (1 << t1), j | (1 << t0), j | (1 << t0) | (1 << t1)};
+      V a[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) a[i] = tile[IX(jj[i])];
+      f(a);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) tile[IX(jj[i])] = a[i];
+    }
+  };
+  // (a, b) <- x (a, b) - i y (b, a)
+  auto mix_i = [](V &a, V &b, R x, R y) {
+    const V p = a, q = b;
+    a = V{mul_add(x, p.x, y, q.y), mul_add(x, p.y, -y, q.x)};
+    b = V{mul_add(x, q.x, y, p.y), mul_add(x, q.y, -y, p.x)};
+  };
   switch (kind) {
-      case PQS_OP_MAT1:
-      case PQS_OP_RX:
+      case PQS_OP_RX: pairs([&](V &a, V &b) { mix_i(a, b, c, s); }); break;
       case PQS_OP_RY:
+        pairs([&](V &a, V &b) {
+          const V p = a, q = b;
+          a = V{mul_add(c, p.x, -s, q.x), mul_add(c, p.y, -s, q.y)};
+          b = V{mul_add(s, p.x, c, q.x), mul_add(s, p.y, c, q.y)};
+        });
+        break;
       case PQS_OP_RZ: {
-        M2 M;
-        mat1_of(op, params, M);
+        const V d0 = V{c, -s}, d1 = V{c, s};
+        const int c0 = t0 < 0 ? int((base >> op->g0) & 1) : -1;
+        for (int j = tid; j < S; j += nthr) {
+          const int b0 = c0 >= 0 ? c0 : ((j >> t0) & 1);
+          tile[IX(j)] = cmul_at(b0 ? d1 : d0, tile[IX(j)]);
+        }
+        break;
+      }
+      case PQS_OP_MAT1: {
+        V m[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) m[i] = V{R(op->m[2 * i]), R(op->m[2 * i + 1])};
         if (t0 < 0) {  // diagonal op on a bit constant over the tile
-          const V d = cvt<R>(M.m[((base >> op->g0) & 1) ? 3 : 0]);
-          for (int j = tid; j < S; j += nthr) tile[IX(j)] = cmul(tile[IX(j)], d);
-        } else if (kind == PQS_OP_RZ) {
-          const V d0 = cvt<R>(M.m[0]), d1 = cvt<R>(M.m[3]);
-          for (int j = tid; j < S; j += nthr) tile[IX(j)] = cmul(tile[IX(j)], ((j >> t0) & 1) ? d1 : d0);
+          const V d = m[((base >> op->g0) & 1) ? 3 : 0];
+          for (int j = tid; j < S; j += nthr) tile[IX(j)] = cmul_at(d, tile[IX(j)]);
         } else {
-          const V m00 = cvt<R>(M.m[0]), m01 = cvt<R>(M.m[1]), m10 = cvt<R>(M.m[2]), m11 = cvt<R>(M.m[3]);
-          for (int u = tid; u < (S >> 1); u += nthr) {
-            const int j0 = ins0(u, t0), j1 = j0 | (1 << t0);
-            const V a = tile[IX(j0)], b = tile[IX(j1)];
-            tile[IX(j0)] = cadd(cmul(m00, a), cmul(m01, b));
-            tile[IX(j1)] = cadd(cmul(m10, a), cmul(m11, b));
-          }
+          pairs([&](V &a, V &b) {
+            const V p = a, q = b;
+            a = cadd(cmul_at(m[0], p), cmul_at(m[1], q));
+            b = cadd(cmul_at(m[2], p), cmul_at(m[3], q));
+          });
         }
         break;
       }
       case PQS_OP_CX: {
-        const bool ctl_in = t0 >= 0;
-        const bool ctl_on = !ctl_in && ((base >> op->g0) & 1);
-        if (ctl_in || ctl_on) {
+        if (t0 >= 0) {
+          quads([&](V(&a)[4]) {
+            const V p = a[2];
+            a[2] = a[3];
+            a[3] = p;
+          });
+        } else if ((base >> op->g0) & 1) {
           for (int u = tid; u < (S >> 1); u += nthr) {
-            const int j0 = ins0(u, t1);
-            if (ctl_in && !((j0 >> t0) & 1)) continue;
-            const int j1 = j0 | (1 << t1);
+            const int j0 = ins0(u, t1), j1 = j0 | (1 << t1);
             const V a = tile[IX(j0)];
             tile[IX(j0)] = tile[IX(j1)];
             tile[IX(j1)] = a;
@@ -294,49 +282,64 @@ __device__ __forceinline__ void apply_lds_op(typename CT<R>::V *tile, const int 
           d[0] = d[1] = d[2] = V{R(1), R(0)};
           d[3] = V{R(-1), R(0)};
         } else {
-          double s_, c_;
-          sincos(0.5 * op_angle(op, params), &s_, &c_);
-          d[0] = d[3] = V{R(c_), R(-s_)};
-          d[1] = d[2] = V{R(c_), R(s_)};
+          d[0] = d[3] = V{c, -s};
+          d[1] = d[2] = V{c, s};
         }
         const int c0 = t0 < 0 ? int((base >> op->g0) & 1) : -1;
         const int c1 = t1 < 0 ? int((base >> op->g1) & 1) : -1;
         for (int j = tid; j < S; j += nthr) {
           const int b0 = c0 >= 0 ? c0 : ((j >> t0) & 1);
           const int b1 = c1 >= 0 ? c1 : ((j >> t1) & 1);
-          tile[IX(j)] = cmul(tile[IX(j)], d[2 * b0 + b1]);
+          const V a = tile[IX(j)], z = d[2 * b0 + b1];
+          tile[IX(j)] = V{fma(a.x, z.x, -(a.y * z.y)), fma(a.y, z.x, a.x * z.y)};
         }
         break;
       }
-      case PQS_OP_MAT2:
       case PQS_OP_RXX:
-      case PQS_OP_RYY:
-      case PQS_OP_FSIM:
+      case PQS_OP_RYY: {
+        const R w = kind == PQS_OP_RXX ? s : -s;  // X(x)X: 00<->11 with +1, Y(x)Y: with -1; 01<->10 with +1
+        quads([&](V(&a)[4]) {
+          mix_i(a[0], a[3], c, w);
+          mix_i(a[1], a[2], c, s);
+        });
+        break;
+      }
+      case PQS_OP_FSIM:  // gates.py:598-606, 619-627, 640-648, 708-716, 729-737
+        quads([&](V(&a)[4]) {
+          mix_i(a[1], a[2], c, s);
+          a[3] = cmul_at(V{cf.cp, -cf.sp}, a[3]);
+        });
+        break;
       case PQS_OP_GEN_FSIM: {
-        M4 M;
-        mat2_of(op, params, M);
+        // as the reference writes them: d_theta leaves the corners, d_phi the block
+        const int sel = op->pauli;
+        const V m15 = sel == 3 ? V{R(1), R(0)} : sel == 2 ? V{-cf.sp, -cf.cp} : V{cf.cp, -cf.sp};
+        quads([&](V(&a)[4]) {
+          if (sel == 2) mix_i(a[1], a[2], c, s);
+          else mix_i(a[1], a[2], -s, c);
+          a[3] = cmul_at(m15, a[3]);
+        });
+        break;
+      }
+      case PQS_OP_MAT2: {
         V m[16];
 #pragma unroll
-        for (int i = 0; i < 16; ++i) m[i] = cvt<R>(M.m[i]);
-        const int lo = t0 < t1 ? t0 : t1, hi = t0 < t1 ? t1 : t0;
-        for (int u = tid; u < (S >> 2); u += nthr) {
-          const int j = ins0(ins0(u, lo), hi);
-          const int jj[4] = {j, j | (1 << t1), j | (1 << t0), j | (1 << t0) | (1 << t1)};
-          V a[4];
-#pragma unroll
-          for (int c = 0; c < 4; ++c) a[c] = tile[IX(jj[c])];
+        for (int i = 0; i < 16; ++i) m[i] = V{R(op->m[2 * i]), R(op->m[2 * i + 1])};
+        quads([&](V(&a)[4]) {
+          V y[4];
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
-            V acc = cmul(m[4 * r], a[0]);
+            y[r] = cmul_at(m[4 * r], a[0]);
 #pragma unroll
-            for (int c = 1; c < 4; ++c) acc = cadd(acc, cmul(m[4 * r + c], a[c]));
-            tile[IX(jj[r])] = acc;
+            for (int i = 1; i < 4; ++i) y[r] = cadd(y[r], cmul_at(m[4 * r + i], a[i]));
           }
-        }
+#pragma unroll
+          for (int r = 0; r < 4; ++r) a[r] = y[r];
+        });
         break;
       }
       case pqs::kPauliSum: {
-                V acc[MAXPER];
+        V acc[MAXPER];
         const int nt = op->nterms;
         const DevTerm *tm = terms + op->term0;
 #pragma unroll
@@ -424,13 +427,35 @@ __device__ __forceinline__ void sweep_lds_body(const DevSweep &sw, const DevOp *
     tile[j] = v;
   }
 
-  const double *params = in.params;
-  for (int o = sw.op_begin; o < sw.op_end; ++o) {
-    const DevOp *op = ops + o;
-    const int tg = op->tangent;
-    if (tg >= 0 && tg != in.tangent) continue;
+  // Ops in runs of one per thread: each thread works out the angles of its op
+  // of the run, then the block walks the run.  Before, every thread computed
+  // the sincos of every op (2000 8-qubit states of 10 HEA layers: 364 -> 277 us;
+  // 500 of 10 XXZ layers 369 -> 215).
+  __shared__ LdsCoef<R> coefs[BLOCK];
+  __shared__ int4 recs[BLOCK];
+  for (int o0 = sw.op_begin; o0 < sw.op_end; o0 += BLOCK) {
+    const int run = sw.op_end - o0 < BLOCK ? sw.op_end - o0 : BLOCK;
     __syncthreads();
-    apply_lds_op<R, 512 / BLOCK, false>(tile, S, op, base, params, terms, tid, BLOCK);
+    if (tid < run) {
+      const DevOp *d = ops + o0 + tid;
+      coefs[tid] = lds_coef<R>(d, in.params);
+      recs[tid] = int4{d->kind, d->t0, d->t1, d->tangent};
+    }
+    __syncthreads();
+    int4 rec = recs[0];
+    LdsCoef<R> cf = coefs[0];
+    for (int i = 0; i < run; ++i) {
+      const int kind = __builtin_amdgcn_readfirstlane(rec.x), t0 = __builtin_amdgcn_readfirstlane(rec.y);
+      const int t1 = __builtin_amdgcn_readfirstlane(rec.z), tg = __builtin_amdgcn_readfirstlane(rec.w);
+      const LdsCoef<R> now = cf;
+      if (i + 1 < run) {
+        rec = recs[i + 1];
+        cf = coefs[i + 1];
+      }
+      if (tg >= 0 && tg != in.tangent) continue;
+      __syncthreads();
+      apply_lds_op<R, 512 / BLOCK, false>(tile, S, ops + o0 + i, kind, t0, t1, now, base, terms, tid, BLOCK);
+    }
   }
   __syncthreads();
 
@@ -825,6 +850,9 @@ __device__ __forceinline__ void sweep_reg_body(const DevSweep &sw, const DevOp *
       r.t01 = int32_t(uint32_t(r.t01) | ((tg & 0xffffu) << 16));
       r.g01 = int32_t(uint32_t(r.g01) | ((tg >> 16) << 16));
     }
+    if constexpr (LDSOPS && sizeof(R) == 4) {  // angles of LDS phases: four floats in (t, f)
+      if (d->coef < 0 && d->kind != pqs::kGen1) *reinterpret_cast<LdsCoef<R> *>(&r.t) = lds_coef<R>(d, params);
+    }
     if (d->coef >= 0) {
       double sn, cs;
       sincos(0.5 * op_angle(d, params), &sn, &cs);
@@ -851,7 +879,9 @@ __device__ __forceinline__ void sweep_reg_body(const DevSweep &sw, const DevOp *
         for (int o = P->op_begin; o < P->op_end; ++o) {
           const DevOp *op = ops + o;
           if (op->tangent >= 0 && op->tangent != in.tangent) continue;
-          apply_lds_op<R, NA, true>(tile, S, op, base, params, terms, tid, nthr);
+          LdsCoef<R> cf{};
+          if constexpr (sizeof(R) == 4) cf = *reinterpret_cast<const LdsCoef<R> *>(&rops[o - sw.op_begin].t);
+          apply_lds_op<R, NA, true>(tile, S, op, op->kind, op->t0, op->t1, cf, base, terms, tid, nthr);
           __syncthreads();
         }
       }
@@ -1012,11 +1042,20 @@ __device__ __forceinline__ void sweep_reg_body(const DevSweep &sw, const DevOp *
           if constexpr (LDSOPS) {
             const DevOp *d = ops + o;
             if (kind == PQS_OP_GEN_FSIM && d->tangent != in.tangent) break;  // uniform per block
-            M4 M;
-            mat2_of(d, params, M);
             V m[16];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) m[i] = cvt<R>(M.m[i]);
+            for (int i = 0; i < 16; ++i) m[i] = V{R(d->m[2 * i]), R(d->m[2 * i + 1])};
+            if (kind != PQS_OP_MAT2) {
+              const LdsCoef<R> cf = lds_coef<R>(d, params);
+              const int sel = kind == PQS_OP_FSIM ? 0 : d->pauli;
+              const bool dth = sel == 1 || sel == 3;  // d_theta, as the reference writes it
+#pragma unroll
+              for (int i = 0; i < 16; ++i) m[i] = V{R(0), R(0)};
+              m[0] = V{R(1), R(0)};
+              m[5] = m[10] = V{dth ? -cf.s : cf.c, R(0)};
+              m[6] = m[9] = V{R(0), dth ? -cf.c : -cf.s};
+              m[15] = sel == 3 ? V{R(1), R(0)} : sel == 2 ? V{-cf.sp, -cf.cp} : V{cf.cp, -cf.sp};
+            }
             SW4(r0, SW4C(r1, reg_mat2<B_, C_>(a, m)));
           }
           break;
