@@ -55,6 +55,7 @@ __device__ __forceinline__ V cmul(V a, V b) { return V{a.x * b.x - a.y * b.y, a.
 __device__ __forceinline__ V cadd(V a, V b) { return V{a.x + b.x, a.y + b.y}; }
 __device__ __forceinline__ int swz(int j) { return j ^ (((j >> 4) ^ (j >> 8) ^ (j >> 12)) & 15); }
 // LDS tile element at a byte offset (phase addresses are XORs of byte offsets)
+#define LDSD(o) (*reinterpret_cast<double *>(reinterpret_cast<char *>(tile) + (o)))
 #define LDSB(o) (*reinterpret_cast<V *>(reinterpret_cast<char *>(tile) + (o)))
 template <int B> __device__ __forceinline__ void ry(V (&a)[NA], R t) {
 #pragma unroll
@@ -331,6 +332,72 @@ std::string jit_source(const pqs_plan &p, std::vector<int> &sweeps_out) {
   return o.str();
 }
 
+static bool can_halve(const pqs_plan &p, int s) {
+  const DevSweep &ds = p.dev_sweeps[size_t(s)];
+  if (p.dtype != PQS_C128 || (p.flags & PQS_PLAN_JIT_PERSISTENT) || ds.phase_end == ds.phase_begin) return false;
+  for (int ph = ds.phase_begin; ph < ds.phase_end; ++ph)
+    if (p.dev_phases[size_t(ph)].lds) return false;
+  return true;
+}
+
+// Slots of a tile of doubles: linear in the tile index, the low five bits such
+// that the first five lane bits of as many phases as possible reach 32
+// different ones, so that 32 lanes read or write 8 bytes each from all banks.
+struct Slots {
+  int col[kMaxTileBits];
+};
+static Slots half_slots(const pqs_plan &p, const DevSweep &ds) {
+  // tile bits of the first five lane bits: the load, the phases, the store
+  std::vector<std::vector<int>> lanes;
+  const int nl = std::min(5, ds.k - kRegBits);
+  std::vector<int> v(static_cast<size_t>(nl));
+  for (int i = 0; i < nl; ++i) v[size_t(i)] = i;
+  if (!ds.direct_load) lanes.push_back(v);
+  for (int ph = ds.phase_begin; ph < ds.phase_end; ++ph) {
+    for (int i = 0; i < nl; ++i) v[size_t(i)] = p.dev_phases[size_t(ph)].tb[i];
+    lanes.push_back(v);
+  }
+  for (int i = 0; i < nl; ++i) v[size_t(i)] = ds.rolling ? ds.sperm[i] : i;
+  if (!ds.direct_store) lanes.push_back(v);
+  auto conflicts = [&](const Slots &c) {
+    int n = 0;
+    for (const auto &l : lanes) {
+      int basis[5] = {0, 0, 0, 0, 0}, rank = 0;
+      for (int bit : l) {
+        int v = c.col[bit] & 31;
+        for (int b = 4; b >= 0 && v; --b) {
+          if (!((v >> b) & 1)) continue;
+          if (!basis[b]) {
+            basis[b] = v;
+            ++rank;
+            v = 0;
+          } else {
+            v ^= basis[b];
+          }
+        }
+      }
+      n += nl - rank;
+    }
+    return n;
+  };
+  Slots best{}, c{};
+  for (int b = 0; b < kMaxTileBits; ++b) best.col[b] = (1 << b) | (b >= 5 ? 1 << (b % 5) : 0);
+  int least = conflicts(best);
+  uint32_t seed = 12345;
+  for (int t = 0; t < 4000 && least > 0; ++t) {
+    for (int b = 0; b < kMaxTileBits; ++b) {
+      seed = seed * 1664525u + 1013904223u;
+      c.col[b] = (1 << b) | (b >= 5 ? int((seed >> 16) & 31) : 0);
+    }
+    const int n = conflicts(c);
+    if (n < least) {
+      least = n;
+      best = c;
+    }
+  }
+  return best;
+}
+
 static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
   const int S_total = int(p.dev_sweeps.size());
   {
@@ -423,10 +490,24 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
     // b + G, b + 2G, ... and issues the loads of its next tile into
     // registers before the current tile's phases, so HBM traffic overlaps
     // compute when only one block fits per CU.
-    o << "extern \"C\" __global__ __launch_bounds__(" << nthr << ") void " << (pair ? "pqs_jit_pair_" : "pqs_jit_sweep_")
+    // Halves: a transition trades the real parts through a tile of doubles,
+    // then the imaginary ones, so a block holds half the LDS.  What bounds
+    // these sweeps is FP64 issue (3/4 of the cycles at 2 waves per SIMD, the
+    // most that whole tiles leave room for); 3 waves cover the LDS round trips
+    // and barriers better: 10,000 16-qubit states of 20 HEA layers 47.5 ->
+    // 45 ms, 1000 12-qubit XXZ states (one 12-bit tile each, all resident at
+    // once) 312 -> 266 us, one 24-qubit state 1144 -> 1065 us; single tiles,
+    // which wait for their own barriers alone, 126 -> 128 us.  A bound of 4
+    // waves spills: up to 2% faster at 16 qubits, 10% slower at 24.  Sweeps
+    // with measurements spill at 3 and keep the whole tile (20-qubit gradient
+    // 1.9 against 6.9 ms), pair kernels too (they hold a second state).
+    const bool halves = can_halve(p, s) && !pair && !nm;
+    Slots slots;
+    if (halves) slots = half_slots(p, ds);
+    o << "extern \"C\" __global__ __launch_bounds__(" << nthr << (halves ? ", 3" : "") << ") void " << (pair ? "pqs_jit_pair_" : "pqs_jit_sweep_")
       << s << "(const InstDev *__restrict__ insts, long long n_active, const V *__restrict__ init_tab"
       << (pair ? ", double2 *__restrict__ pov" : p.n_meas ? ", double *__restrict__ mpart" : "") << ") {\n";
-    o << "  __shared__ V tile[" << S << "];\n";
+    o << "  __shared__ " << (halves ? "double" : "V") << " tile[" << S << "];\n";
     o << "  __shared__ double2 tf[" << (na > 0 ? na : 1) << "];\n";
     o << "  const int tid = threadIdx.x;\n";
     if (nm) o << "  __shared__ double mred[" << nm * nwaves << "];\n";
@@ -538,8 +619,42 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
     o << "  const u64 dl = base | dtid;\n";
     o << "  const double *params = in.params;\n";
     o << "  __syncthreads();\n";
-    if (!dload)
+    // registers carried into a phase that takes its layout by an exchange, and
+    // the imaginary parts between the two halves of a transition
+    o << "  V areg[NA];\n";
+    if (halves) o << "  int hb;\n";
+    bool half_pending = false;
+    std::string half_sync;
+    int half_kv[NA_()];
+    // the real parts are in the tile: read them, then trade the imaginary ones
+    auto second_half = [&](const char *a, const int *kv) {
+      for (int v = 0; v < NA_(); ++v) o << "    " << a << "[" << v << "].x = LDSD(ptb ^ " << 8 * kv[v] << ");\n";
+      o << half_sync;
+      for (int v = 0; v < NA_(); ++v) o << "    LDSD(hb ^ " << 8 * half_kv[v] << ") = areg[" << v << "].y;\n";
+      o << half_sync;
+      for (int v = 0; v < NA_(); ++v) o << "    " << a << "[" << v << "].y = LDSD(ptb ^ " << 8 * kv[v] << ");\n";
+      half_pending = false;
+    };
+    // slot of a thread whose bit i is tile bit b[i] (halves), as an expression
+    auto thread_slot = [&](const char *tid, auto bit, int n) {
+      std::ostringstream e;
+      e << "0";
+      for (int i = 0; i < n; ++i) e << " ^ (-((" << tid << " >> " << i << ") & 1) & " << slots.col[bit(i)] << ")";
+      return e.str();
+    };
+    if (!dload && halves) {
+      o << "  hb = 8 * (" << thread_slot("tid", [](int i) { return i; }, kt) << ");\n";
+      for (int v = 0; v < NA_(); ++v) {
+        half_kv[v] = 0;
+        for (int b = 0; b < kRegBits; ++b)
+          if (v & (1 << b)) half_kv[v] ^= slots.col[kt + b];
+        o << "  LDSD(hb ^ " << 8 * half_kv[v] << ") = pre[" << v << "].x;\n  areg[" << v << "].y = pre[" << v << "].y;\n";
+      }
+      half_sync = "    __syncthreads();\n";
+      half_pending = true;
+    } else if (!dload) {
       o << "#pragma unroll\n  for (int m = 0; m < NA; ++m) tile[swz(tid + m * " << nthr << ")] = pre[m];\n";
+    }
     if (persist) o << "  if (t + gridDim.x < total) fetch(t + gridDim.x, pre);\n";
     if (na > 0) {
       o << "  for (int i = tid; i < " << na << "; i += " << nthr << ") {\n";
@@ -562,8 +677,6 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
     // is applied at the end of the sweep, at the end of a phase with
     // per-lane sign flips, or early by the growth check
     o << "  double fs = 1.0;\n";
-    // registers carried into a phase that takes its layout by an exchange
-    o << "  V areg[NA];\n";
     // (tan, cos) of the next phase's first rotations, read from the angle
     // table before this phase's LDS writes: LDS returns in issue order, so
     // a table read issued after the transition's 16 reads would hold the
@@ -632,20 +745,28 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
         o << "    const int ptid = tid;\n";
       o << "    const int toff = 0";
       for (int i = 0; i < P.ntb; ++i) o << " | (((ptid >> " << i << ") & 1) << " << P.tb[i] << ")";
-      o << ";\n    const int pt = swz(toff);\n";
+      o << ";\n";
+      auto slot_of = [&](int bit) { return halves ? slots.col[bit] : swz_host(1 << bit); };
+      if (halves) {
+        o << "    const int pt = " << thread_slot("ptid", [&](int i) { return P.tb[i]; }, P.ntb) << ";\n";
+      } else {
+        o << "    const int pt = swz(toff);\n";
+      }
       int kv[NA_()];
       for (int v = 0; v < NA_(); ++v) {
         int a = 0;
         for (int i = 0; i < kRegBits; ++i)
-          if (v & (1 << i)) a ^= swz_host(1 << P.rb[i]);
+          if (v & (1 << i)) a ^= slot_of(P.rb[i]);
         kv[v] = a;
       }
-      o << "    const int ptb = pt * int(sizeof(V));\n    V a[NA];\n";
+      o << "    const int ptb = pt * int(sizeof(*tile));\n    V a[NA];\n";
       if (carry) {
         for (int v = 0; v < NA_(); ++v) o << "    a[" << v << "] = areg[" << v << "];\n";
         carry = false;
       } else if (dload && ph == ds.phase_begin) {
         for (int v = 0; v < NA_(); ++v) o << "    a[" << v << "] = pre[" << v << "];\n";
+      } else if (half_pending) {
+        second_half("a", kv);
       } else {
         for (int v = 0; v < NA_(); ++v)
           o << "    a[" << v << "] = LDSB(ptb ^ (" << kv[v] << " * int(sizeof(V))));\n";
@@ -966,7 +1087,7 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
         if (any) {
           o << "    const int pst = pt";
           for (int r = 0; r < kRegBits; ++r)
-            if (fl[r]) o << " ^ (" << xf(r) << " ? " << swz_host(1 << P.rb[r]) << " : 0)";
+            if (fl[r]) o << " ^ (" << xf(r) << " ? " << slot_of(P.rb[r]) << " : 0)";
           o << ";\n";
         } else {
           o << "    const int pst = pt;\n";
@@ -1005,9 +1126,17 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
         continue;
       }
       next_pre = preload(ph + 1);
-      o << "    const int pstb = pst * int(sizeof(V));\n";
-      for (int v = 0; v < NA_(); ++v)
-        o << "    LDSB(pstb ^ (" << kv[v] << " * int(sizeof(V)))) = a[" << v << "];\n";
+      if (halves) {
+        o << "    hb = pst * 8;\n";
+        for (int v = 0; v < NA_(); ++v) {
+          half_kv[v] = kv[v];
+          o << "    LDSD(hb ^ " << 8 * kv[v] << ") = a[" << v << "].x;\n    areg[" << v << "].y = a[" << v << "].y;\n";
+        }
+      } else {
+        o << "    const int pstb = pst * int(sizeof(V));\n";
+        for (int v = 0; v < NA_(); ++v)
+          o << "    LDSB(pstb ^ (" << kv[v] << " * int(sizeof(V)))) = a[" << v << "];\n";
+      }
       // the next phase keeps the wave bits (thread bits 6..): its LDS reads
       // touch only this wave's amplitudes, which this wave's own earlier
       // LDS writes (executed in order) already hold
@@ -1017,19 +1146,36 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
         wave_local = !Q.lds && Q.ntb == P.ntb;
         for (int i = 6; wave_local && i < P.ntb; ++i) wave_local = Q.tb[i] == P.tb[i];
       }
-      if (wave_local)
-        o << "    __builtin_amdgcn_fence(__ATOMIC_RELEASE, \"wavefront\");\n"
-             "    __builtin_amdgcn_wave_barrier();\n"
-             "    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");\n  }\n";
-      else
-        o << "    __syncthreads();\n  }\n";
+      half_sync = wave_local ? "    __builtin_amdgcn_fence(__ATOMIC_RELEASE, \"wavefront\");\n"
+                               "    __builtin_amdgcn_wave_barrier();\n"
+                               "    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, \"wavefront\");\n"
+                             : "    __syncthreads();\n";
+      half_pending = halves;
+      o << half_sync << "  }\n";
     }
+    if (halves && !dstore) {
+      // the store's layout, read through the halves as a phase's
+      auto bit = [&](int i) { return ds.rolling ? ds.sperm[i] : i; };
+      int kv[NA_()];
+      for (int v = 0; v < NA_(); ++v) {
+        kv[v] = 0;
+        for (int b = 0; b < kRegBits; ++b)
+          if (v & (1 << b)) kv[v] ^= slots.col[bit(kt + b)];
+      }
+      o << "  V w[NA];\n  {\n    const int ptb = 8 * (" << thread_slot("tid", bit, kt) << ");\n";
+      second_half("w", kv);
+      o << "  }\n";
+    }
+    auto stored = [&](int m, const std::string &index) {
+      return halves ? "w[" + std::to_string(m) + "]" : "tile[swz(" + index + ")]";
+    };
     if (dstore) {
       // stored by the last phase
     } else if (!ds.rolling) {
       for (int m = 0; m < NA_(); ++m) {
-        o << "  {\n    const V w = tile[swz(tid + " << m * nthr << ")];\n    dst[dl | " << hp(m) << "ull] = w;\n";
-        capture(std::to_string(m), "w");
+        o << "  {\n    const V x = " << stored(m, "tid + " + std::to_string(m * nthr)) << ";\n    dst[dl | " << hp(m)
+          << "ull] = x;\n";
+        capture(std::to_string(m), "x");
         o << "  }\n";
       }
     } else {
@@ -1050,8 +1196,9 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
             cm |= 1ull << ds.wpos[ds.sperm[kt + b]];
             jm |= 1 << ds.sperm[kt + b];
           }
-        o << "    {\n    const V w = tile[swz(jdl | " << jm << ")];\n    dst[wdl | " << cm << "ull] = w;\n";
-        capture(std::to_string(m), "w");
+        o << "    {\n    const V x = " << stored(m, "jdl | " + std::to_string(jm)) << ";\n    dst[wdl | " << cm
+          << "ull] = x;\n";
+        capture(std::to_string(m), "x");
         o << "    }\n";
       }
       o << "  }\n";
