@@ -4024,9 +4024,10 @@ int cgram_mfma(pqs_ctx *ctx, int32_t dtype, const void *a, int64_t lda, int64_t 
   // The split over K: a 4-wide step of 8 blocks takes one wave about 1 us, and
   // every chunk's partials are written and read once (half of them for A =
   // B).  The split with the least sum of the two (chunks of at least two ring
-  // turns, partials within 2 GiB); the first of them at a tie.  Measured, 1000
-  // states of 12 qubits: 320 us for the product in 15 chunks and 95 us for
-  // their sum, 330 and 12 us in 7.
+  // turns, partials within 2 GiB); the first of them at a tie.  A wave alone
+  // on its SIMD waits for its loads: a tenth more (2000 states of 16 qubits:
+  // 1 chunk 20.1 ms, 2 chunks 17.9).  Measured, 1000 states of 12 qubits: 320 us for the product in
+  // 15 chunks and 95 us for their sum, 330 and 12 us in 7.
   const int64_t slots = 4 * SYWAVES * int64_t(ctx->n_cu);
   const int64_t ks_max = std::max<int64_t>(
       1, std::min<int64_t>({Kc / (2 * ring), int64_t(64), int64_t((size_t(2) << 30) / (size_t(m) * size_t(nn) * 16))}));
@@ -4035,7 +4036,8 @@ int cgram_mfma(pqs_ctx *ctx, int32_t dtype, const void *a, int64_t lda, int64_t 
   for (int64_t k = 1; k <= ks_max; ++k) {
     const int64_t per_simd = (T * k + slots / 2 - 1) / (slots / 2);
     const int64_t chunk = ((Kc + k - 1) / k + ring - 1) / ring * ring;
-    const double us = double(chunk / CGK * per_simd) + double(k) * double(m) * double(nn) * (sym ? 16 : 32) / 4e6;
+    const double us = double(chunk / CGK * per_simd) * (per_simd == 1 ? 1.1 : 1.0) +
+                      double(k) * double(m) * double(nn) * (sym ? 16 : 32) / 4e6;
     if (us < best) {
       best = us;
       ks = k;

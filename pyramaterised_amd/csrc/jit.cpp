@@ -493,14 +493,15 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
     // Halves: a transition trades the real parts through a tile of doubles,
     // then the imaginary ones, so a block holds half the LDS.  What bounds
     // these sweeps is FP64 issue (3/4 of the cycles at 2 waves per SIMD, the
-    // most that whole tiles leave room for); 3 waves cover the LDS round trips
-    // and barriers better: 10,000 16-qubit states of 20 HEA layers 47.5 ->
-    // 45 ms, 1000 12-qubit XXZ states (one 12-bit tile each, all resident at
-    // once) 312 -> 266 us, one 24-qubit state 1144 -> 1065 us; single tiles,
-    // which wait for their own barriers alone, 126 -> 128 us.  A bound of 4
-    // waves spills: up to 2% faster at 16 qubits, 10% slower at 24.  Sweeps
-    // with measurements spill at 3 and keep the whole tile (20-qubit gradient
-    // 1.9 against 6.9 ms), pair kernels too (they hold a second state).
+    // most that whole tiles leave room for, and at the card's power limit: an
+    // effective 1.9 GHz); 3 waves cover the LDS round trips and barriers
+    // better: 10,000 16-qubit states of 20 HEA layers 47.5 -> 45.6 ms, 1000
+    // 12-qubit XXZ states (one 12-bit tile each, all resident at once) 312 ->
+    // 266 us, one 24-qubit state 1144 -> 1065 us; single tiles, which wait for
+    // their own barriers alone, 126 -> 128 us.  A bound of 4 waves spills: up
+    // to 2% faster at 16 qubits, 10% slower at 24.  Sweeps with measurements
+    // hold more registers and keep the whole tile (20-qubit gradient bounded
+    // to 4 waves: 6.9 against 1.9 ms), pair kernels too (a second state).
     const bool halves = can_halve(p, s) && !pair && !nm;
     Slots slots;
     if (halves) slots = half_slots(p, ds);
@@ -703,7 +704,6 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
     };
     std::vector<int> next_pre;
     int n_meas_done = 0;  // measurements whose wave totals are in mred
-    int mg = 0;           // groups emitted (names)
     bool carry = false;
     int nrot = 0;  // rotations since the last check of the accumulated scale
     // phases
@@ -804,7 +804,6 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
           << ">(ln);\n      if ((ln & " << (64 / M - 1) << ") == 0 && f < " << mvals.size() << ") mred[(ptid >> 6) * "
           << nm << " + " << n_meas_done << " + f] = mv[0]; }\n";
         n_meas_done += int(mvals.size());
-        ++mg;
         mvals.clear();
       };
       for (int i = P.op_begin; i < P.op_end; ++i) {
