@@ -321,6 +321,14 @@ int pqs_run_batch_noalloc(pqs_ctx *ctx, pqs_plan *plan, void *states_dev, int64_
                           const double *params_dev, int64_t param_stride, int32_t init, const void *src_dev,
                           void *alt_dev, const void *init_table_dev, void *stream);
 
+/* pqs_run_batch with the parameters (batch rows of n_params doubles, at least
+ * one) and the product table in host memory: they travel with the instance
+ * table in one upload.  For calls whose inputs are small and start on the host;
+ * the inputs occupy context workspace. */
+int pqs_run_batch_host(pqs_ctx *ctx, pqs_plan *plan, void *states_dev, int64_t state_stride, int64_t batch,
+                       const double *params_host, int64_t n_params, const int32_t *tangents_host, int32_t init,
+                       const void *src_dev, const void *init_table_host, void *stream);
+
 /* All derivative states in one pass: psi_dev gets U|psi0>, jac_dev (row t =
  * tangent t, n_tangents rows of 2^N) gets every d psi / d theta_t.  Tangent t
  * is spawned from the plain state at the sweep that holds its generator and
@@ -329,6 +337,11 @@ int pqs_run_batch_noalloc(pqs_ctx *ctx, pqs_plan *plan, void *states_dev, int64_
 int pqs_jacobian(pqs_ctx *ctx, pqs_plan *plan, const double *params_dev,
                  int32_t init, const void *src_dev, const void *init_table_dev,
                  void *psi_dev, void *jac_dev, void *stream);
+
+/* pqs_jacobian with the parameters (n_params doubles, at least one) and the
+ * product table in host memory, as pqs_run_batch_host. */
+int pqs_jacobian_host(pqs_ctx *ctx, pqs_plan *plan, const double *params_host, int64_t n_params, int32_t init,
+                      const void *src_dev, const void *init_table_host, void *psi_dev, void *jac_dev, void *stream);
 
 /* out[p] = <a_p|b_p> (complex, dtype of the states) for n_pairs pairs, each
  * pair given by element offsets (in amplitudes) from base_dev.

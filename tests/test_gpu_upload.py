@@ -189,3 +189,42 @@ def test_device_written_batch_tables(E, dtype, rolling):
     ref = (st[0:B:2].conj() * st[1:B:2]).sum(1)
     # 2^7 products of unit vectors: 128 roundings of at most 2^-53 each
     assert float((ov.cpu() - ref).abs().max()) < 128 * 2.0 ** -53
+
+
+@pytest.mark.parametrize("dtype", ["complex128", "complex64"])
+def test_host_inputs_match_device_inputs(E, dtype):
+    """Runs and Jacobians whose inputs travel with the instance table give the
+    bits of the same calls with inputs on the GPU: every initial state, row
+    counts around the size limit, tangents, and the caller's arrays reused at
+    once behind a busy stream."""
+    import pyramaterised_amd as pyqc
+    from pyramaterised_amd import templates as T
+    n = 5
+    rng = np.random.default_rng(17)
+    qc = pyqc.PQC(n)
+    for layer in T.clifford_HE_layers(1, n):
+        qc.add_layer(layer)
+    P = qc.n_true_params
+    plain, full = E.Plan(n, qc.ops(), dtype=dtype), E.Plan(n, qc.ops(True), dtype=dtype)
+    vec = rng.normal(size=1 << n) + 1j * rng.normal(size=1 << n)
+    prod = [v / np.linalg.norm(v) for v in rng.normal(size=(n, 2)) + 1j * rng.normal(size=(n, 2))]
+    x = torch.ones(1 << 26, dtype=torch.float64, device="cuda")
+    edge = E.HOST_INPUT_BYTES // (8 * P + 48)
+    for init in (E.Init.zero(), E.Init.product(prod), E.Init.from_vector(vec / np.linalg.norm(vec))):
+        for B in (1, 2, edge - 1, edge, edge + 1):
+            th = rng.random((B, P)) * 2 * np.pi
+            dev = torch.as_tensor(th, device="cuda")
+            tg = [-1] * (B - 1) + [P - 1]
+            _busy(x, 2)
+            got, got_t = E.run(plain, th, init), E.run(full, th, init, tangents=tg)
+            psi, J = E.jacobian(full, th[0], init)
+            want = th[0].copy()
+            th[:] = 0.5  # the caller reuses its array at once
+            assert torch.equal(got, E.run(plain, dev, init)), (init.kind, B)
+            assert torch.equal(got_t, E.run(full, dev, init, tangents=tg)), (init.kind, B)
+            pd, Jd = E.jacobian(full, torch.as_tensor(want, device="cuda"), init)
+            assert torch.equal(psi, pd) and torch.equal(J, Jd), (init.kind, B)
+    with pytest.raises(E.EngineError):
+        E.run(full, want, E.Init.zero(), tangents=[P])
+    bare = E.Plan(n, [], dtype=dtype)  # no parameters at all
+    assert torch.equal(E.run(bare, np.zeros(0), E.Init.zero()), E.run(bare, torch.zeros(1, device="cuda"), E.Init.zero()))
