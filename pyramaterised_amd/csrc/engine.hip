@@ -851,7 +851,11 @@ __device__ __forceinline__ void sweep_reg_body(const DevSweep &sw, const DevOp *
       r.g01 = int32_t(uint32_t(r.g01) | ((tg >> 16) << 16));
     }
     if constexpr (LDSOPS && sizeof(R) == 4) {  // angles of LDS phases: four floats in (t, f)
-      if (d->coef < 0 && d->kind != pqs::kGen1) *reinterpret_cast<LdsCoef<R> *>(&r.t) = lds_coef<R>(d, params);
+      if (d->coef < 0 && d->kind != pqs::kGen1) {
+        const LdsCoef<R> cf = lds_coef<R>(d, params);
+        __builtin_memcpy(&r.t, &cf.c, sizeof(double));
+        __builtin_memcpy(&r.f, &cf.cp, sizeof(double));
+      }
     }
     if (d->coef >= 0) {
       double sn, cs;
@@ -880,7 +884,10 @@ __device__ __forceinline__ void sweep_reg_body(const DevSweep &sw, const DevOp *
           const DevOp *op = ops + o;
           if (op->tangent >= 0 && op->tangent != in.tangent) continue;
           LdsCoef<R> cf{};
-          if constexpr (sizeof(R) == 4) cf = *reinterpret_cast<const LdsCoef<R> *>(&rops[o - sw.op_begin].t);
+          if constexpr (sizeof(R) == 4) {
+            __builtin_memcpy(&cf.c, &rops[o - sw.op_begin].t, sizeof(double));
+            __builtin_memcpy(&cf.cp, &rops[o - sw.op_begin].f, sizeof(double));
+          }
           apply_lds_op<R, NA, true>(tile, S, op, op->kind, op->t0, op->t1, cf, base, terms, tid, nthr);
           __syncthreads();
         }
