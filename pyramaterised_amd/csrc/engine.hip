@@ -1154,16 +1154,20 @@ __global__ __launch_bounds__(MAXT) void k_sweep_reg(const DevSweep sw, const Dev
 // the partner fetch of any other op.  Op records come 64 at a time, one per
 // lane, and are read out into scalar registers, so no op waits for memory and
 // dispatch is scalar.  Angles belong to the instance: at a refill each lane
-// computes (tan, cos) of kWaveAngles of its tile's angles (their parameters
-// were loaded a refill ahead) into 4 KB of LDS.  Rotations are in scaled
-// form, the scale clamped and checked as in the specialised kernels (jit.cpp).
+// computes (sin, cos) of half of kWaveAngles of its tile's angles (their
+// parameters were loaded a refill ahead) into 4 KB of LDS.  Rotations apply
+// both, two operations per real part: the specialised kernels' scaled form
+// (jit.cpp) takes one, but its products of cosines would round once more per
+// rotation and need bounds wherever two amplitudes meet in a product.
 //
 // Bound by instruction latency for a few hundred states, then by vector
-// issue (about 590 vector instructions per HEA layer of 8 qubits).  Measured,
-// 8 qubits, 10 layers of (R_y, R_z, CNOT chain): one state 153 -> 29 us, 2000
-// states 763 -> 43 us, 16,000 states 234 us; 4 qubits, 3 layers, one state
-// 26 -> 11 us.  Before: a pass over LDS, a barrier and a sincos in every
-// thread for each op (still the route of complex64 tiles of this size).
+// issue.  Measured, 8 qubits, 10 layers of (R_y, R_z, CNOT chain): one state
+// 153 -> 24.5 us, 2000 states 763 -> 38.6 us; 4 qubits, 3 layers, one state
+// 26 -> 10.3 us.  Before: a pass over LDS, a barrier and a sincos in every
+// thread for each op (still the route of complex64 tiles of this size).  In
+// the scaled form: 29, 43 and 11 us, and states a fifth further from an 80-bit
+// evolution (8 qubits, 10 layers, rms: HEA 1.06e-15, now 0.82e-15; XXZ, whose
+// gates share angles, 2.26e-15, now 1.63e-15).
 // Tried and slower: one dispatch case per op and register bit on 16
 // amplitudes per lane (143 us for the 2000 states: the joins of some 90 cases
 // move the whole register file), and one generic op at a time with partners
@@ -1231,31 +1235,32 @@ __device__ __forceinline__ double sign_flip(double x, uint32_t s) {
   return __hiloint2double(int(uint32_t(__double2hiint(x)) ^ (s << 31)), __double2loint(x));
 }
 
-// R_y (REAL) or R_x with t = tan(a/2) on lane bit B
+// R_y (REAL) or R_x on lane bit B, r = (sin, cos) of half the angle
 template <int B, bool REAL, int N>
-__device__ __forceinline__ void wave_lane_rot(double2 (&a)[N], double t, int lane) {
-  const double u = REAL ? (((lane >> B) & 1) ? t : -t) : t;
+__device__ __forceinline__ void wave_lane_rot(double2 (&a)[N], double2 r, int lane) {
+  const double u = REAL ? (((lane >> B) & 1) ? r.x : -r.x) : r.x, c = r.y;
 #pragma unroll
   for (int v = 0; v < N; ++v) {
     const double2 p = xor_lane<(1 << B)>(a[v]);
-    if constexpr (REAL) a[v] = double2{fma(u, p.x, a[v].x), fma(u, p.y, a[v].y)};
-    else a[v] = double2{fma(u, p.y, a[v].x), fma(-u, p.x, a[v].y)};
+    if constexpr (REAL) a[v] = double2{fma(u, p.x, c * a[v].x), fma(u, p.y, c * a[v].y)};
+    else a[v] = double2{fma(u, p.y, c * a[v].x), fma(-u, p.x, c * a[v].y)};
   }
 }
 
 // the same on register bit B
 template <int B, bool REAL, int N>
-__device__ __forceinline__ void wave_reg_rot(double2 (&a)[N], double t) {
+__device__ __forceinline__ void wave_reg_rot(double2 (&a)[N], double2 r) {
+  const double t = r.x, c = r.y;
 #pragma unroll
   for (int v = 0; v < N; ++v) {
     if ((v >> B) & 1) continue;
     const double2 x = a[v], y = a[v | (1 << B)];
     if constexpr (REAL) {
-      a[v] = double2{fma(-t, y.x, x.x), fma(-t, y.y, x.y)};
-      a[v | (1 << B)] = double2{fma(t, x.x, y.x), fma(t, x.y, y.y)};
+      a[v] = double2{fma(-t, y.x, c * x.x), fma(-t, y.y, c * x.y)};
+      a[v | (1 << B)] = double2{fma(t, x.x, c * y.x), fma(t, x.y, c * y.y)};
     } else {
-      a[v] = double2{fma(t, y.y, x.x), fma(-t, y.x, x.y)};
-      a[v | (1 << B)] = double2{fma(t, x.y, y.x), fma(-t, x.x, y.y)};
+      a[v] = double2{fma(t, y.y, c * x.x), fma(-t, y.x, c * x.y)};
+      a[v | (1 << B)] = double2{fma(t, x.y, c * y.x), fma(-t, x.x, c * y.y)};
     }
   }
 }
@@ -1271,7 +1276,6 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
                                           const double2 *__restrict__ init_tab, int n, int s, int n_sweeps,
                                           double2 *lds, double *__restrict__ meas = nullptr) {
   constexpr int N = 1 << RB;
-  constexpr double cmin = 1e-20, rescale = 1e-100;
   constexpr int NANG = pqs::kWaveAngles;
   const int lane = threadIdx.x;
   const int k = sw.k, lt = k - RB, T = 1 << lt;
@@ -1352,7 +1356,6 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
     }
   }
 
-  double fs = 1.0;
   auto field = [](uint32_t v, int i) { return uint32_t(__builtin_amdgcn_readlane(int(v), i)); };
   // the lane's part of the parity of j & z and base & zg
   auto lane_parity = [&](uint32_t zl, uint64_t zg) -> uint32_t {
@@ -1395,36 +1398,24 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
       for (int b = 0; b < 6; ++b) cur[b] = ca[b];
       auto layer = [&](auto real) {
         constexpr bool RE = decltype(real)::value;
-        if (lt > 0) wave_lane_rot<0, RE>(a, cur[0].x, lane), fs *= cur[0].y;
-        if (lt > 1) wave_lane_rot<1, RE>(a, cur[1].x, lane), fs *= cur[1].y;
-        if (lt > 2) wave_lane_rot<2, RE>(a, cur[2].x, lane), fs *= cur[2].y;
-        if (lt > 3) wave_lane_rot<3, RE>(a, cur[3].x, lane), fs *= cur[3].y;
+        if (lt > 0) wave_lane_rot<0, RE>(a, cur[0], lane);
+        if (lt > 1) wave_lane_rot<1, RE>(a, cur[1], lane);
+        if (lt > 2) wave_lane_rot<2, RE>(a, cur[2], lane);
+        if (lt > 3) wave_lane_rot<3, RE>(a, cur[3], lane);
         // lane bits 4 and 5 trade places with the top register bit
         if (lt > 4) {
-          fs *= cur[4].y;
           lane_reg_swap<4, RB>(a);
-          wave_reg_rot<RB - 1, RE>(a, cur[4].x);
+          wave_reg_rot<RB - 1, RE>(a, cur[4]);
           lane_reg_swap<4, RB>(a);
         }
         if (lt > 5) {
-          fs *= cur[5].y;
           lane_reg_swap<5, RB>(a);
-          wave_reg_rot<RB - 1, RE>(a, cur[5].x);
+          wave_reg_rot<RB - 1, RE>(a, cur[5]);
           lane_reg_swap<5, RB>(a);
         }
-        double2 c = ca[lt];
-        fs *= c.y;
-        wave_reg_rot<0, RE>(a, c.x);
-        if constexpr (RB > 1) {
-          c = ca[lt + 1];
-          fs *= c.y;
-          wave_reg_rot<1, RE>(a, c.x);
-        }
-        if constexpr (RB > 2) {
-          c = ca[lt + 2];
-          fs *= c.y;
-          wave_reg_rot<2, RE>(a, c.x);
-        }
+        wave_reg_rot<0, RE>(a, ca[lt]);
+        if constexpr (RB > 1) wave_reg_rot<1, RE>(a, ca[lt + 1]);
+        if constexpr (RB > 2) wave_reg_rot<2, RE>(a, ca[lt + 2]);
       };
       if (code == pqs::kWLayerRy) layer(std::true_type{});
       else layer(std::false_type{});
@@ -1438,21 +1429,19 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
       for (int b = 0; b < 6; ++b)
         if (b < lt) {
           const double2 c = ca[b];
-          fs *= c.y;
           const double t = ((l >> b) & 1) ? -c.x : c.x;
-          w = double2{fma(t, w.y, w.x), fma(-t, w.x, w.y)};
+          w = double2{fma(t, w.y, c.y * w.x), fma(-t, w.x, c.y * w.y)};
         }
       double2 ph[N];
       ph[0] = w;
 #pragma unroll
       for (int b = 0; b < RB; ++b) {
         const double2 c = ca[lt + b];
-        fs *= c.y;
 #pragma unroll
         for (int v = 0; v < (1 << b); ++v) {
           const double2 y = ph[v];
-          ph[v] = double2{fma(c.x, y.y, y.x), fma(-c.x, y.x, y.y)};
-          ph[v | (1 << b)] = double2{fma(-c.x, y.y, y.x), fma(c.x, y.x, y.y)};
+          ph[v] = double2{fma(c.x, y.y, c.y * y.x), fma(-c.x, y.x, c.y * y.y)};
+          ph[v | (1 << b)] = double2{fma(-c.x, y.y, c.y * y.x), fma(c.x, y.x, c.y * y.y)};
         }
       }
 #pragma unroll
@@ -1477,20 +1466,11 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
             half_turn(sn, cs);
             f = 0.5 * pscale[m];
           }
-          if (fabs(cs) < cmin) cs = cs < 0.0 ? -cmin : cmin;
-          mine_tab[l + m * T] = double2{sn / cs, f * cs};
+          mine_tab[l + m * T] = double2{f * sn, f * cs};
         }
       }
       wave_fence();
       ahead(c + int(x));
-      continue;
-    }
-    if (code == pqs::kWCheck) {
-      if (fabs(fs) < rescale) {
-#pragma unroll
-        for (int v = 0; v < N; ++v) a[v] = double2{a[v].x * fs, a[v].y * fs};
-        fs = 1.0;
-      }
       continue;
     }
     const uint64_t zg = uint64_t(field(held[1].x, i)) | (uint64_t(field(held[1].y, i)) << 32);
@@ -1526,12 +1506,11 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
     const uint32_t xr = x >> lt, zl = z & uint32_t(T - 1), zr = z >> lt;
     if (code == pqs::kWPhase) {
       const double2 ca = mine_tab[ang];
-      fs *= ca.y;
       const double t0 = sign_flip(ca.x, lane_parity(zl, zg) ^ uint32_t(c));
 #pragma unroll
       for (int v = 0; v < N; ++v) {
         const double t = sign_flip(t0, reg_parity(v, zr));
-        a[v] = double2{fma(t, a[v].y, a[v].x), fma(-t, a[v].x, a[v].y)};
+        a[v] = double2{fma(t, a[v].y, ca.y * a[v].x), fma(-t, a[v].x, ca.y * a[v].y)};
       }
       continue;
     }
@@ -1549,14 +1528,13 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
       double2 p[N];
       put();
       partner(p, x);
-      fs *= ca.y;
       const double t0 = sign_flip(ca.x, lane_parity(zl, zg) ^ uint32_t(c));
 #pragma unroll
       for (int v = 0; v < N; ++v) {
         const double t = sign_flip(t0, reg_parity(v, zr));
         // the imaginary form is the real one on (p.y, -p.x)
         const double px = code == pqs::kWRotI ? p[v].y : p[v].x, py = code == pqs::kWRotI ? -p[v].x : p[v].y;
-        a[v] = double2{fma(t, px, a[v].x), fma(t, py, a[v].y)};
+        a[v] = double2{fma(t, px, ca.y * a[v].x), fma(t, py, ca.y * a[v].y)};
       }
       continue;
     }
@@ -1603,7 +1581,7 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
           re = fma(a[v].x, px, fma(a[v].y, py, re));
           im = fma(a[v].x, py, fma(-a[v].y, px, im));
         }
-        double y = (d->m[0] * re - d->m[1] * im) * fs * fs;
+        double y = d->m[0] * re - d->m[1] * im;
         y = sign_flip(y, lane_parity(zl, 0) ^ (uint32_t(__popc(x & z)) & 1));
         for (int q = 1; q < T; q <<= 1) y += __shfl_xor(y, q);
         if (live && l == 0) meas[tangent] = y;
@@ -1644,7 +1622,7 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
       const double2 ct = mine_tab[ang], cp = int(z) >= 0 ? mine_tab[z] : double2{0, 1};
       double dg, of;
       double2 ph;
-      fsim_coef(code == pqs::kWFsim ? 0 : dops[c].pauli, ct.x * ct.y, ct.y, cp.x * cp.y, cp.y, dg, of, ph);
+      fsim_coef(code == pqs::kWFsim ? 0 : dops[c].pauli, ct.x, ct.y, cp.x, cp.y, dg, of, ph);
       double2 p[N];
       put();
       partner(p, x);
@@ -1685,7 +1663,7 @@ __device__ __forceinline__ void wave_body(const DevSweep &sw, const pqs::WaveOp 
   }
   if (live) {
 #pragma unroll
-    for (int v = 0; v < N; ++v) dst[offset(v)] = double2{a[v].x * fs, a[v].y * fs};
+    for (int v = 0; v < N; ++v) dst[offset(v)] = a[v];
   }
 }
 

@@ -109,9 +109,7 @@ static void masks_of(int n, const pqs_op &o, qmask &active, qmask &diag) {
 // the deferred ones are gathered into one record: equal rotations on distinct
 // qubits (a layer record, where they cover at least half of the tile), and
 // runs of CNOTs (one index map).  An angle refill covers the next kWaveAngles
-// angles per lane of a tile; ops refer to it by their position in it.  A
-// growth check every 10 rotations applies the accumulated scale early (the
-// scaled rotation form of the specialised kernels, with their bound).
+// angles per lane of a tile; ops refer to it by their position in it.
 static void wave_stream(pqs_plan &p, const DevSweep &ds) {
   p.wave_begin.push_back(int(p.dev_wave.size()));
   p.angle_begin.push_back(int(p.dev_angles.size()));
@@ -123,7 +121,7 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
     p.dev_wave.push_back(w);
     return p.dev_wave.back();
   };
-  int n_ang = 0, refill_at = -1, refill_first = 0, rot = 0;
+  int n_ang = 0, refill_at = -1, refill_first = 0;
   // room for `need` angles in the current refill
   auto reserve = [&](int need) {
     if (refill_at >= 0 && n_ang + need - refill_first <= per_refill) return;
@@ -160,21 +158,13 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
     w.tangent = tangent;
     return w;
   };
-  auto rotations = [&](int count) {  // at most 10 between two checks
-    if (rot + count > 10) {
-      emit(kWCheck);
-      rot = 0;
-    }
-    rot += count;
-  };
   auto single = [&](int o) {
     const DevOp &d = p.dev_ops[size_t(o)];
     const uint32_t b0 = d.t0 >= 0 ? 1u << d.t0 : 0, b1 = d.t1 >= 0 ? 1u << d.t1 : 0;
     const uint64_t h0 = d.t0 < 0 && d.g0 >= 0 ? uint64_t(1) << d.g0 : 0;
     const uint64_t h1 = d.t1 < 0 && d.g1 >= 0 ? uint64_t(1) << d.g1 : 0;
-    // exp(-i a/2 P) = cos (1 - i t P), P = i^y (-1)^{(j ^ x).z} X^x on a[j ^ x]
+    // exp(-i a/2 P) = cos - i sin P, P = i^y (-1)^{(j ^ x).z} X^x on a[j ^ x]
     auto rotation = [&](uint32_t x, uint32_t z, uint64_t zg, int y) {
-      rotations(1);
       reserve(1);
       const uint16_t a = angle(d.scale, d.offset, d.slot, d.shift);
       WaveOp &w = emit(!x ? kWPhase : y & 1 ? kWRotR : kWRotI);
@@ -217,7 +207,7 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
       case PQS_OP_FSIM:
       case PQS_OP_GEN_FSIM: {
         reserve(2);
-        // doubled: the table holds (tan, cos) of half of each angle
+        // doubled: the table holds (sin, cos) of half of each angle
         const uint16_t a = angle(2 * d.scale, 2 * d.offset, d.slot, kNoShift);
         const uint32_t f = d.slot2 >= 0 ? angle(2.0, 0.0, d.slot2, kNoShift) : 0xffffffffu;
         WaveOp &w = d.kind == PQS_OP_FSIM ? emit(kWFsim) : generator(kWGenFsim, d.tangent);
@@ -308,7 +298,6 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
       rest.assign(rem.begin() + 1, rem.end());
     }
     if (layer && 2 * int(got.size()) >= k) {
-      rotations(k);
       reserve(k);
       int first = -1;
       for (int t = 0; t < k; ++t) {

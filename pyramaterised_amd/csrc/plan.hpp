@@ -131,15 +131,14 @@ constexpr int wave_reg_bits(int k) { return k == 1 ? 1 : k == 9 ? 3 : 2; }
 enum WaveCode : int32_t {
   kWEnd = 0,
   kWRefill,   // c: first angle, x: count
-  kWCheck,    // growth check of the scaled rotations
   kWSkip,     // the next x records are generators of tangents z .. c
   kWLayerRx,  // R_x on every bit, angles ang .. ang + k - 1 (identity: angle 0)
   kWLayerRy,
   kWLayerRz,
   kWMap,      // a'[j] = a[m(j)], m linear: the masks of m on bits 0, 1, .. are the
               // 16-bit halves of x, z, zg, c
-  kWRotI,     // a - (+) i t (-1)^{j.z} a[j ^ x] (c: 1 flips the sign)
-  kWRotR,     // a + (-) t (-1)^{j.z} a[j ^ x] (c: 1 flips the sign)
+  kWRotI,     // cos a - (+) i sin (-1)^{j.z} a[j ^ x] (c: 1 flips the sign)
+  kWRotR,     // cos a + (-) sin (-1)^{j.z} a[j ^ x] (c: 1 flips the sign)
   kWPhase,    // kWRotI with x = 0
   kWCx,       // control outside the tile: a[j ^ x] where zg's bit is set
   kWCz,       // -1 where all bits of z and zg are set
