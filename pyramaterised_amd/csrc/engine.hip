@@ -2797,12 +2797,20 @@ int plan_wait(pqs_plan *p, hipStream_t st) {
   return PQS_OK;
 }
 
+// Measurement plans run with pqs_adjoint alone: their specialised sweeps take
+// one argument more than the others, and their records name outputs.  Asked by
+// every other entry point, also by those that find the plan on the device.
+int refuse_meas(const pqs_plan *p) {
+  return p->n_meas ? fail(PQS_ERR_UNSUPPORTED, "a plan with measurements runs with pqs_adjoint") : PQS_OK;
+}
+
 // The plan's arrays on the context's device, copied at its first launch in
 // that launch's stream order (no host wait).
 int plan_upload(pqs_ctx *ctx, pqs_plan *p, hipStream_t st, bool meas = false) {
   if (p->dev_device >= 0 && p->dev_device != ctx->device)
     return fail(PQS_ERR_ARG, "plan already bound to another device");
-  if (p->n_meas && !meas) return fail(PQS_ERR_UNSUPPORTED, "a plan with measurements runs with pqs_adjoint");
+  if (!meas)
+    if (const int rc = refuse_meas(p)) return rc;
   if (p->d_ops) return plan_wait(p, st);
   if (!p->up_event) {
     hipEvent_t ev;
@@ -3690,6 +3698,7 @@ int pqs_run_table(pqs_ctx *ctx, pqs_plan *p, const void *table, int64_t batch, c
   Range rg_("pqs_run_table");
   if (!ctx || !p || !table) return fail(PQS_ERR_ARG, "NULL ctx, plan or table");
   if (batch <= 0) return fail(PQS_ERR_ARG, "batch must be positive");
+  if (const int rc = refuse_meas(p)) return rc;
   if (!p->d_ops || p->dev_device != ctx->device) return fail(PQS_ERR_ARG, "plan not on this device: table it first");
   DeviceGuard g(ctx->device);
   hipStream_t st = (hipStream_t)stream;
@@ -3714,6 +3723,7 @@ int pqs_run_batch_noalloc(pqs_ctx *ctx, pqs_plan *p, void *states, int64_t state
   if (init < 0 || init > 2) return fail(PQS_ERR_ARG, "init must be 0, 1 or 2");
   if (init == 2 && !init_tab) return fail(PQS_ERR_ARG, "product init needs an init table");
   if (p->n_tangents > 0) return fail(PQS_ERR_UNSUPPORTED, "no-allocation runs take plans without tangents");
+  if (const int rc = refuse_meas(p)) return rc;
   if (!ctx->scratch) return fail(PQS_ERR_UNSUPPORTED, "no scratch array on this device");
   if (!p->d_ops || p->dev_device != ctx->device)
     return fail(PQS_ERR_ARG, "plan not on this device: run it once with pqs_run_batch first");

@@ -1,0 +1,51 @@
+"""Entry points refuse what they cannot run: measurement plans outside
+pqs_adjoint, also once the plan is on the device, and host parameter rows
+shorter than the plan's slots; the energy gradient without room for the
+one-plan pass."""
+import ctypes as C
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def pyqc():
+    import pyramaterised_amd
+    return pyramaterised_amd
+
+
+def _hea(pyqc, n, layers=2):
+    from pyramaterised_amd import templates as T
+    qc = pyqc.PQC(n)
+    qc.add_layers(T.clifford_HE_layers(layers, n))
+    return qc
+
+
+@pytest.mark.parametrize("n", [5, 10])
+def test_measurement_plans_run_with_pqs_adjoint_alone(pyqc, n):
+    from pyramaterised_amd import _lib as L
+    from pyramaterised_amd import adjoint
+    from pyramaterised_amd import engine as E
+    lib, ctx = L.lib(), E.context()
+    qc = _hea(pyqc, n)
+    th = np.random.default_rng(n).random(qc.n_true_params)
+    prog = adjoint.program(qc)
+    prog._want_jit = True
+    adjoint.energy_and_gradient(qc, th)  # the plan is on the device now
+    plan, dim = prog.fused_plan(), 1 << (n + 1)
+    out = torch.full((2, dim), 7.0, dtype=torch.complex128, device="cuda")
+    alt = torch.empty_like(out)
+    p = E.to_device(th)
+    table = torch.zeros(lib.pqs_batch_table_bytes(2), dtype=torch.uint8, device="cuda")
+    st = E.stream_ptr()
+    tail = (1, None, E.ptr(alt))
+    for rc in (lib.pqs_run_batch_noalloc(ctx.handle, plan.handle, E.ptr(out), dim, 2, E.ptr(p), 0, *tail, None, st),
+               lib.pqs_run_table(ctx.handle, plan.handle, E.ptr(table), 2, None, st),
+               lib.pqs_batch_table(ctx.handle, plan.handle, E.ptr(out), dim, 2, E.ptr(p), 0, *tail, E.ptr(table), st),
+               lib.pqs_run_batch(ctx.handle, plan.handle, E.ptr(out), dim, 2, E.ptr(p), 0, None, 1, None, None, st),
+               lib.pqs_jacobian(ctx.handle, plan.handle, E.ptr(p), 1, None, None, E.ptr(out), None, st)):
+        assert rc == L.PQS_ERR_UNSUPPORTED
+    assert bool((out == 7.0).all())
