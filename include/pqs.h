@@ -322,8 +322,9 @@ int pqs_run_batch_noalloc(pqs_ctx *ctx, pqs_plan *plan, void *states_dev, int64_
                           void *alt_dev, const void *init_table_dev, void *stream);
 
 /* pqs_run_batch with the parameters (batch rows of n_params doubles, at least
- * one) and the product table in host memory: they travel with the instance
- * table in one upload.  For calls whose inputs are small and start on the host;
+ * one and more than the largest slot of the plan's ops, else PQS_ERR_ARG) and
+ * the product table in host memory: they travel with the instance table in
+ * one upload.  For calls whose inputs are small and start on the host;
  * the inputs occupy context workspace. */
 int pqs_run_batch_host(pqs_ctx *ctx, pqs_plan *plan, void *states_dev, int64_t state_stride, int64_t batch,
                        const double *params_host, int64_t n_params, const int32_t *tangents_host, int32_t init,
@@ -338,8 +339,8 @@ int pqs_jacobian(pqs_ctx *ctx, pqs_plan *plan, const double *params_dev,
                  int32_t init, const void *src_dev, const void *init_table_dev,
                  void *psi_dev, void *jac_dev, void *stream);
 
-/* pqs_jacobian with the parameters (n_params doubles, at least one) and the
- * product table in host memory, as pqs_run_batch_host. */
+/* pqs_jacobian with the parameters (n_params doubles) and the product table in
+ * host memory, as pqs_run_batch_host. */
 int pqs_jacobian_host(pqs_ctx *ctx, pqs_plan *plan, const double *params_host, int64_t n_params, int32_t init,
                       const void *src_dev, const void *init_table_host, void *psi_dev, void *jac_dev, void *stream);
 

@@ -3177,6 +3177,14 @@ struct HostIn {
   }
 };
 
+// Every slot of the plan within the rows of n_params parameters.
+static int check_slots(const pqs_plan *p, int64_t n_params) {
+  if (n_params > p->max_slot) return PQS_OK;
+  const std::string what = "the plan reads parameter " + std::to_string(p->max_slot) + " of rows of " +
+                           std::to_string(n_params);
+  return fail(PQS_ERR_ARG, what.c_str());
+}
+
 // Partials per pair of a batch's overlaps (0: none wanted): per last-sweep tile
 // where the last sweep's pair kernel forms them (fused), else per chunk.
 static int64_t pair_chunks(const pqs_ctx *ctx, const pqs_plan *p, bool pairs, bool &fused) {
@@ -3449,6 +3457,7 @@ int pqs_run_batch_host(pqs_ctx *ctx, pqs_plan *p, void *states, int64_t state_st
   Range rg_("pqs_run_batch_host");
   if (!ctx || !p || !states || !params_host) return fail(PQS_ERR_ARG, "NULL ctx, plan, states or parameters");
   if (batch < 0 || n_params < 1) return fail(PQS_ERR_ARG, "negative batch or no parameters");
+  if (const int rc = check_slots(p, n_params)) return rc;
   if (batch == 0) return PQS_OK;
   if (state_stride < (int64_t(1) << p->n)) return fail(PQS_ERR_ARG, "state stride below 2^N");
   if (init < 0 || init > 2) return fail(PQS_ERR_ARG, "init must be 0, 1 or 2");
@@ -3888,6 +3897,7 @@ int pqs_jacobian_host(pqs_ctx *ctx, pqs_plan *p, const double *params_host, int6
                       const void *src, const void *init_tab_host, void *psi, void *jac, void *stream) {
   Range rg_("pqs_jacobian_host");
   if (!ctx || !p || !params_host || n_params < 1) return fail(PQS_ERR_ARG, "NULL ctx, plan or parameters");
+  if (const int rc = check_slots(p, n_params)) return rc;
   const bool table = init == 2 && init_tab_host;
   const HostIn in{params_host, n_params, table ? init_tab_host : nullptr,
                   table ? size_t(2 * p->n) * amp_bytes(p->dtype) : 0};

@@ -369,6 +369,7 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
   p.n_tangents = 0;
   p.n_sub = 0;
   p.n_meas = 0;
+  p.max_slot = -1;
 
   bool pair_touched = false;
   for (int i = 0; i < n_ops; ++i) {
@@ -378,6 +379,10 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
     pair_touched = pair_touched || ops[i].q0 == 0 || (is_two_qubit(ops[i].kind) && ops[i].q1 == 0) ||
                    ((ops[i].kind == PQS_OP_GEN || ops[i].kind == PQS_OP_MEAS) && ops[i].q1 == 0);
     if (ops[i].tangent >= 0) p.n_tangents = std::max(p.n_tangents, ops[i].tangent + 1);
+    const bool fsim = ops[i].kind == PQS_OP_FSIM || ops[i].kind == PQS_OP_GEN_FSIM;
+    if (fsim || (ops[i].kind >= PQS_OP_RX && ops[i].kind <= PQS_OP_RZ) ||
+        (ops[i].kind >= PQS_OP_RXX && ops[i].kind <= PQS_OP_RZZ))
+      p.max_slot = std::max({p.max_slot, ops[i].slot, fsim ? ops[i].slot2 : -1});
   }
 
   if (p.n_meas) {

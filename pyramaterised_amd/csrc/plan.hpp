@@ -178,6 +178,7 @@ struct pqs_plan {
   // the first runs as a sub-tangent n_tangents.. whose state is summed into
   // its parent's row at the end of a run.  n_sub counts all of them.
   int n_sub = 0;
+  int max_slot = -1;  // largest parameter index that an op reads
   int n_meas = 0;  // PQS_OP_MEAS ops: qubit 0 is then in every tile
   std::vector<int> tangent_parent;  // per tangent / sub-tangent: caller tangent
   std::vector<pqs_op> src_ops;

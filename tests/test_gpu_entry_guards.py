@@ -49,3 +49,27 @@ def test_measurement_plans_run_with_pqs_adjoint_alone(pyqc, n):
                lib.pqs_jacobian(ctx.handle, plan.handle, E.ptr(p), 1, None, None, E.ptr(out), None, st)):
         assert rc == L.PQS_ERR_UNSUPPORTED
     assert bool((out == 7.0).all())
+
+
+@pytest.mark.parametrize("kind", ["rotations", "fsim"])
+def test_host_rows_cover_the_plan_slots(pyqc, kind):
+    from pyramaterised_amd import engine as E
+    n = 4
+    if kind == "rotations":
+        qc = _hea(pyqc, n)
+    else:  # the largest slot is fSim's phi
+        qc = pyqc.PQC(n)
+        qc.add_layer([pyqc.R_y(0, n), pyqc.fSim([1, 2], n)])
+    P = qc.n_true_params
+    plan, full = E.Plan(n, qc.ops()), E.Plan(n, qc.ops(True))
+    th = np.random.default_rng(1).random((2, P))
+    assert bool(torch.isfinite(torch.view_as_real(E.run(plan, th, qc.init()))).all())
+    for short in (th[:, :P - 1], th[0, :P - 1], np.zeros(0)):
+        with pytest.raises(E.EngineError):
+            E.run(plan, short, qc.init())
+    E.jacobian(full, th[0], qc.init())
+    with pytest.raises(E.EngineError):
+        E.jacobian(full, th[0, :P - 1], qc.init())
+    # a longer vector is fine: the plan reads its slots
+    longer = np.concatenate([th, np.full((2, 3), 9.0)], axis=1)
+    assert torch.equal(E.run(plan, longer, qc.init()), E.run(plan, th, qc.init()))
