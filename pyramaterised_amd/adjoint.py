@@ -179,6 +179,11 @@ class AdjointProgram:
     # partials of the measurements (one per tile and term) above this many
     # bytes: the point-by-point form
     FUSED_PARTIAL_BYTES = 4 << 30
+    # the same for the evolved pair and its second buffer, which the context's
+    # workspace then keeps (the point-by-point form evolves the pair in place):
+    # 32 GiB is 29 qubits, a ninth of the card; at 32 qubits the two would
+    # take 256 GiB next to the pair's 128
+    FUSED_WORKSPACE_BYTES = 32 << 30
 
     def fused_ops(self):
         """The backward pass as one op list on n + 1 qubits (qubit 0: lambda
@@ -213,7 +218,9 @@ class AdjointProgram:
             self._uses += 1
             if k >= 10 and not (self._want_jit or (self._may_jit and self._uses >= PASSES_BEFORE_JIT)):
                 return None
-            if k >= 4 and (k < 10 or (8 * self.n_terms << (self.n + 1 - k)) <= self.FUSED_PARTIAL_BYTES):
+            fits = (8 * self.n_terms << (self.n + 1 - k)) <= self.FUSED_PARTIAL_BYTES and \
+                (2 * 16 << (self.n + 1)) <= self.FUSED_WORKSPACE_BYTES
+            if k >= 4 and (k < 10 or fits):
                 self._fused = E.Plan(self.n + 1, self.fused_ops(), dtype=self.dtype, tile_bits=k, low_bits=min(3, k),
                                      flags=L.PQS_PLAN_ROLLING)
                 if k >= 10:
@@ -234,12 +241,15 @@ class AdjointProgram:
         ctx = E.context()
         th = E._params_tensor(params, pair.device)
         plan = self.fused_plan()
+        real = None
         if plan is not None:
             vals = torch.empty(self.n_terms, dtype=torch.float64, device=pair.device)
-            E.check(L.lib().pqs_adjoint(ctx.handle, plan.handle, E.ptr(th), E.ptr(pair), E.ptr(vals), E.stream_ptr()))
-            E._keepalive(th, pair)
-            real = vals.cpu().numpy()
-        else:
+            rc = L.lib().pqs_adjoint(ctx.handle, plan.handle, E.ptr(th), E.ptr(pair), E.ptr(vals), E.stream_ptr())
+            if rc != L.PQS_ERR_NOMEM:  # no room for its workspace: the form without
+                E.check(rc)
+                E._keepalive(th, pair)
+                real = vals.cpu().numpy()
+        if real is None:
             out = torch.empty((max(1, self.n_terms), 2), dtype=torch.float64, device=pair.device)
             off = 0
             for step, nt, xs, zs, cs, _ in self.steps:

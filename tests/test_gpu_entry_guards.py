@@ -73,3 +73,30 @@ def test_host_rows_cover_the_plan_slots(pyqc, kind):
     # a longer vector is fine: the plan reads its slots
     longer = np.concatenate([th, np.full((2, 3), 9.0)], axis=1)
     assert torch.equal(E.run(plan, longer, qc.init()), E.run(plan, th, qc.init()))
+
+
+def test_gradient_without_room_for_the_one_plan_pass(pyqc, monkeypatch):
+    """A failed workspace reservation takes the point-by-point pass: both
+    round each amplitude by a few eps per gate, gradients of size <= 4."""
+    from pyramaterised_amd import _lib as L
+    from pyramaterised_amd import adjoint
+    n = 6
+    qc = _hea(pyqc, n)
+    th = np.random.default_rng(3).random(qc.n_true_params)
+    e0, g0 = adjoint.energy_and_gradient(qc, th)
+    real = L.lib()
+
+    class NoRoom:
+        calls = 0
+
+        def __getattr__(self, name):
+            return getattr(real, name)
+
+        def pqs_adjoint(self, *args):
+            NoRoom.calls += 1
+            return L.PQS_ERR_NOMEM
+
+    monkeypatch.setattr(adjoint.L, "lib", lambda: NoRoom())
+    e1, g1 = adjoint.energy_and_gradient(qc, th)
+    assert NoRoom.calls == 1
+    assert e1 == e0 and np.max(np.abs(g0 - g1)) < 1e-12
