@@ -264,38 +264,40 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
     }
   };
   auto in_tile = [&](const DevOp &d) { return d.t0 >= 0 && (d.g1 < 0 || d.t1 >= 0); };
-  std::vector<int> rem, rest, got;
-  for (int o = ds.op_begin; o < ds.op_end; ++o) rem.push_back(o);
-  while (!rem.empty()) {
-    const int kind = p.dev_ops[size_t(rem[0])].kind;
+  uint64_t tile = 0;
+  for (int b = 0; b < k; ++b) tile |= tpos[b];
+  // ops not yet in a record, linked in circuit order: a gathering looks ahead
+  // only until every bit of the tile is blocked for its kind, about a layer, so
+  // the stream takes time linear in the ops
+  std::vector<int> next(size_t(ds.op_end - ds.op_begin));
+  for (int o = ds.op_begin; o < ds.op_end; ++o) next[size_t(o - ds.op_begin)] = o + 1;
+  auto after = [&](int o) -> int & { return next[size_t(o - ds.op_begin)]; };
+  std::vector<int> got;
+  for (int head = ds.op_begin; head < ds.op_end; head = after(head)) {
+    const int kind = p.dev_ops[size_t(head)].kind;
     const bool layer = (kind == PQS_OP_RX || kind == PQS_OP_RY || kind == PQS_OP_RZ) &&
-                       in_tile(p.dev_ops[size_t(rem[0])]);
-    const bool map = kind == PQS_OP_CX && in_tile(p.dev_ops[size_t(rem[0])]);
-    got.assign(1, rem[0]);
-    rest.clear();
+                       in_tile(p.dev_ops[size_t(head)]);
+    const bool map = kind == PQS_OP_CX && in_tile(p.dev_ops[size_t(head)]);
+    got.assign(1, head);
     if (layer || map) {
       uint64_t blocked_any = 0, blocked_act = 0;
-      uint32_t taken = layer ? 1u << p.dev_ops[size_t(rem[0])].t0 : 0;
-      for (size_t i = 1; i < rem.size(); ++i) {
-        const DevOp &d = p.dev_ops[size_t(rem[i])];
+      uint32_t taken = layer ? 1u << p.dev_ops[size_t(head)].t0 : 0;
+      for (int last = head, o = after(head); o < ds.op_end; o = after(last)) {
+        const DevOp &d = p.dev_ops[size_t(o)];
         uint64_t act, all;
-        masks(rem[i], act, all);
+        masks(o, act, all);
         const bool free = !(act & blocked_any) && !(all & blocked_act);
         if (free && d.kind == kind && in_tile(d) && (map || !((taken >> d.t0) & 1))) {
-          got.push_back(rem[i]);
+          got.push_back(o);
           if (layer) taken |= 1u << d.t0;
+          after(last) = after(o);
         } else {
-          rest.push_back(rem[i]);
+          last = o;
           blocked_any |= all;
           blocked_act |= act;
-          if (blocked_act == ~uint64_t(0)) {  // nothing further can pass
-            rest.insert(rest.end(), rem.begin() + long(i) + 1, rem.end());
-            break;
-          }
+          if (((kind == PQS_OP_RZ ? blocked_act : blocked_act | blocked_any) & tile) == tile) break;
         }
       }
-    } else {
-      rest.assign(rem.begin() + 1, rem.end());
     }
     if (layer && 2 * int(got.size()) >= k) {
       reserve(k);
@@ -333,7 +335,6 @@ static void wave_stream(pqs_plan &p, const DevSweep &ds) {
     } else {
       for (int o : got) single(o);
     }
-    rem.swap(rest);
   }
   // whole blocks of 64 records, and one block more that is loaded ahead
   do emit(kWEnd);
