@@ -656,26 +656,20 @@ __device__ __forceinline__ void reg_z(V (&a)[NA]) {
     if (v & (1 << B)) a[v] = cneg(a[v]);
 }
 
-// 1 - i t P (form A) or u - i P (form B) on register bits B0, B1, with P =
-// X(x)X, or Y(x)Y = X(x)X on 01, 10 and -X(x)X on 00, 11
-template <int B0, int B1, bool FB, bool YY, typename V, typename R>
-__device__ __forceinline__ void reg_rpp(V (&a)[NA], R t) {
+// c - i t P on register bits B0, B1, with P = X(x)X, or Y(x)Y = X(x)X on 01, 10
+// and -X(x)X on 00, 11.  Not in the scaled form: a shared angle's rounding would
+// enter the scale once per gate more.
+template <int B0, int B1, bool YY, typename V, typename R>
+__device__ __forceinline__ void reg_rpp(V (&a)[NA], R c, R t) {
   if constexpr (B0 != B1) {
 #pragma unroll
     for (int v = 0; v < NA; ++v) {
       const int w = v ^ (1 << B0) ^ (1 << B1);
       if (w < v) continue;
-      const bool neg = YY && !(((v >> B0) ^ (v >> B1)) & 1);
+      const R u = YY && !(((v >> B0) ^ (v >> B1)) & 1) ? -t : t;
       const V x = a[v], y = a[w];
-      if constexpr (!FB) {
-        const R u = neg ? -t : t;
-        a[v] = V{fma(u, y.y, x.x), fma(-u, y.x, x.y)};
-        a[w] = V{fma(u, x.y, y.x), fma(-u, x.x, y.y)};
-      } else {
-        const V p = neg ? V{-y.x, -y.y} : y, q = neg ? V{-x.x, -x.y} : x;
-        a[v] = V{fma(t, x.x, p.y), fma(t, x.y, -p.x)};
-        a[w] = V{fma(t, y.x, q.y), fma(t, y.y, -q.x)};
-      }
+      a[v] = V{fma(u, y.y, c * x.x), fma(-u, y.x, c * x.y)};
+      a[w] = V{fma(u, x.y, c * y.x), fma(-u, x.x, c * y.y)};
     }
   }
 }
@@ -862,7 +856,10 @@ __device__ __forceinline__ void sweep_reg_body(const DevSweep &sw, const DevOp *
       sincos(0.5 * op_angle(d, params), &sn, &cs);
       const bool turned = d->shift == in.tangent;
       if (turned) half_turn(sn, cs);
-      if (fabs(cs) >= fabs(sn)) {
+      if (d->kind == PQS_OP_RXX || d->kind == PQS_OP_RYY) {
+        r.t = turned ? 0.5 * d->scale * sn : sn;
+        r.f = cs;
+      } else if (fabs(cs) >= fabs(sn)) {
         r.t = sn / cs;
         r.f = cs;
       } else {
@@ -1025,22 +1022,14 @@ __device__ __forceinline__ void sweep_reg_body(const DevSweep &sw, const DevOp *
         }
         case PQS_OP_RXX:
           if constexpr (LDSOPS) {
-            fscale *= op.f;
-            if (fb) {
-              SW4(r0, SW4C(r1, reg_rpp<B_, C_, true, false>(a, t)));
-            } else {
-              SW4(r0, SW4C(r1, reg_rpp<B_, C_, false, false>(a, t)));
-            }
+            const R c = R(op.f);
+            SW4(r0, SW4C(r1, reg_rpp<B_, C_, false>(a, c, t)));
           }
           break;
         case PQS_OP_RYY:
           if constexpr (LDSOPS) {
-            fscale *= op.f;
-            if (fb) {
-              SW4(r0, SW4C(r1, reg_rpp<B_, C_, true, true>(a, t)));
-            } else {
-              SW4(r0, SW4C(r1, reg_rpp<B_, C_, false, true>(a, t)));
-            }
+            const R c = R(op.f);
+            SW4(r0, SW4C(r1, reg_rpp<B_, C_, true>(a, c, t)));
           }
           break;
         case PQS_OP_FSIM:
