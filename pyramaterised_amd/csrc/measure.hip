@@ -391,7 +391,7 @@ void mw_split(int n, int &M, int64_t &ncg, int &groups) {
 // 10) by one LDS round trip of the block.  Bound by FP64 adds (N per value).
 // A block keeps its state's (Re c + Im c, Im c - Re c) in LDS (N <= 12) and
 // its amplitudes in registers over the X parts it takes.  Measured: 200
-// complex128 states of 10 qubits 1255 -> 180 us (before: complex transforms
+// complex128 states of 10 qubits 1255 -> 182 us (before: complex transforms
 // bit by bit in LDS, a barrier each), about half of the FP64 add rate.
 enum { kSquare = 0, kRoot = 1, kPower = 2 };
 
@@ -402,16 +402,23 @@ __device__ __forceinline__ double magic_term(double f, double scale, double alph
   return FORM == kSquare ? a2 * a2 : pow(a2, alpha);
 }
 
-// Sum of the first M values (a power of two), in pairs: the identity's term is
-// about a quarter of a whole sum, and every addition after it in a chain would
-// round at its size.
-template <int M>
-__device__ __forceinline__ double pair_sum(double (&t)[16]) {
+// The terms of M values (a power of two), in four chains: the identity's term
+// is about a quarter of a whole sum, and every addition after it would round at
+// its size.
+template <int FORM, int M>
+__device__ __forceinline__ double magic_terms(const double (&f)[16], double scale, double alpha) {
+  constexpr int W = M < 4 ? M : 4;
+  double c[W];
 #pragma unroll
-  for (int h = M / 2; h > 0; h >>= 1)
+  for (int u = 0; u < M; ++u) {
+    const double t = magic_term<FORM>(f[u], scale, alpha);
+    c[u % W] = u < W ? t : c[u % W] + t;
+  }
 #pragma unroll
-    for (int u = 0; u < h; ++u) t[u] += t[u + h];
-  return t[0];
+  for (int h = W / 2; h > 0; h >>= 1)
+#pragma unroll
+    for (int u = 0; u < h; ++u) c[u] += c[u + h];
+  return c[0];
 }
 
 // 2^{-N/2} x: of odd N the rounding of sqrt(1/2) would be in every term alike,
@@ -527,9 +534,7 @@ __global__ __launch_bounds__(magic_block(N)) void k_magic(const typename CT<R>::
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     wht_regs<0, NLOW>(f);
-#pragma unroll
-    for (int u = 0; u < 16; ++u) f[u] = magic_term<FORM>(f[u], scale, alpha);
-    acc += pair_sum<16>(f);
+    acc += magic_terms<FORM, 16>(f, scale, alpha);
   }
   if constexpr (FORM == kRoot) acc = root_scale<N>(acc);
 #pragma unroll
@@ -579,9 +584,8 @@ __global__ __launch_bounds__(256) void k_magic_small(const typename CT<R>::V *__
         const double o = __shfl_xor(f[u], 1);
         f[u] = t ? o - f[u] : f[u] + o;
       }
-      f[u] = magic_term<FORM>(f[u], scale, alpha);
     }
-    acc = pair_sum<NR>(f);
+    acc = magic_terms<FORM, NR>(f, scale, alpha);
     if constexpr (FORM == kRoot) acc = root_scale<N>(acc);
   }
 #pragma unroll
