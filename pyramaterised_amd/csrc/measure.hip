@@ -391,7 +391,7 @@ void mw_split(int n, int &M, int64_t &ncg, int &groups) {
 // 10) by one LDS round trip of the block.  Bound by FP64 adds (N per value).
 // A block keeps its state's (Re c + Im c, Im c - Re c) in LDS (N <= 12) and
 // its amplitudes in registers over the X parts it takes.  Measured: 200
-// complex128 states of 10 qubits 1255 -> 182 us (before: complex transforms
+// complex128 states of 10 qubits 1255 -> 180 us (before: complex transforms
 // bit by bit in LDS, a barrier each), about half of the FP64 add rate.
 enum { kSquare = 0, kRoot = 1, kPower = 2 };
 
@@ -402,23 +402,14 @@ __device__ __forceinline__ double magic_term(double f, double scale, double alph
   return FORM == kSquare ? a2 * a2 : pow(a2, alpha);
 }
 
-// The terms of M values (a power of two), in four chains: the identity's term
-// is about a quarter of a whole sum, and every addition after it would round at
-// its size.
+// acc + the terms of M values, the last one first, and the X parts likewise:
+// the identity's term (f[0] of the first thread, j = 0) is about a quarter of a
+// whole sum, and every addition after it would round at its size.
 template <int FORM, int M>
-__device__ __forceinline__ double magic_terms(const double (&f)[16], double scale, double alpha) {
-  constexpr int W = M < 4 ? M : 4;
-  double c[W];
+__device__ __forceinline__ double magic_terms(double acc, const double (&f)[16], double scale, double alpha) {
 #pragma unroll
-  for (int u = 0; u < M; ++u) {
-    const double t = magic_term<FORM>(f[u], scale, alpha);
-    c[u % W] = u < W ? t : c[u % W] + t;
-  }
-#pragma unroll
-  for (int h = W / 2; h > 0; h >>= 1)
-#pragma unroll
-    for (int u = 0; u < h; ++u) c[u] += c[u + h];
-  return c[0];
+  for (int u = M - 1; u >= 0; --u) acc += magic_term<FORM>(f[u], scale, alpha);
+  return acc;
 }
 
 // 2^{-N/2} x: of odd N the rounding of sqrt(1/2) would be in every term alike,
@@ -491,7 +482,7 @@ __global__ __launch_bounds__(magic_block(N)) void k_magic(const typename CT<R>::
   }
   const double scale = 1.0 / D;
   double acc = 0;
-  for (int it = 0; it < JPB / C; ++it) {
+  for (int it = JPB / C - 1; it >= 0; --it) {
     const int j = j0 + it * C + grp;
     double f[16];
 #pragma unroll
@@ -534,7 +525,7 @@ __global__ __launch_bounds__(magic_block(N)) void k_magic(const typename CT<R>::
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
     wht_regs<0, NLOW>(f);
-    acc += magic_terms<FORM, 16>(f, scale, alpha);
+    acc = magic_terms<FORM, 16>(acc, f, scale, alpha);
   }
   if constexpr (FORM == kRoot) acc = root_scale<N>(acc);
 #pragma unroll
@@ -585,7 +576,7 @@ __global__ __launch_bounds__(256) void k_magic_small(const typename CT<R>::V *__
         f[u] = t ? o - f[u] : f[u] + o;
       }
     }
-    acc = magic_terms<FORM, NR>(f, scale, alpha);
+    acc = magic_terms<FORM, NR>(acc, f, scale, alpha);
     if constexpr (FORM == kRoot) acc = root_scale<N>(acc);
   }
 #pragma unroll
