@@ -674,25 +674,6 @@ __device__ __forceinline__ void reg_rpp(V (&a)[NA], R c, R t) {
   }
 }
 
-// fSim and its derivatives: [[d, -i o], [-i o, d]] on 01, 10 and p on 11
-template <int B0, int B1, typename V, typename R>
-__device__ __forceinline__ void reg_fsim(V (&a)[NA], R d, R o, V p) {
-  if constexpr (B0 != B1) {
-#pragma unroll
-    for (int v = 0; v < NA; ++v) {
-      if ((v >> B0) & 1) {
-        if ((v >> B1) & 1) a[v] = cmul(a[v], p);
-        continue;
-      }
-      if (!((v >> B1) & 1)) continue;
-      const int w = v ^ (1 << B0) ^ (1 << B1);
-      const V x = a[v], y = a[w];
-      a[v] = V{fma(d, x.x, o * y.y), fma(d, x.y, -o * y.x)};
-      a[w] = V{fma(d, y.x, o * x.y), fma(d, y.y, -o * x.x)};
-    }
-  }
-}
-
 // dense 4x4, BH the more significant register bit of its basis
 template <int BH, int BL, typename V>
 __device__ __forceinline__ void reg_mat2(V (&a)[NA], const V (&m)[16]) {

@@ -549,13 +549,20 @@ static void emit_sweep(const pqs_plan &p, int s, std::ostringstream &o) {
     // these sweeps is FP64 issue (3/4 of the cycles at 2 waves per SIMD, the
     // most that whole tiles leave room for, and at the card's power limit: an
     // effective 1.9 GHz); 3 waves cover the LDS round trips and barriers
-    // better: 10,000 16-qubit states of 20 HEA layers 47.5 -> 45.6 ms, 1000
-    // 12-qubit XXZ states (one 12-bit tile each, all resident at once) 312 ->
-    // 266 us, one 24-qubit state 1144 -> 1065 us; single tiles, which wait for
-    // their own barriers alone, 126 -> 128 us.  A bound of 4 waves spills: up
-    // to 2% faster at 16 qubits, 10% slower at 24.  Sweeps with measurements
-    // hold more registers and keep the whole tile (20-qubit gradient bounded
-    // to 4 waves: 6.9 against 1.9 ms), pair kernels too (a second state).
+    // better: 10,000 16-qubit states of 20 HEA layers 47.5 -> 45.6 ms, one
+    // 24-qubit state 1144 -> 1065 us; single tiles, which wait for their own
+    // barriers alone, 126 -> 128 us.  The bound of 3 (168 registers): HEA sweeps
+    // on 11 bits need 133-144, so it does nothing there; sweeps with two-qubit
+    // gates, 13-bit tiles and some of the longest spill 8-24 registers under it.
+    // Bound 2 against 3, halves in both: 1000 12-qubit XXZ states 210.5 / 196.5
+    // us, fSim 129.9 / 124.9 us (one 12-bit tile each, all resident at once),
+    // the 16-qubit Jacobian 1861 / 1851 us; slower under 3: 200 16-qubit XXZ
+    // states 815 / 836 us, 500 13-qubit HEA states 157.8 / 160.6 us.  A bound of
+    // 4 spills more: up to 2% faster at 16 qubits, 10% slower at 24.  Sweeps with
+    // measurements keep the whole tile and run at one wave per SIMD: the
+    // compiler holds the amplitudes of each measurement until its sums are
+    // folded (370-512 registers; 20-qubit gradient bounded to 4 waves: 6.9
+    // against 1.9 ms).  Pair kernels keep the whole tile for a second state.
     const bool halves = can_halve(p, s) && !pair && !nm;
     Slots slots;
     if (halves) slots = half_slots(p, ds);

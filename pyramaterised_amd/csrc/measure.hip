@@ -134,10 +134,11 @@ __device__ __forceinline__ void bit_sums(const V (&a)[16], double (&v)[16]) {
 // their own that hold those bits in registers and read the state once more;
 // all blocks of a state run on one XCD side by side, so those reads hit its
 // L2.  A block takes two chunks, the second one's loads under the first one's
-// sums (1000 states of 16 qubits: 376 us against 441 us with one chunk per
-// block).  Measured: 1000 complex128 states of 16 qubits 1320 -> 376 us, 2.8
-// TB/s of state (before: an LDS pass and a block tree per bit, partner chunks
-// re-read); 16,000 of 12 qubits 244 us, 4.3 TB/s.
+// sums (1000 states of 16 qubits in a loop over one tensor: 376 us against 441
+// us with one chunk per block).  Measured: the entanglement call on 1000
+// complex128 states of 16 qubits 1320 -> 309 us, 3.4 TB/s of state, the loop 376
+// to 385 us (before: an LDS pass and a block tree per bit, partner chunks
+// re-read); 16,000 of 12 qubits 247 us, 4.2 TB/s.
 template <typename R, int N, bool PART>
 __global__ __launch_bounds__(MB, 2) void k_mw(const typename CT<R>::V *__restrict__ states, int n, int64_t batch,
                                            int64_t ncg, int M, int groups, double *__restrict__ rho,

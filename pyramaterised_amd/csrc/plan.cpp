@@ -355,13 +355,12 @@ int build_plan(pqs_plan &p, int n, const pqs_op *ops, int n_ops, const pqs_plan_
   k = std::min(k, n);
   int low = o.low_bits > 0 ? o.low_bits : 5;
   low = std::min(low, k);
-  int block = o.block > 0 ? o.block : 512;
-  if (block != 256 && block != 512 && block != 1024) return fail(PQS_ERR_ARG, "block must be 256, 512 or 1024");
+  if (o.block > 0 && o.block != 256 && o.block != 512 && o.block != 1024)
+    return fail(PQS_ERR_ARG, "block must be 256, 512 or 1024");
 
   p.n = n;
   p.tile_bits = k;
   p.low_bits = low;
-  p.block = block;
   p.dtype = o.dtype;
   p.flags = o.flags;
   p.src_ops.assign(ops, ops + n_ops);

@@ -169,7 +169,6 @@ struct pqs_plan {
   int n = 0;
   int tile_bits = 0;
   int low_bits = 0;
-  int block = 0;
   int dtype = 0;
   int flags = 0;
   bool rolling = false;  // rolling layouts in effect (PQS_PLAN_ROLLING honoured)
