@@ -75,7 +75,8 @@ enum pqs_op_kind {
   /* Measurement of a pair of states: the plan's state is [a; b], qubit 0
    * selecting the half, and no other op touches qubit 0.  At this point of the
    * circuit Re(coef <a|P|b>), P and coef as for PQS_OP_GEN on qubits >= 1, goes
-   * to output i (the i-th such op of the list).  pqs_adjoint runs such plans. */
+   * to output i (the i-th such op of the list).  pqs_adjoint runs such plans;
+   * every other entry point returns PQS_ERR_UNSUPPORTED for them. */
   PQS_OP_MEAS = 13
 };
 

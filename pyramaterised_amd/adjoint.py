@@ -211,8 +211,9 @@ class AdjointProgram:
     def fused_plan(self):
         """The plan of ``fused_ops`` if this pass runs fused, else None.
         12-bit tiles (11 qubits and the pair's), 20 qubits, 40 layers: 19
-        sweeps in 1.08 ms; 11-bit 1.22 ms, 13-bit 1.87, 10-bit 1.35.  At 13-16
-        qubits 11-bit tiles are 6% faster."""
+        sweeps in 1.10 ms; 11-bit 1.22 ms, 13-bit 1.87, 10-bit 1.35.  At 13-16
+        qubits 11-bit tiles are 6% faster.  Building the plan compiles it, about
+        17 ms per measured term (cached on disk)."""
         if self._fused is None and self.dtype == L.PQS_C128 and self.n_terms:
             k = min(12, self.n + 1)
             self._uses += 1
