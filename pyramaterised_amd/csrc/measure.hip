@@ -449,7 +449,9 @@ __device__ __forceinline__ void wht_lane(double (&f)[16]) {
 
 constexpr int magic_block(int N) { return N >= 12 ? 512 : 256; }
 // X parts of one block: enough to reuse its amplitudes, few enough that one
-// state of 8 qubits and more still makes several blocks
+// state of 8 qubits and more still makes several blocks.  All 128 of 7 qubits in
+// one block need no second kernel: 2000 states 35.8 us, in two blocks 41.3; one
+// state 15 and 17.7
 constexpr int magic_parts(int N) { return N == 7 ? 128 : N <= 9 ? 64 : 32; }
 
 template <typename R, int N, int FORM>

@@ -48,3 +48,28 @@ def test_gradient_at_clifford_angles(pyqc, n, layers, angles):
         assert np.isfinite(g).all(), (draw, np.flatnonzero(~np.isfinite(g)))
         assert abs(e - np.real(np.vdot(psi, hpsi))) < 1e-12
         assert np.max(np.abs(g - want)) < 1e-12, draw
+
+
+@pytest.mark.parametrize("angles", ["pi", "multiples"])
+@pytest.mark.parametrize("n", [9, 11])
+def test_specialised_gradient_at_clifford_angles(pyqc, n, angles):
+    """The same with specialised sweeps (tiles of 10 bits and more)."""
+    from pyramaterised_amd import adjoint
+    from pyramaterised_amd import templates as T
+    layers = 10
+    qc = pyqc.PQC(n)
+    for layer in T.clifford_HE_layers(layers, n):
+        qc.add_layer(layer)
+    H = pyqc.PauliSum(n, {(1,) * 2 + (0,) * (n - 2): 0.5, (0,) * (n - 2) + (3,) * 2: -1.0, (2,) + (0,) * (n - 1): 0.3})
+    P = qc.n_true_params
+    prog = adjoint.program(qc)
+    rng = np.random.default_rng(n)
+    for _ in range(1 if angles == "pi" else 4):
+        th = np.full(P, np.pi) if angles == "pi" else rng.integers(0, 4, P) * (np.pi / 2)
+        prog._fused = False  # point by point
+        e0, g0 = adjoint.energy_and_gradient(qc, th, H)
+        prog._fused, prog._want_jit = None, True
+        e1, g1 = adjoint.energy_and_gradient(qc, th, H)
+        assert prog.fused_plan() is not None
+        assert np.isfinite(g1).all() and abs(e0 - e1) < 1e-12
+        assert np.max(np.abs(g0 - g1)) < 1e-12
