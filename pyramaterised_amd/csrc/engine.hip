@@ -4080,8 +4080,9 @@ int cgram_mfma(pqs_ctx *ctx, int32_t dtype, const void *a, int64_t lda, int64_t 
   // on its SIMD waits for its loads: a tenth more.  Without / with that tenth,
   // qubits x states: 16 x 2000 20.0 / 17.9 ms, 16 x 500 1404 / 1247 us, 14 x 400
   // 243 / 229, 12 x 700 182 / 170; the same splits or within 2% the other way at
-  // 11 further shapes (8 x 2000 102.5 / 104).  Measured, 1000 states of 12 qubits: 320 us for the product in
-  // 15 chunks and 95 us for their sum, 330 and 12 us in 7.
+  // 11 further shapes (8 x 2000 102.5 / 104).  Measured, 1000 states of 12
+  // qubits: 320 us for the product in 15 chunks and 95 us for their sum, 330 and
+  // 12 us in 7.
   const int64_t slots = 4 * SYWAVES * int64_t(ctx->n_cu);
   const int64_t ks_max = std::max<int64_t>(
       1, std::min<int64_t>({Kc / (2 * ring), int64_t(64), int64_t((size_t(2) << 30) / (size_t(m) * size_t(nn) * 16))}));
